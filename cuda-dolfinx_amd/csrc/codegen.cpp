@@ -328,6 +328,27 @@ bool owner_pipe_emitted(const mf_form& f, const Integral& I) {
   return f.opt("owner_f32acc", 0) == 0 && 16 * cap + 2 * lists + table + 256 <= 160 * 1024;
 }
 
+// Rows (scalar values) per workgroup of the owner vector kernel.  Every cell
+// with a row in a chunk is computed by that chunk, so small chunks repeat
+// cells; large ones leave compute units without a workgroup.  The line lies at
+// three workgroups per CU (768 on a 256-CU chip).  Times of the cell integral
+// by values per chunk, on 132,651 rows (P1, 50^3 cubes): 2048 (65 workgroups)
+// 94 us, 768 42 us, 192 (691 workgroups) 19.5 us, 96 20.1 us; on 389,017 rows
+// (P3, 24^3): 2048 43 us, 768 30 us, 384 27.6 us, 192 31 us; above 768 values
+// nothing is gained (2.7 million rows, vector P2: 68 us at 768, 71 us at
+// 2048), so that is the LDS accumulator's size, the same for every mesh.
+int64_t vector_cap(const mf_form& f) {
+  return f.opt("vector_chunk_values", std::max<int64_t>(768, f.dm[0]->bs));
+}
+
+int64_t vector_chunk(const mf_form& f) {
+  const int64_t cap = vector_cap(f);
+  if (f.options.count("vector_chunk_values")) return cap;
+  const int64_t n = f.dm[0]->num_nodes * f.dm[0]->bs;
+  const int64_t even = (n + 3LL * f.ctx->num_cus - 1) / (3LL * f.ctx->num_cus);
+  return std::min(cap, std::max<int64_t>(48, (even + 15) / 16 * 16));
+}
+
 std::string kernel_name(const char* what, int type, int index) {
   static const char* tn[] = {"cell", "ext", "int"};
   return std::string("mf_") + what + "_" + tn[type] + "_" + std::to_string(index);
@@ -633,7 +654,7 @@ std::string generate_vbatch_source(const std::vector<const mf_form*>& forms,
     m["$BS0"] = std::to_string(d0->bs);
     m["$NR"] = std::to_string(d0->nd * d0->bs);
     m["$TAB"] = I.tab_name;
-    const int64_t vcap = f.opt("vector_chunk_values", 2048);
+    const int64_t vcap = vector_cap(f);
     cap = std::max(cap, vcap);
     m["$VCAP"] = std::to_string(vcap);
     m["$VPF"] = f.opt("vector_prefetch", 1) ? "1" : "0";
@@ -965,7 +986,7 @@ std::string generate_form_source(const mf_form& f) {
         m["$VK"] = "  __shared__ double acc[CAPV];\n"
                    "  const int k = mf_xcd_chunk(nchunks);\n"
                    "  if (k < 0) return;";
-        m["$VCAP"] = std::to_string(f.opt("vector_chunk_values", 2048));
+        m["$VCAP"] = std::to_string(vector_cap(f));
         m["$VPF"] = f.opt("vector_prefetch", 1) ? "1" : "0";
         os << subst(kOwnerVectorTemplate, m);
       }

@@ -235,7 +235,7 @@ std::shared_ptr<OwnerPlan> vector_plan(mf_form* L, Integral& I) {
   const mf_dofmap* d0 = L->dm[0];
   std::shared_ptr<OwnerPlan> plan;
   if (d0->nd <= 32) {
-    const int64_t per = std::max<int64_t>(1, L->opt("vector_chunk_values", 2048) / d0->bs);
+    const int64_t per = std::max<int64_t>(1, vector_chunk(*L) / d0->bs);
     std::vector<int32_t> rows;
     for (int64_t r = 0; r < d0->num_nodes; r += per) rows.push_back(static_cast<int32_t>(r));
     rows.push_back(static_cast<int32_t>(d0->num_nodes));

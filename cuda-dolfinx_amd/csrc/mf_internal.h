@@ -388,6 +388,10 @@ OwnerShape owner_shape(const mf_form& f, const Integral& I);
 bool owner_pipe_emitted(const mf_form& f, const Integral& I);
 int64_t record_bytes(const mf_form& f, const Integral& I);
 std::string kernel_name(const char* what, int type, int index);
+// owner vector kernel: the LDS accumulator's values (compile time) and the
+// scalar rows per workgroup of a form (run time, at most that)
+int64_t vector_cap(const mf_form& f);
+int64_t vector_chunk(const mf_form& f);
 bool dg_owner_emitted(const mf_form& f);
 // sparsity (sparsity.cpp): blocked pattern of all integrals
 void build_pattern(const mf_form& a, std::vector<int32_t>& rpb, std::vector<int32_t>& colsb);
