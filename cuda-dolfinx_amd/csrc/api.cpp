@@ -387,7 +387,8 @@ void compile_form(mf_form* f, int verbose) {
             I->records.alloc(f->mesh->num_cells * I->record_bytes / 8);
           }
         } else if (I->type == MF_CELL && !I->staged_src.empty()) {
-          I->k_slift = f->mod->get(mf::kernel_name("slift", I->type, I->index));
+          if (mf::staged_lift_emitted(*I))
+            I->k_slift = f->mod->get(mf::kernel_name("slift", I->type, I->index));
           if (mf::owner_supported(*f, *I)) {
             I->k_owner = f->mod->get(mf::kernel_name("owner", I->type, I->index));
             I->k_owner32 = mf::staged_trace(*I)
@@ -1230,32 +1231,25 @@ int mf_apply_lifting(mf_form* const* a, int nforms, double* b, int64_t n,
           MF_CHECK(!capturing, MF_ESTATE,
                    "apply_lifting under graph capture needs one uncaptured call with this form "
                    "and Dirichlet set first (it builds the lifting entity lists)");
-          mf::DevArray<int32_t> list, cnt;
-          list.alloc(std::max<int64_t>(1, I->n));
-          cnt.alloc(1);
-          mf::k_fill_i32(cnt.ptr, 1, 0, S(s));
-          mf::k_lift_list(list.ptr, cnt.ptr, I->d_ents.ptr, I->n, mf::entity_stride(I->type),
-                          mf::entity_ncell(I->type), f->dm[1]->dev.ptr, f->dm[1]->nd,
-                          f->dm[1]->bs, bc->markers.ptr, S(s));
-          int32_t h = 0;
-          MF_HIP(hipMemcpyAsync(&h, cnt.ptr, sizeof(int32_t), hipMemcpyDeviceToHost, S(s)));
-          MF_HIP(hipStreamSynchronize(S(s)));
-          it = I->lift_lists.emplace(bc->key, std::make_pair(std::move(list), (int64_t)h)).first;
+          it = I->lift_lists.emplace(bc->key, mf::build_lift_list(*f, *I, *bc, S(s))).first;
         }
-        const int64_t nl = it->second.second;
+        const mf::LiftList& ll = it->second;
+        const int64_t nl = ll.n;
         if (nl == 0 || nothing) continue;
         if (I->k_slift && f->opt("lift_kernel", 0) != 1) {
-          const int64_t nt = nl * f->dm[0]->nd;
-          mf::launch(I->k_slift, static_cast<uint32_t>((nt + 127) / 128), 128, 0, S(s),
+          uint32_t grid, threads;
+          mf::staged_lift_shape(*f, *I, nl, &grid, &threads);
+          mf::launch(I->k_slift, grid, threads, 0, S(s),
                      static_cast<int32_t>(nl), static_cast<const int32_t*>(nullptr),
-                     it->second.first.ptr, I->d_ents.ptr,
+                     ll.list.ptr, ll.pairs.ptr, ll.slot.ptr, ll.blk_ptr.ptr, ll.blk_row.ptr,
+                     ll.mask.ptr, I->d_ents.ptr,
                      f->mesh->cells.ptr, f->mesh->x.ptr, f->packed.ptr, f->consts.ptr,
                      f->dm[0]->dev.ptr, f->dm[1]->dev.ptr, bc->markers.ptr, bc->g.ptr, xk, scale,
                      b);
         } else {
           mf::launch(I->k_lift, static_cast<uint32_t>((nl + block - 1) / block), block, 0, S(s),
                      static_cast<int32_t>(nl), static_cast<const int32_t*>(nullptr),
-                     it->second.first.ptr, I->d_ents.ptr,
+                     ll.list.ptr, I->d_ents.ptr,
                      f->mesh->cells.ptr, f->mesh->x.ptr, f->packed.ptr, f->consts.ptr,
                      f->dm[0]->dev.ptr, f->dm[1]->dev.ptr, bc->markers.ptr, bc->g.ptr, xk, scale,
                      b, f->mesh->fperm.ptr);
@@ -1304,9 +1298,13 @@ int mf_apply_lifting_noalloc(mf_form* const* a, int nforms, double* b, int64_t n
                         mf::entity_ncell(I->type), f->dm[1]->dev.ptr, f->dm[1]->nd,
                         f->dm[1]->bs, bc->markers.ptr, S(s));
         if (I->k_slift && f->opt("lift_kernel", 0) != 1) {
-          const int64_t nt = I->n * f->dm[0]->nd;
-          mf::launch(I->k_slift, static_cast<uint32_t>((nt + 127) / 128), 128, 0, S(s),
+          uint32_t grid, threads;
+          mf::staged_lift_shape(*f, *I, I->n, &grid, &threads);
+          mf::launch(I->k_slift, grid, threads, 0, S(s),
                      static_cast<int32_t>(I->n), static_cast<const int32_t*>(count), list,
+                     static_cast<const int32_t*>(nullptr), static_cast<const uint16_t*>(nullptr),
+                     static_cast<const int32_t*>(nullptr), static_cast<const int32_t*>(nullptr),
+                     static_cast<const uint64_t*>(nullptr),
                      I->d_ents.ptr, f->mesh->cells.ptr, f->mesh->x.ptr, f->packed.ptr,
                      f->consts.ptr, f->dm[0]->dev.ptr, f->dm[1]->dev.ptr, bc->markers.ptr,
                      bc->g.ptr, xk, scale, b);

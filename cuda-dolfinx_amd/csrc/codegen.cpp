@@ -32,6 +32,7 @@ typedef signed char int8_t;
 typedef __hip_internal::int32_t int32_t;
 typedef __hip_internal::int64_t int64_t;
 typedef __hip_internal::uint32_t uint32_t;
+typedef __hip_internal::uint64_t uint64_t;
 typedef __hip_internal::int16_t int16_t;
 typedef unsigned short uint16_t;
 )";
@@ -347,6 +348,12 @@ int64_t vector_chunk(const mf_form& f) {
   const int64_t n = f.dm[0]->num_nodes * f.dm[0]->bs;
   const int64_t even = (n + 3LL * f.ctx->num_cus - 1) / (3LL * f.ctx->num_cus);
   return std::min(cap, std::max<int64_t>(48, (even + 15) / 16 * 16));
+}
+
+// the staged lifting kernel keeps up to 64 cells x nd rows and columns in LDS
+bool staged_lift_emitted(const Integral& I) {
+  return I.type == MF_CELL && !I.staged_src.empty() && !is_hex_staged(I) &&
+         staged_define(I.staged_src, "SK_ND") <= 128;
 }
 
 std::string kernel_name(const char* what, int type, int index) {
@@ -973,7 +980,7 @@ std::string generate_form_source(const mf_form& f) {
           }
         }
         m["$KNAME"] = kernel_name("slift", I->type, I->index);
-        os << subst(rename(kStagedLiftTemplate), m);
+        if (staged_lift_emitted(*I)) os << subst(rename(kStagedLiftTemplate), m);
       }
     } else if (f.rank == 1) {
       m["$KNAME"] = kernel_name("vec", I->type, I->index);

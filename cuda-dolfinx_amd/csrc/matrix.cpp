@@ -245,6 +245,83 @@ std::shared_ptr<OwnerPlan> vector_plan(mf_form* L, Integral& I) {
   return plan;
 }
 
+LiftList build_lift_list(const mf_form& f, const Integral& I, const mf_bc& bc, hipStream_t s) {
+  const mf_dofmap* d0 = f.dm[0];
+  const mf_dofmap* d1 = f.dm[1];
+  LiftList L;
+  DevArray<int32_t> cnt;
+  L.list.alloc(std::max<int64_t>(1, I.n));
+  cnt.alloc(1);
+  k_fill_i32(cnt.ptr, 1, 0, s);
+  k_lift_list(L.list.ptr, cnt.ptr, I.d_ents.ptr, I.n, entity_stride(I.type), entity_ncell(I.type),
+              d1->dev.ptr, d1->nd, d1->bs, bc.markers.ptr, s);
+  int32_t n = 0;
+  MF_HIP(hipMemcpyAsync(&n, cnt.ptr, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  MF_HIP(hipStreamSynchronize(s));
+  L.n = n;
+  if (n == 0) return L;
+  std::vector<int32_t> list(n);
+  MF_HIP(hipMemcpy(list.data(), L.list.ptr, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+  std::sort(list.begin(), list.end());           // the kernel appends in no particular order
+  L.list.upload(list);
+  const int nd = d0->nd, bs1 = d1->bs;
+  if (!I.k_slift || d1->nd * bs1 > 64 || (int64_t)n * nd >= INT32_MAX) return L;
+  std::vector<uint8_t> constrained(d1->num_nodes * bs1, 0);
+  for (int32_t d : bc.h_dofs) constrained[d] = 1;
+  std::vector<uint64_t> mask(n, 0);
+  for (int32_t k = 0; k < n; ++k) {
+    const int64_t c = I.h_ents[list[k]];
+    for (int j = 0; j < d1->nd * bs1; ++j) {
+      const int64_t node = d1->host[c * d1->nd + j / bs1];
+      mask[k] |= static_cast<uint64_t>(constrained[bs1 * node + j % bs1]) << j;
+    }
+  }
+  // row of every (cell, local row), in the order the kernel visits them
+  std::vector<int32_t> row(static_cast<size_t>(n) * nd);
+  const bool by_cell = staged_trace(I);
+  if (by_cell) {
+    for (int32_t k = 0; k < n; ++k)
+      for (int i = 0; i < nd; ++i) row[(size_t)k * nd + i] = d0->host[(int64_t)I.h_ents[list[k]] * nd + i];
+  } else {
+    std::vector<int32_t> start(d0->num_nodes + 1, 0), pairs(row.size());
+    for (int32_t k = 0; k < n; ++k)
+      for (int i = 0; i < nd; ++i) start[d0->host[(int64_t)I.h_ents[list[k]] * nd + i] + 1]++;
+    for (int64_t r = 0; r < d0->num_nodes; ++r) start[r + 1] += start[r];
+    for (int32_t k = 0; k < n; ++k)
+      for (int i = 0; i < nd; ++i) {
+        const int32_t r = d0->host[(int64_t)I.h_ents[list[k]] * nd + i];
+        row[start[r]] = r;
+        pairs[start[r]++] = k * nd + i;
+      }
+    L.pairs.upload(pairs);
+  }
+  const size_t per = by_cell ? 64u * nd : 128u;          // contributions per workgroup
+  std::vector<int32_t> ptr{0}, rows, seen;
+  std::vector<uint16_t> slot(row.size());
+  for (size_t p0 = 0; p0 < row.size(); p0 += per) {
+    const size_t p1 = std::min(row.size(), p0 + per);
+    seen.assign(row.begin() + p0, row.begin() + p1);
+    std::sort(seen.begin(), seen.end());
+    seen.erase(std::unique(seen.begin(), seen.end()), seen.end());
+    for (size_t p = p0; p < p1; ++p)
+      slot[p] = static_cast<uint16_t>(std::lower_bound(seen.begin(), seen.end(), row[p]) - seen.begin());
+    rows.insert(rows.end(), seen.begin(), seen.end());
+    ptr.push_back(static_cast<int32_t>(rows.size()));
+  }
+  L.slot.upload(slot);
+  L.blk_ptr.upload(ptr);
+  L.blk_row.upload(rows);
+  L.mask.upload(mask);
+  return L;
+}
+
+void staged_lift_shape(const mf_form& f, const Integral& I, int64_t n, uint32_t* grid, uint32_t* block) {
+  // 64 cells by four waves of rows, or 128 (cell, row) pairs per workgroup
+  const bool by_cell = staged_trace(I);
+  *block = by_cell ? 256 : 128;
+  *grid = static_cast<uint32_t>(by_cell ? (n + 63) / 64 : (n * f.dm[0]->nd + 127) / 128);
+}
+
 namespace {
 
 DevArray<int32_t>& get_table(mf_form* a, Integral& I, mf_matrix* A, hipStream_t s) {

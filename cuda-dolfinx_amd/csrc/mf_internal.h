@@ -220,6 +220,19 @@ struct mf_bc {
 };
 
 namespace mf {
+// Entities of an integral that touch a constrained column dof, in ascending
+// order.  For the staged lifting kernels also the constrained scalar columns of
+// every listed cell, the rows of each workgroup (ascending) and the place of
+// every (cell, local row) among its workgroup's rows; forms without a reference
+// tensor take the (list position * nd + local row) pairs sorted by row.  These
+// are empty when a cell has more than 64 scalar columns or the pairs exceed
+// int32.
+struct LiftList {
+  DevArray<int32_t> list, pairs, blk_ptr, blk_row;
+  DevArray<uint16_t> slot;
+  DevArray<uint64_t> mask;
+  int64_t n = 0;
+};
 struct Integral {
   int type = 0, id = -1;
   std::string tab_name, tab_src, staged_src;
@@ -243,7 +256,7 @@ struct Integral {
   int64_t owner_gridp = 0, owner_gridp32 = 0;
   int64_t record_bytes = 0;
   // lifting entity lists per constrained set (mf_bc::key)
-  std::map<uint64_t, std::pair<DevArray<int32_t>, int64_t>> lift_lists;
+  std::map<uint64_t, LiftList> lift_lists;
 };
 struct Coef {
   mf_dofmap* dm = nullptr;
@@ -379,6 +392,7 @@ std::vector<std::string> rtc_compile_options(const std::string& arch);
 bool owner_supported(const mf_form& f, const Integral& I);
 bool is_hex_staged(const Integral& I);
 bool staged_trace(const Integral& I);
+bool staged_lift_emitted(const Integral& I);
 bool hex_owner_supported(const mf_form& f, const Integral& I);
 int hex_batch(const mf_form& f, const Integral& I, int prec);
 int hex_block(const mf_form& f, int prec);
@@ -422,4 +436,9 @@ void build_block_pattern(const std::vector<mf_form*>& forms, int nr, int nc, int
 std::shared_ptr<OwnerPlan> vector_plan(mf_form* L, Integral& I);
 int entity_stride(int type);
 int entity_ncell(int type);
+// lifting entity list of integral I of the bilinear form f for one Dirichlet
+// set (reads the list's length back: not under graph capture)
+LiftList build_lift_list(const mf_form& f, const Integral& I, const mf_bc& bc, hipStream_t s);
+// workgroups and threads of the staged lifting kernel over n listed cells
+void staged_lift_shape(const mf_form& f, const Integral& I, int64_t n, uint32_t* grid, uint32_t* block);
 }  // namespace mf

@@ -24,7 +24,8 @@
 // Staged lifting kernel.  One thread per (cell touching a constrained
 // column, local row i): b_i -= scale * sum_j A_ij (g_j - x0_j) over the
 // constrained columns only, with the element blocks rebuilt from the staged
-// description (no nd x nd element tensor in registers or scratch).
+// description (no nd x nd element tensor in registers or scratch), the rows
+// of a workgroup added up in LDS.
 #include "mf_internal.h"
 
 namespace mf {
@@ -640,27 +641,89 @@ $VK
 }
 )";
 
+// Lifting over the cells that touch a constrained dof.  Bound by latency, by
+// the gathers of a cell's geometry and by the adds into b: global FP64 atomics
+// run at about 25 G/s here, and the cells at a boundary share most of their
+// rows.  A workgroup therefore adds its rows up in LDS (slot: the LDS place of
+// each of its contributions; blk_row[blk_ptr[k] ..]: the rows of workgroup k)
+// and issues one global atomic per row it holds, and a cell's constrained
+// scalar columns come as a mask (lmask), so all its values load at once
+// instead of node, marker and value one after the other per column.  Without
+// slots (null: the list was built on the device, length *nlist_dev) every
+// column's marker is read and each row goes straight to memory.
+//
+// Forms with a reference tensor: a workgroup takes 64 listed cells, lane = cell,
+// and each of its four waves a quarter of the local rows, so the tensor entries
+// are wave-uniform and an entry costs 6 multiply-adds, not a sum over the
+// quadrature points.  P3 on 24^3 cubes, 20 thousand boundary cells: 155 -> 14 us
+// (one thread per (cell, row), sorted by row, was 27 us: it gathers every
+// cell's geometry 20 times); P1 on 50^3: 18 -> 8 us.
+// Other forms: one thread per (cell, local row), sorted by row (pairs), 128 to
+// a workgroup.  Vector P2, one face of 48^3 cubes: 32 -> 19 us.
 const char* kStagedLiftTemplate = R"(
-extern "C" __global__ void __launch_bounds__(128)
+#ifdef SK_TRACE
+#define MF_LIFT_BLOCK 256
+#define MF_LIFT_ROWS (64 * SK_ND)
+#else
+#define MF_LIFT_BLOCK 128
+#define MF_LIFT_ROWS 128
+#endif
+extern "C" __global__ void __launch_bounds__(MF_LIFT_BLOCK)
 $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t* __restrict__ list,
-       const int32_t* __restrict__ ents,
+       const int32_t* __restrict__ pairs, const uint16_t* __restrict__ slot,
+       const int32_t* __restrict__ blk_ptr, const int32_t* __restrict__ blk_row,
+       const uint64_t* __restrict__ lmask, const int32_t* __restrict__ ents,
        const int32_t* __restrict__ geo, const double* __restrict__ xg,
        const double* __restrict__ coeffs, const double* __restrict__ consts,
        const int32_t* __restrict__ dm0, const int32_t* __restrict__ dm1,
        const int8_t* __restrict__ bc1, const double* __restrict__ g,
        const double* __restrict__ x0, const double scale, double* __restrict__ b)
 {
-  constexpr int ND = SK_ND, BS = SK_BS, NQ = SK_NQ, NV = $NV, W = $W;
+  constexpr int ND = SK_ND, BS = SK_BS, NQ = SK_NQ, NV = $NV, W = $W, NT = MF_LIFT_BLOCK;
   // cells in the list: nlist, or *nlist_dev when the list was built on the
   // device in the same stream (the grid then covers the largest possible list)
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (nlist_dev ? *nlist_dev : nlist) * ND) return;
-  const int e = list[t / ND], i = t % ND;
-  const int64_t c = ents[e];
+  const int nl = nlist_dev ? *nlist_dev : nlist;
+  const int tid = threadIdx.x;
+  __shared__ double sacc[MF_LIFT_ROWS * BS];
+  const int rows = slot ? blk_ptr[blockIdx.x + 1] - blk_ptr[blockIdx.x] : 0;
+  for (int p = tid; p < rows * BS; p += NT) sacc[p] = 0.0;
+#ifdef SK_TRACE
+  __shared__ double sv[ND * 64];                       // values to lift: [column][cell]
+  const int li = blockIdx.x * 64 + (tid & 63);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool live = li < nl;
+#else
+  const int t = blockIdx.x * NT + tid;
+  const bool live = t < nl * ND;
+  const int pr = live ? (pairs ? pairs[t] : t) : 0;
+  const int li = pr / ND, i = pr - li * ND;
+#endif
+  const int64_t c = live ? ents[list[li]] : 0;
+  const uint64_t mask = live && slot ? lmask[li] : 0;
+  // 0 at unconstrained columns
+  auto value = [&](const int k, const int64_t col) -> double {
+    const bool on = slot ? (mask >> (k & 63)) & 1 : bc1[col] != 0;
+    return on ? scale * (g[col] - (x0 ? x0[col] : 0.0)) : 0.0;
+  };
+#ifdef SK_TRACE
+#pragma unroll
+  for (int j0 = 0; j0 < ND; j0 += 4) {
+    const int j = j0 + wave;
+    if (j < ND) sv[j * 64 + (tid & 63)] = live ? value(j, dm1[c * ND + j]) : 0.0;
+  }
+#else
+  double v[ND * BS];
+#pragma unroll
+  for (int j = 0; j < ND; ++j) {
+    const int64_t n1 = dm1[c * ND + j];
+#pragma unroll
+    for (int bb = 0; bb < BS; ++bb) v[j * BS + bb] = live ? value(j * BS + bb, BS * n1 + bb) : 0.0;
+  }
+#endif
   double x[NV][3];
-  for (int v = 0; v < NV; ++v) {
-    const int64_t gv = geo[c * NV + v];
-    x[v][0] = xg[3 * gv]; x[v][1] = xg[3 * gv + 1]; x[v][2] = xg[3 * gv + 2];
+  for (int v_ = 0; v_ < NV; ++v_) {
+    const int64_t gv = geo[c * NV + v_];
+    x[v_][0] = xg[3 * gv]; x[v_][1] = xg[3 * gv + 1]; x[v_][2] = xg[3 * gv + 2];
   }
   const double J00 = x[1][0] - x[0][0], J01 = x[2][0] - x[0][0], J02 = x[3][0] - x[0][0];
   const double J10 = x[1][1] - x[0][1], J11 = x[2][1] - x[0][1], J12 = x[3][1] - x[0][1];
@@ -672,25 +735,53 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
                        (J12 * J20 - J10 * J22) * id, (J00 * J22 - J02 * J20) * id, (J02 * J10 - J00 * J12) * id,
                        (J10 * J21 - J11 * J20) * id, (J01 * J20 - J00 * J21) * id, (J00 * J11 - J01 * J10) * id};
   const double adet = fabs(det);
+  const double* w = coeffs + c * W;
+#ifdef SK_TRACE
+  // metric |det J| K K^T: tr G_ij = sum_rs M_rs R_ij[r][s]
+  const double M00 = adet * (K[0] * K[0] + K[1] * K[1] + K[2] * K[2]);
+  const double M11 = adet * (K[3] * K[3] + K[4] * K[4] + K[5] * K[5]);
+  const double M22 = adet * (K[6] * K[6] + K[7] * K[7] + K[8] * K[8]);
+  const double M01 = adet * (K[0] * K[3] + K[1] * K[4] + K[2] * K[5]);
+  const double M02 = adet * (K[0] * K[6] + K[1] * K[7] + K[2] * K[8]);
+  const double M12 = adet * (K[3] * K[6] + K[4] * K[7] + K[5] * K[8]);
+  constexpr int RI = (ND + 3) / 4;                     // rows per wave
+  double be[RI];
+#pragma unroll
+  for (int r = 0; r < RI; ++r) be[r] = 0.0;
+  __syncthreads();                                     // sv and sacc written
+  for (int j = 0; j < ND; ++j) {
+    const double vj = sv[j * 64 + (tid & 63)];
+    if (!__any(vj != 0.0)) continue;
+#pragma unroll
+    for (int r = 0; r < RI; ++r) {
+      const int i = min(wave * RI + r, ND - 1);
+      const double* R = SK_RS[i][j];
+      // the combine of these forms reads G[0] + G[4] + G[8]
+      double G[9] = {0, 0, 0, 0, -0.0, 0, 0, 0, -0.0};
+      G[0] = M00 * R[0] + M11 * R[1] + M22 * R[2] + M01 * R[3] + M02 * R[4] + M12 * R[5];
+      double blk[1];
+      sk_combine(G, w, consts, blk);
+      if (vj != 0.0) be[r] -= blk[0] * vj;
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < RI; ++r) {
+    const int i = wave * RI + r;
+    if (!live || i >= ND) continue;
+    if (slot) atomicAdd(&sacc[slot[(int64_t)li * ND + i]], be[r]);
+    else atomicAdd(&b[dm0[c * ND + i]], be[r]);
+  }
+#else
   double gi[NQ][3];
   for (int q = 0; q < NQ; ++q)
     for (int d = 0; d < 3; ++d)
       gi[q][d] = K[d] * SK_DPHI[q][i][0] + K[3 + d] * SK_DPHI[q][i][1] + K[6 + d] * SK_DPHI[q][i][2];
   double be[BS];
   for (int a = 0; a < BS; ++a) be[a] = 0.0;
-  const double* w = coeffs + c * W;
+#pragma unroll
   for (int j = 0; j < ND; ++j) {
-    const int64_t n1 = dm1[c * ND + j];
-    double v[BS];
     bool any = false;
-    for (int bb = 0; bb < BS; ++bb) {
-      const int64_t col = BS * n1 + bb;
-      v[bb] = 0.0;
-      if (bc1[col]) {
-        any = true;
-        v[bb] = scale * (g[col] - (x0 ? x0[col] : 0.0));
-      }
-    }
+    for (int bb = 0; bb < BS; ++bb) any |= v[j * BS + bb] != 0.0;
     if (!any) continue;
     double G[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     for (int q = 0; q < NQ; ++q) {
@@ -704,11 +795,27 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
     double blk[BS * BS];
     sk_combine(G, w, consts, blk);
     for (int a = 0; a < BS; ++a)
-      for (int bb = 0; bb < BS; ++bb) be[a] -= blk[a * BS + bb] * v[bb];
+      for (int bb = 0; bb < BS; ++bb) be[a] -= blk[a * BS + bb] * v[j * BS + bb];
   }
-  const int64_t n0 = dm0[c * ND + i];
-  for (int a = 0; a < BS; ++a) atomicAdd(&b[BS * n0 + a], be[a]);
+  __syncthreads();                                     // sacc zeroed
+  if (live) {
+    if (slot) {
+      for (int a = 0; a < BS; ++a) atomicAdd(&sacc[slot[t] * BS + a], be[a]);
+    } else {
+      const int64_t n0 = dm0[c * ND + i];
+      for (int a = 0; a < BS; ++a) atomicAdd(&b[BS * n0 + a], be[a]);
+    }
+  }
+#endif
+  if (slot) {
+    __syncthreads();
+    const int32_t* row = blk_row + blk_ptr[blockIdx.x];
+    for (int p = tid; p < rows * BS; p += NT)
+      atomicAdd(&b[(int64_t)BS * row[p / BS] + p % BS], sacc[p]);
+  }
 }
+#undef MF_LIFT_BLOCK
+#undef MF_LIFT_ROWS
 )";
 
 // Parameters of the warp-specialised owner-computes kernel.

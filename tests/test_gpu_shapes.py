@@ -1,0 +1,77 @@
+"""GPU parity at the sizes where a kernel's split into workgroups changes:
+partly filled, exactly filled and single workgroups, one-cell problems and
+constrained sets that leave some components free.  Against the oracle, to the
+relative 1e-12 that the FP64 paths are held to everywhere (the sums here have
+at most a few hundred terms of one sign pattern, 1e-14 at worst)."""
+import numpy as np
+import pytest
+
+from oracle import cpu
+from mifem import forms, problems
+from mifem.fem import DirichletBC, Function, functionspace
+from mifem.mesh import create_unit_cube
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-12
+
+
+def _rel(x, ref):
+    return np.linalg.norm(x - ref) / max(np.linalg.norm(ref), 1e-300)
+
+
+def _poisson(n, k):
+    mesh = create_unit_cube(n, jitter=0.2, seed=n)
+    V = functionspace(mesh, ("P", k))
+    kappa, f = Function(functionspace(mesh, ("DG", 0))), Function(V)
+    rng = np.random.default_rng(k)
+    kappa.x[:] = rng.uniform(1, 2, mesh.num_cells)
+    f.x[:] = rng.uniform(-1, 1, V.size)
+    return V, forms.stiffness(V, kappa), forms.source(V, f)
+
+
+def _elasticity(n):
+    P = problems.elasticity_p2(n)
+    return P.V, P.a, P.L
+
+
+def _some_dofs(V, share, seed):
+    """A Dirichlet set of single scalar dofs: components of a node may stay free."""
+    rng = np.random.default_rng(seed)
+    dofs = np.flatnonzero(rng.random(V.size) < share).astype(np.int32)
+    if dofs.size == 0:
+        dofs = np.array([V.size // 2], dtype=np.int32)
+    g = np.zeros(V.size)
+    g[dofs] = rng.uniform(-1, 1, dofs.size)
+    return DirichletBC(V, dofs, g)
+
+
+@pytest.mark.parametrize("form,n,share", [
+    ((1,), 1, 0.2), ((1,), 4, 0.02), ((2,), 3, 0.5), ((3,), 1, 0.0), ((3,), 4, 0.1),
+    ((), 1, 0.1), ((), 3, 0.0), ((), 4, 0.3)])
+def test_lifting_over_any_constrained_set(form, n, share):
+    import cudolfinx as cufem
+    print(f"[gpu-test] lifting {'P%d' % form if form else 'vector P2'} n={n} share={share}", flush=True)
+    V, a, L = _poisson(n, *form) if form else _elasticity(n)
+    bc = _some_dofs(V, share, 3)
+    x0 = np.random.default_rng(9).uniform(-1, 1, V.size)
+    af, Lf = cufem.form(a), cufem.form(L)
+    asm = cufem.CUDAAssembler()
+    b = asm.assemble_vector(Lf)
+    xv = asm.create_vector(Lf)
+    xv.data.upload(x0)
+    asm.apply_lifting(b, [af], [asm.pack_bcs([bc])], x0=[xv], scale=-0.7)
+    asm.synchronize()
+    ref = cpu.OracleAssembler(L).assemble_vector()
+    cpu.OracleAssembler(a).apply_lifting(ref, [bc], x0=x0, scale=-0.7)
+    assert _rel(b.to_host(), ref) <= TOL
+
+
+@pytest.mark.parametrize("n,k", [(1, 1), (9, 1), (17, 1), (2, 3), (9, 2), (13, 3)])
+def test_right_hand_side_rows_per_workgroup(n, k):
+    import cudolfinx as cufem
+    print(f"[gpu-test] right-hand side P{k} n={n}", flush=True)
+    V, _, L = _poisson(n, k)
+    asm = cufem.CUDAAssembler()
+    b = asm.assemble_vector(cufem.form(L))
+    asm.synchronize()
+    assert _rel(b.to_host(), cpu.OracleAssembler(L).assemble_vector()) <= TOL
