@@ -378,6 +378,8 @@ void compile_form(mf_form* f, int verbose) {
         I->k_mat = f->mod->get(mf::kernel_name("mat", I->type, I->index));
         I->k_lift = f->mod->get(mf::kernel_name("lift", I->type, I->index));
         if (I->type == MF_CELL && mf::is_hex_staged(*I)) {
+          if (mf::hex_lift_emitted(*f, *I))
+            I->k_hlift = f->mod->get(mf::kernel_name("hlift", I->type, I->index));
           if (mf::hex_owner_supported(*f, *I)) {
             I->k_hprep = f->mod->get(mf::kernel_name("hprep", I->type, I->index));
             const char* names[3] = {"howner64", "howner32", "howner16"};
@@ -1246,6 +1248,11 @@ int mf_apply_lifting(mf_form* const* a, int nforms, double* b, int64_t n,
                      f->mesh->cells.ptr, f->mesh->x.ptr, f->packed.ptr, f->consts.ptr,
                      f->dm[0]->dev.ptr, f->dm[1]->dev.ptr, bc->markers.ptr, bc->g.ptr, xk, scale,
                      b);
+        } else if (I->k_hlift && f->opt("lift_kernel", 0) != 1) {
+          mf::launch(I->k_hlift, static_cast<uint32_t>(nl), 64, 0, S(s), static_cast<int32_t>(nl),
+                     static_cast<const int32_t*>(nullptr), ll.list.ptr, I->d_ents.ptr,
+                     f->mesh->cells.ptr, f->mesh->x.ptr, f->dm[0]->dev.ptr, bc->markers.ptr,
+                     bc->g.ptr, xk, scale, b);
         } else {
           mf::launch(I->k_lift, static_cast<uint32_t>((nl + block - 1) / block), block, 0, S(s),
                      static_cast<int32_t>(nl), static_cast<const int32_t*>(nullptr),
@@ -1308,6 +1315,11 @@ int mf_apply_lifting_noalloc(mf_form* const* a, int nforms, double* b, int64_t n
                      I->d_ents.ptr, f->mesh->cells.ptr, f->mesh->x.ptr, f->packed.ptr,
                      f->consts.ptr, f->dm[0]->dev.ptr, f->dm[1]->dev.ptr, bc->markers.ptr,
                      bc->g.ptr, xk, scale, b);
+        } else if (I->k_hlift && f->opt("lift_kernel", 0) != 1) {
+          mf::launch(I->k_hlift, static_cast<uint32_t>(I->n), 64, 0, S(s),
+                     static_cast<int32_t>(I->n), static_cast<const int32_t*>(count), list,
+                     I->d_ents.ptr, f->mesh->cells.ptr, f->mesh->x.ptr, f->dm[0]->dev.ptr,
+                     bc->markers.ptr, bc->g.ptr, xk, scale, b);
         } else {
           mf::launch(I->k_lift, static_cast<uint32_t>((I->n + block - 1) / block), block, 0, S(s),
                      static_cast<int32_t>(I->n), static_cast<const int32_t*>(count), list,

@@ -268,6 +268,16 @@ bool hex_owner_supported(const mf_form& f, const Integral& I) {
          f.dm[0]->bs == 1 && f.dm[0]->nd == 64;
 }
 
+// The lifting kernel of hexahedral forms takes any degree whose stages fit its
+// LDS arrays (12 of at most 8^3 doubles).
+bool hex_lift_emitted(const mf_form& f, const Integral& I) {
+  if (!is_hex_staged(I) || f.rank != 2 || f.dm[0] != f.dm[1] || f.mesh->nv != 8 || f.W != 0)
+    return false;
+  const int k1 = staged_define(I.staged_src, "HX_K") + 1, m1 = staged_define(I.staged_src, "HX_NQ1");
+  return k1 >= 1 && k1 <= 8 && m1 >= 1 && m1 <= 8 && f.dm[0]->bs == 1 &&
+         f.dm[0]->nd == k1 * k1 * k1 && staged_define(I.staged_src, "HX_ND") == f.dm[0]->nd;
+}
+
 // Threads per workgroup of the hex matrix-core kernel: 512 for the FP32 / BF16
 // operand paths (more waves to overlap the MFMA chains with the operand
 // loads), 256 for FP64; option hex_block overrides both.
@@ -376,6 +386,7 @@ extern const char* kPrepTemplate;
 extern const char* kHexRecord;
 extern const char* kHexPrepTemplate;
 extern const char* kHexOwnerTemplate;
+extern const char* kHexLiftTemplate;
 extern const char* kDGOwnerMatrix;        // dg_kernel.cpp
 extern const char* kDGOwnerVector;
 extern const char* kDGCaseCellMat;
@@ -906,6 +917,10 @@ std::string generate_form_source(const mf_form& f) {
       os << subst(subst(kLift, {{"$GATHER", gather}}), m);
       if (I->type == MF_CELL && is_hex_staged(*I)) {
         os << "\n" << I->staged_src << "\n";
+        if (hex_lift_emitted(f, *I)) {
+          m["$KNAME"] = kernel_name("hlift", I->type, I->index);
+          os << subst(kHexLiftTemplate, m);
+        }
         if (hex_owner_supported(f, *I)) {
           m["$TAG"] = "H" + std::to_string(I->index);
           os << subst(kHexRecord, m);

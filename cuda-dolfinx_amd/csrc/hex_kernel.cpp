@@ -64,6 +64,153 @@ $KNAME(const int32_t n, const int32_t* __restrict__ ents, const int32_t* __restr
 }
 )";
 
+// Lifting over the hexahedra that touch a constrained dof: the element matrix
+// is applied to the values to lift, v_j = scale (g_j - x0_j) at constrained
+// columns and 0 elsewhere, without being formed.  One wave per listed cell:
+// the gradient and the value of sum_j v_j phi_j at the quadrature points by
+// contractions over x, y and z in turn, D_q applied at each point, and the
+// transposed contractions back to the rows; stages pass through LDS.  About
+// 5 thousand multiply-adds per cell at Q3 with 4 points per direction, against
+// the 64 x 64 x 64 x 4 of the element tensor that the per-entity kernel builds
+// in 34 KB of scratch per thread: 3,176 boundary cells (24^3 Q3) 86.6 ms
+// with that kernel, 8.5 us here.  Bound by latency and by its FP64 atomics into
+// b (25 G/s).
+const char* kHexLiftTemplate = R"(
+extern "C" __global__ void __launch_bounds__(64)
+$KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t* __restrict__ list,
+       const int32_t* __restrict__ ents, const int32_t* __restrict__ geo,
+       const double* __restrict__ xg, const int32_t* __restrict__ dm,
+       const int8_t* __restrict__ bc1, const double* __restrict__ g,
+       const double* __restrict__ x0, const double scale, double* __restrict__ b)
+{
+  constexpr int K1 = HX_K + 1, ND = HX_ND, M1 = HX_NQ1, NQ = M1 * M1 * M1;
+  if ((int)blockIdx.x >= (nlist_dev ? *nlist_dev : nlist)) return;
+  __shared__ double sx[24], sL[M1 * K1], sG[M1 * K1], sv[ND];
+  __shared__ double a0[M1 * K1 * K1], a1[M1 * K1 * K1];             // x done: value, x-derivative
+  __shared__ double bv[M1 * M1 * K1], bx[M1 * M1 * K1], by[M1 * M1 * K1];   // x and y done
+  __shared__ double f0[NQ], f1[NQ], f2[NQ], f3[NQ];                 // D_q (gradient, value)
+  const int lane = threadIdx.x;
+  const int64_t c = ents[list[blockIdx.x]];
+  for (int p = lane; p < M1 * K1; p += 64) {
+    sL[p] = HX_L[p / K1][p % K1];
+    sG[p] = HX_DL[p / K1][p % K1];
+  }
+  if (lane < 24) sx[lane] = xg[3 * (int64_t)geo[c * 8 + lane / 3] + lane % 3];
+  for (int p = lane; p < ND; p += 64) {
+    const int64_t col = dm[c * ND + p];
+    sv[p] = bc1[col] ? scale * (g[col] - (x0 ? x0[col] : 0.0)) : 0.0;
+  }
+  __syncthreads();
+  for (int p = lane; p < M1 * K1 * K1; p += 64) {
+    const int q1 = p % M1, jj = p / M1;                             // jj = jb + K1 jc
+    double u = 0.0, ux = 0.0;
+    for (int j = 0; j < K1; ++j) {
+      const double v = sv[j + K1 * jj];
+      u += sL[q1 * K1 + j] * v;
+      ux += sG[q1 * K1 + j] * v;
+    }
+    a0[p] = u;
+    a1[p] = ux;
+  }
+  __syncthreads();
+  for (int p = lane; p < M1 * M1 * K1; p += 64) {
+    const int q1 = p % M1, q2 = (p / M1) % M1, jc = p / (M1 * M1);
+    double u = 0.0, ux = 0.0, uy = 0.0;
+    for (int j = 0; j < K1; ++j) {
+      const int s = q1 + M1 * (j + K1 * jc);
+      u += sL[q2 * K1 + j] * a0[s];
+      ux += sL[q2 * K1 + j] * a1[s];
+      uy += sG[q2 * K1 + j] * a0[s];
+    }
+    bv[p] = u;
+    bx[p] = ux;
+    by[p] = uy;
+  }
+  __syncthreads();
+  for (int p = lane; p < NQ; p += 64) {
+    const int q1 = p % M1, q2 = (p / M1) % M1, q3 = p / (M1 * M1);
+    double u = 0.0, ux = 0.0, uy = 0.0, uz = 0.0;
+    for (int j = 0; j < K1; ++j) {
+      const int s = q1 + M1 * (q2 + M1 * j);
+      u += sL[q3 * K1 + j] * bv[s];
+      ux += sL[q3 * K1 + j] * bx[s];
+      uy += sL[q3 * K1 + j] * by[s];
+      uz += sG[q3 * K1 + j] * bv[s];
+    }
+    // trilinear geometry at this point (as in the matrix kernel)
+    const double X = HX_X1[q1], Y = HX_X1[q2], Z = HX_X1[q3];
+    double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+    for (int v = 0; v < 8; ++v) {
+      const int a = v & 1, bb = (v >> 1) & 1, cc = v >> 2;
+      const double fx = a ? X : 1 - X, fy = bb ? Y : 1 - Y, fz = cc ? Z : 1 - Z;
+      const double d0 = (a ? 1.0 : -1.0) * fy * fz, d1 = fx * (bb ? 1.0 : -1.0) * fz;
+      const double d2 = fx * fy * (cc ? 1.0 : -1.0);
+      for (int i = 0; i < 3; ++i) {
+        const double xv = sx[3 * v + i];
+        J[i][0] += xv * d0; J[i][1] += xv * d1; J[i][2] += xv * d2;
+      }
+    }
+    const double m00 = J[1][1] * J[2][2] - J[1][2] * J[2][1];
+    const double m01 = J[0][2] * J[2][1] - J[0][1] * J[2][2];
+    const double m02 = J[0][1] * J[1][2] - J[0][2] * J[1][1];
+    const double det = J[0][0] * m00 + J[1][0] * m01 + J[2][0] * m02;
+    const double id = 1.0 / det;
+    double K[3][3];
+    K[0][0] = m00 * id; K[0][1] = m01 * id; K[0][2] = m02 * id;
+    K[1][0] = (J[1][2] * J[2][0] - J[1][0] * J[2][2]) * id;
+    K[1][1] = (J[0][0] * J[2][2] - J[0][2] * J[2][0]) * id;
+    K[1][2] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id;
+    K[2][0] = (J[1][0] * J[2][1] - J[1][1] * J[2][0]) * id;
+    K[2][1] = (J[0][1] * J[2][0] - J[0][0] * J[2][1]) * id;
+    K[2][2] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
+    const double wq = HX_W1[q1] * HX_W1[q2] * HX_W1[q3] * fabs(det);
+    const double s = HX_KAPPA * wq;
+    // physical gradient K^T u, back to reference components K (K^T u)
+    const double gx = K[0][0] * ux + K[1][0] * uy + K[2][0] * uz;
+    const double gy = K[0][1] * ux + K[1][1] * uy + K[2][1] * uz;
+    const double gz = K[0][2] * ux + K[1][2] * uy + K[2][2] * uz;
+    f0[p] = s * (K[0][0] * gx + K[0][1] * gy + K[0][2] * gz);
+    f1[p] = s * (K[1][0] * gx + K[1][1] * gy + K[1][2] * gz);
+    f2[p] = s * (K[2][0] * gx + K[2][1] * gy + K[2][2] * gz);
+    f3[p] = -HX_K2 * wq * u;
+  }
+  __syncthreads();
+  for (int p = lane; p < M1 * M1 * K1; p += 64) {
+    const int q1 = p % M1, q2 = (p / M1) % M1, ic = p / (M1 * M1);
+    double r = 0.0, rx = 0.0, ry = 0.0;
+    for (int q = 0; q < M1; ++q) {
+      const int s = q1 + M1 * (q2 + M1 * q);
+      r += sG[q * K1 + ic] * f2[s] + sL[q * K1 + ic] * f3[s];
+      rx += sL[q * K1 + ic] * f0[s];
+      ry += sL[q * K1 + ic] * f1[s];
+    }
+    bv[p] = r;
+    bx[p] = rx;
+    by[p] = ry;
+  }
+  __syncthreads();
+  for (int p = lane; p < M1 * K1 * K1; p += 64) {
+    const int q1 = p % M1, ib = (p / M1) % K1, ic = p / (M1 * K1);
+    double r = 0.0, rx = 0.0;
+    for (int q = 0; q < M1; ++q) {
+      const int s = q1 + M1 * (q + M1 * ic);
+      r += sG[q * K1 + ib] * by[s] + sL[q * K1 + ib] * bv[s];
+      rx += sL[q * K1 + ib] * bx[s];
+    }
+    a0[p] = r;
+    a1[p] = rx;
+  }
+  __syncthreads();
+  for (int p = lane; p < ND; p += 64) {
+    const int ia = p % K1, ii = p / K1;
+    double r = 0.0;
+    for (int q = 0; q < M1; ++q)
+      r += sG[q * K1 + ia] * a1[q + M1 * ii] + sL[q * K1 + ia] * a0[q + M1 * ii];
+    atomicAdd(&b[dm[c * ND + p]], -r);
+  }
+}
+)";
+
 const char* kHexOwnerTemplate = R"(
 #if MF_HX_PREC == 16
 typedef short mf_bf4 __attribute__((ext_vector_type(4)));

@@ -241,7 +241,7 @@ struct Integral {
   int64_t n = 0;
   int index = 0;                      // position in the form
   hipFunction_t k_mat = nullptr, k_vec = nullptr, k_lift = nullptr, k_owner = nullptr;
-  hipFunction_t k_vown = nullptr, k_slift = nullptr, k_prep = nullptr;
+  hipFunction_t k_vown = nullptr, k_slift = nullptr, k_hlift = nullptr, k_prep = nullptr;
   hipFunction_t k_hprep = nullptr, k_howner[3] = {nullptr, nullptr, nullptr};  // FP64, FP32, BF16
   hipFunction_t k_scl = nullptr;      // rank 0: per-block partial sums
   int64_t scl_off = 0;                // rank 0: first partial of this integral
@@ -394,6 +394,7 @@ bool is_hex_staged(const Integral& I);
 bool staged_trace(const Integral& I);
 bool staged_lift_emitted(const Integral& I);
 bool hex_owner_supported(const mf_form& f, const Integral& I);
+bool hex_lift_emitted(const mf_form& f, const Integral& I);
 int hex_batch(const mf_form& f, const Integral& I, int prec);
 int hex_block(const mf_form& f, int prec);
 struct OwnerShape { int nb = 0, maxp = 0; };

@@ -66,6 +66,35 @@ def test_lifting_over_any_constrained_set(form, n, share):
     assert _rel(b.to_host(), ref) <= TOL
 
 
+@pytest.mark.parametrize("degree,n,share,noalloc", [
+    (1, 1, 0.3, False), (1, 5, 0.1, False), (2, 3, 0.05, True), (3, 1, 0.0, False), (3, 3, 0.2, True),
+    (3, 4, 0.02, False)])
+def test_hexahedral_lifting(degree, n, share, noalloc):
+    """The sum-factorised lifting of Q1 to Q3 Helmholtz forms on jittered hexahedra."""
+    import ctypes as C
+    import cudolfinx as cufem
+    from cudolfinx import _lib
+    print(f"[gpu-test] hexahedral lifting Q{degree} n={n} share={share} noalloc={noalloc}", flush=True)
+    P = problems.helmholtz_q3(n, seed=4, degree=degree)
+    bc = _some_dofs(P.V, share, 5)
+    x0 = np.random.default_rng(2).uniform(-1, 1, P.V.size)
+    af, Lf = cufem.form(P.a), cufem.form(P.L)
+    asm = cufem.CUDAAssembler()
+    b, xv = asm.create_vector(Lf), asm.create_vector(Lf)
+    xv.data.upload(x0)
+    dbc = asm.pack_bcs([bc])
+    if noalloc:
+        _lib.check(_lib.lib().mf_apply_lifting_noalloc(
+            (C.c_void_p * 1)(af.handle.value), 1, b.ptr, b.size,
+            (C.c_void_p * 1)(dbc._get_cpp_bcs(P.V).handle.value), (C.c_void_p * 1)(xv.ptr.value), 0.9, None))
+    else:
+        asm.apply_lifting(b, [af], [dbc], x0=[xv], scale=0.9)
+    asm.synchronize()
+    ref = np.zeros(P.V.size)
+    cpu.OracleAssembler(P.a).apply_lifting(ref, [bc], x0=x0, scale=0.9)
+    assert _rel(b.to_host(), ref) <= TOL
+
+
 @pytest.mark.parametrize("n,k", [(1, 1), (9, 1), (17, 1), (2, 3), (9, 2), (13, 3)])
 def test_right_hand_side_rows_per_workgroup(n, k):
     import cudolfinx as cufem
