@@ -290,7 +290,8 @@ int hex_batch(const mf_form& f, const Integral& I, int prec) {
   const int64_t cap = f.opt("chunk_values", 4096), maxr = f.opt("chunk_rows", 64);
   const int64_t budget = f.opt("owner_lds", 78 * 1024);
   const int64_t fixed = 8 * cap + 4 * (maxr + 1) + 4 * f.opt("owner_pairs", 384) + 64;
-  const int64_t per_cell = 464 + 4 + (int64_t)nq1 * nq1 * nq1 * 8 * (prec == 64 ? 8 : 4);
+  const int64_t nq = (int64_t)nq1 * nq1 * nq1;
+  const int64_t per_cell = 464 + 4 + (prec == 64 ? 8 * (8 * nq + 8) : 4 * 8 * nq);
   int64_t nb = (budget - fixed) / per_cell;
   nb = std::min<int64_t>(nb, f.opt("owner_nb", 16));
   MF_CHECK(nb >= 1, MF_EUNSUPPORTED, "hexahedral owner kernel does not fit the LDS budget");
