@@ -376,6 +376,8 @@ void compile_form(mf_form* f, int verbose) {
     for (auto& I : f->ints) {
       if (f->rank == 2) {
         I->k_mat = f->mod->get(mf::kernel_name("mat", I->type, I->index));
+        if (mf::tensor_emitted(*f, *I))
+          I->k_ten = f->mod->get(mf::kernel_name("ten", I->type, I->index));
         I->k_lift = f->mod->get(mf::kernel_name("lift", I->type, I->index));
         if (I->type == MF_CELL && mf::is_hex_staged(*I)) {
           if (mf::hex_lift_emitted(*f, *I))
@@ -1254,7 +1256,8 @@ int mf_apply_lifting(mf_form* const* a, int nforms, double* b, int64_t n,
                      f->mesh->cells.ptr, f->mesh->x.ptr, f->dm[0]->dev.ptr, bc->markers.ptr,
                      bc->g.ptr, xk, scale, b);
         } else {
-          mf::launch(I->k_lift, static_cast<uint32_t>((nl + block - 1) / block), block, 0, S(s),
+          mf::launch(I->k_lift, static_cast<uint32_t>((nl + block - 1) / block * mf::row_groups(*f, *I)),
+                     block, 0, S(s),
                      static_cast<int32_t>(nl), static_cast<const int32_t*>(nullptr),
                      ll.list.ptr, I->d_ents.ptr,
                      f->mesh->cells.ptr, f->mesh->x.ptr, f->packed.ptr, f->consts.ptr,
@@ -1321,7 +1324,8 @@ int mf_apply_lifting_noalloc(mf_form* const* a, int nforms, double* b, int64_t n
                      I->d_ents.ptr, f->mesh->cells.ptr, f->mesh->x.ptr, f->dm[0]->dev.ptr,
                      bc->markers.ptr, bc->g.ptr, xk, scale, b);
         } else {
-          mf::launch(I->k_lift, static_cast<uint32_t>((I->n + block - 1) / block), block, 0, S(s),
+          mf::launch(I->k_lift, static_cast<uint32_t>((I->n + block - 1) / block * mf::row_groups(*f, *I)),
+                     block, 0, S(s),
                      static_cast<int32_t>(I->n), static_cast<const int32_t*>(count), list,
                      I->d_ents.ptr, f->mesh->cells.ptr, f->mesh->x.ptr, f->packed.ptr,
                      f->consts.ptr, f->dm[0]->dev.ptr, f->dm[1]->dev.ptr, bc->markers.ptr,

@@ -349,6 +349,58 @@ DevArray<int32_t>& get_table(mf_form* a, Integral& I, mf_matrix* A, hipStream_t 
 
 }  // namespace
 
+// Gather plan of one integral (built once per matrix, on the device but for
+// the prefix sum), null when the workspace would exceed 4 GiB (its offsets are
+// int32, and one matrix holds it for good), or when it does not exist yet and
+// s is being captured: the per-entity kernel with its offset table serves then.
+static GatherPlan* gather_plan(mf_form* a, Integral& I, mf_matrix* A, hipStream_t s) {
+  const auto key = std::make_pair(a->uid, I.index);
+  auto it = A->gathers.find(key);
+  if (it != A->gathers.end()) return it->second.get();
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  MF_HIP(hipStreamIsCapturing(s, &cs));
+  if (cs != hipStreamCaptureStatusNone) return nullptr;
+  const mf_dofmap* d0 = a->dm[0];
+  const mf_dofmap* d1 = a->dm[1];
+  const int ncell = entity_ncell(I.type), ni = ncell * d0->nd, nj = ncell * d1->nd;
+  const int64_t planes = (int64_t)ni * d0->bs * nj * d1->bs, ws = (I.n + 63) / 64 * 64 * planes;
+  if (ws > (int64_t(1) << 29) || I.n * ni * nj >= INT32_MAX) return A->gathers[key].get();
+  auto g = std::make_unique<GatherPlan>();
+  DevArray<int32_t> count, missing;
+  count.alloc(std::max<int64_t>(1, A->nnz_b));
+  missing.alloc(1);
+  k_fill_i32(count.ptr, A->nnz_b, 0, s);
+  k_fill_i32(missing.ptr, 1, 0, s);
+  auto pass = [&](int32_t* fill) {
+    k_gather_plan(count.ptr, fill, I.d_ents.ptr, I.n, entity_stride(I.type), ncell, d0->dev.ptr,
+                  d0->nd, d1->dev.ptr, d1->nd, d0->bs, d1->bs, A->rpb.ptr, A->colsb.ptr, missing.ptr, s);
+  };
+  pass(nullptr);
+  std::vector<int32_t> ptr(A->nnz_b + 1, 0);
+  int32_t h_missing = 0;
+  MF_HIP(hipMemcpyAsync(ptr.data(), count.ptr, sizeof(int32_t) * A->nnz_b, hipMemcpyDeviceToHost, s));
+  MF_HIP(hipMemcpyAsync(&h_missing, missing.ptr, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  MF_HIP(hipStreamSynchronize(s));
+  MF_CHECK(h_missing == 0, MF_ENOTFOUND,
+           std::to_string(h_missing) + " element entries are missing from the sparsity pattern");
+  int32_t sum = 0;
+  for (int64_t q = 0; q <= A->nnz_b; ++q) {
+    const int32_t c = ptr[q];
+    ptr[q] = sum;
+    sum += c;
+  }
+  g->ptr.upload(ptr);
+  MF_HIP(hipMemcpyAsync(count.ptr, g->ptr.ptr, sizeof(int32_t) * A->nnz_b, hipMemcpyDeviceToDevice, s));
+  g->at.alloc(std::max<int32_t>(1, sum));
+  g->pos.alloc(std::max<int64_t>(1, A->nnz_b));
+  pass(g->at.ptr);
+  k_gather_sort(g->at.ptr, g->ptr.ptr, g->pos.ptr, A->nnz_b, A->nrows_b, A->rpb.ptr, A->row_ptr.ptr,
+                d0->bs, d1->bs, s);
+  g->ws.alloc(std::max<int64_t>(1, ws));
+  MF_HIP(hipStreamSynchronize(s));                     // count and missing are freed here
+  return (A->gathers[key] = std::move(g)).get();
+}
+
 // ---------------------------------------------------------------------------
 // Cell-owner schedule for discontinuous spaces (kernel: dg_kernel.cpp)
 // ---------------------------------------------------------------------------
@@ -668,12 +720,35 @@ void assemble_matrix(mf_form* a, mf_matrix* A, const mf_bc* bc0, const mf_bc* bc
            A->colsb.ptr, n0, A->values, diagonal, flags);
     }
     }
-  } else if (zero) {
-    k_fill(A->values, A->nnz, 0.0, s);
   }
+  // Without an owner kernel, an overwriting call takes the integral with the
+  // most element entries through the gather: its tensors into a workspace, then
+  // one sum and one store per CSR value, where the per-entity kernel zeroes
+  // the values and adds every entry with a global atomic.
+  Integral* gathered = nullptr;
+  if (!owner && zero && mode == 0) {
+    auto entries = [&](const Integral& I) {
+      return I.n * entity_ncell(I.type) * (int64_t)entity_ncell(I.type);
+    };
+    for (auto& I : a->ints)
+      if (I->n && I->k_ten && (!gathered || entries(*I) > entries(*gathered))) gathered = I.get();
+    if (GatherPlan* g = gathered ? gather_plan(a, *gathered, A, s) : nullptr) {
+      const Integral& I = *gathered;
+      const int nc = entity_ncell(I.type) * a->dm[1]->nd * a->dm[1]->bs;
+      launch(I.k_ten, static_cast<uint32_t>((I.n + 63) / 64), 64, 0, s,
+             static_cast<int32_t>(I.n), I.d_ents.ptr, a->mesh->cells.ptr, a->mesh->x.ptr,
+             a->packed.ptr, a->consts.ptr, a->dm[0]->dev.ptr, a->dm[1]->dev.ptr, m0, m1, g->ws.ptr,
+             a->mesh->fperm.ptr);
+      k_gather(A->values, g->ws.ptr, g->ptr.ptr, g->at.ptr, g->pos.ptr, A->nnz_b, a->dm[0]->bs,
+               a->dm[1]->bs, nc, s);
+    } else {
+      gathered = nullptr;
+    }
+  }
+  if (!owner && !gathered && zero) k_fill(A->values, A->nnz, 0.0, s);
   const uint32_t block = static_cast<uint32_t>(a->opt("block", 128));
   for (auto& I : a->ints) {
-    if (I.get() == owner || I->n == 0) continue;
+    if (I.get() == owner || I.get() == gathered || I->n == 0) continue;
     auto& table = get_table(a, *I, A, s);
     launch(I->k_mat, static_cast<uint32_t>((I->n + block - 1) / block), block, 0, s,
            static_cast<int32_t>(I->n), I->d_ents.ptr, a->mesh->cells.ptr, a->mesh->x.ptr,

@@ -159,6 +159,16 @@ void k_build_table(int32_t* table, const int32_t* ents, int64_t nents, int strid
                    const int32_t* dm0, int nd0, const int32_t* dm1, int nd1, int bs0, int bs1,
                    const int32_t* row_ptr, const int32_t* rpb, const int32_t* colsb,
                    int32_t* missing, hipStream_t s);
+// Gather of an integral's element tensors into the CSR values: counting and
+// filling the contributions of every blocked entry, ordering them, and the sum.
+void k_gather_plan(int32_t* count, int32_t* fill, const int32_t* ents, int64_t nents, int stride,
+                   int ncell, const int32_t* dm0, int nd0, const int32_t* dm1, int nd1, int bs0,
+                   int bs1, const int32_t* rpb, const int32_t* colsb, int32_t* missing,
+                   hipStream_t s);
+void k_gather_sort(int32_t* fill, const int32_t* ptr, int2* pos, int64_t nq, int64_t nrows_b,
+                   const int32_t* rpb, const int32_t* row_ptr, int bs0, int bs1, hipStream_t s);
+void k_gather(double* values, const double* ws, const int32_t* ptr, const int32_t* at,
+              const int2* pos, int64_t nq, int bs0, int bs1, int row_stride, hipStream_t s);
 // Appends the index of every entity with a constrained column dof to list.
 void k_lift_list(int32_t* list, int32_t* count, const int32_t* ents, int64_t nents, int stride,
                  int ncell, const int32_t* dm1, int nd1, int bs1, const int8_t* bc1,
@@ -240,6 +250,7 @@ struct Integral {
   DevArray<int32_t> d_ents;
   int64_t n = 0;
   int index = 0;                      // position in the form
+  hipFunction_t k_ten = nullptr;      // element tensors into a workspace
   hipFunction_t k_mat = nullptr, k_vec = nullptr, k_lift = nullptr, k_owner = nullptr;
   hipFunction_t k_vown = nullptr, k_slift = nullptr, k_hlift = nullptr, k_prep = nullptr;
   hipFunction_t k_hprep = nullptr, k_howner[3] = {nullptr, nullptr, nullptr};  // FP64, FP32, BF16
@@ -267,6 +278,15 @@ struct Coef {
   // own values changed since they were last packed (a coefficient bound to
   // caller device memory, ext, is always packed: it can change unseen)
   bool dirty = true;
+};
+// Gather of one integral's element tensors into a matrix's values: per blocked
+// CSR entry q the contributions at[ptr[q] .. ptr[q + 1]) (workspace offsets,
+// ascending) and its place in the values.  The workspace belongs to the matrix:
+// a call that overwrites the values cannot run beside another on that matrix.
+struct GatherPlan {
+  DevArray<int32_t> ptr, at;
+  DevArray<int2> pos;
+  DevArray<double> ws;
 };
 struct OwnerPlan;   // cooperative owner-computes schedule (matrix.cpp)
 // Cell-owner schedule for forms on discontinuous spaces (matrix.cpp)
@@ -375,6 +395,8 @@ struct mf_matrix {
   // makes them stale; they are rebuilt on the next assembly)
   std::map<std::pair<uint64_t, int>, std::pair<uint64_t, std::shared_ptr<mf::OwnerPlan>>> plans;
   std::map<uint64_t, std::shared_ptr<mf::DGPlan>> dgplans;   // per form uid (null: unsupported)
+  // per (form uid, integral index) gathers of element tensors (null: too large)
+  std::map<std::pair<uint64_t, int>, std::unique_ptr<mf::GatherPlan>> gathers;
   // adopted caller pattern without the bs-unrolled block structure: the form
   // assembles into `inner` (its own pattern), whose value k is then added at
   // position inner_map[k] of this matrix's values
@@ -403,6 +425,10 @@ OwnerShape owner_shape(const mf_form& f, const Integral& I);
 bool owner_pipe_emitted(const mf_form& f, const Integral& I);
 int64_t record_bytes(const mf_form& f, const Integral& I);
 std::string kernel_name(const char* what, int type, int index);
+// the element-tensor kernel (mf_ten_*) is emitted
+bool tensor_emitted(const mf_form& f, const Integral& I);
+// row groups of the per-entity lifting kernel
+int row_groups(const mf_form& f, const Integral& I);
 // owner vector kernel: the LDS accumulator's values (compile time) and the
 // scalar rows per workgroup of a form (run time, at most that)
 int64_t vector_cap(const mf_form& f);

@@ -229,6 +229,101 @@ __global__ void table_kernel(int32_t* __restrict__ table, const int32_t* __restr
   }
 }
 
+// Contributions of an integral to each blocked CSR entry q: fill == nullptr
+// counts them (count[q]); otherwise count holds the next free place of q and
+// fill gets each contribution's offset in the element-tensor workspace (entity
+// e, local nodes i, j: plane (i bs0) NJ bs1 + j bs1 of the 64 entities of e).
+__global__ void gather_plan_kernel(int32_t* __restrict__ count, int32_t* __restrict__ fill,
+                                   const int32_t* __restrict__ ents, int64_t nents, int stride,
+                                   int ncell, const int32_t* __restrict__ dm0, int nd0,
+                                   const int32_t* __restrict__ dm1, int nd1, int bs0, int bs1,
+                                   const int32_t* __restrict__ rpb,
+                                   const int32_t* __restrict__ colsb, int32_t* __restrict__ missing) {
+  const int NI = ncell * nd0, NJ = ncell * nd1;
+  const int64_t total = nents * NI * NJ;
+  const int64_t gs = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; l < total; l += gs) {
+    const int64_t e = l / (NI * NJ);
+    const int ij = static_cast<int>(l - e * NI * NJ);
+    const int i = ij / NJ, j = ij - i * NJ;
+    const int32_t ci = ents[e * stride + 2 * (i / nd0)], cj = ents[e * stride + 2 * (j / nd1)];
+    const int32_t rn = dm0[(int64_t)ci * nd0 + (i % nd0)], cn = dm1[(int64_t)cj * nd1 + (j % nd1)];
+    const int64_t hi = rpb[rn + 1], p = search(colsb, rpb[rn], hi, cn);
+    if (p >= hi || colsb[p] != cn) {
+      atomicAdd(missing, 1);
+      continue;
+    }
+    const int32_t k = atomicAdd(&count[p], 1);
+    if (fill) {
+      const int64_t plane = (int64_t)i * bs0 * NJ * bs1 + (int64_t)j * bs1;
+      const int64_t planes = (int64_t)NI * bs0 * NJ * bs1;
+      fill[k] = static_cast<int32_t>(((e >> 6) * planes + plane) * 64 + (e & 63));
+    }
+  }
+}
+
+// Ascending order within every entry's contributions (a fixed order of
+// summation), and the entry's place in the bs-unrolled CSR: pos[q] = (offset of
+// its first value, length of its scalar rows).
+__global__ void gather_sort_kernel(int32_t* __restrict__ fill, const int32_t* __restrict__ ptr,
+                                   int2* __restrict__ pos, int64_t nq, int64_t nrows_b,
+                                   const int32_t* __restrict__ rpb,
+                                   const int32_t* __restrict__ row_ptr, int bs0, int bs1) {
+  const int64_t gs = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < nq; q += gs) {
+    for (int32_t a = ptr[q] + 1; a < ptr[q + 1]; ++a) {
+      const int32_t v = fill[a];
+      int32_t b = a - 1;
+      for (; b >= ptr[q] && fill[b] > v; --b) fill[b + 1] = fill[b];
+      fill[b + 1] = v;
+    }
+    int64_t lo = 0, hi = nrows_b;                      // row of q
+    while (hi - lo > 1) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (rpb[mid] <= q) lo = mid;
+      else hi = mid;
+    }
+    const int32_t r0 = row_ptr[lo * bs0];
+    pos[q] = make_int2(r0 + static_cast<int32_t>(q - rpb[lo]) * bs1, row_ptr[lo * bs0 + 1] - r0);
+  }
+}
+
+// values = sum of each entry's element-tensor contributions, in ascending order
+// (0 where it has none): one thread per scalar value.  Bound by memory: the
+// tensors (8 B) and their places (4 B) read once, the values written once.
+// Workgroups of one XCD take a contiguous eighth of the entries, whose
+// contributions lie close together in the workspace.
+__global__ void __launch_bounds__(kBlock) gather_kernel(
+    double* __restrict__ values, const double* __restrict__ ws, const int32_t* __restrict__ ptr,
+    const int32_t* __restrict__ at, const int2* __restrict__ pos, int64_t nq, int bs0, int bs1,
+    int row_stride) {
+  const int64_t per = (gridDim.x + 7) / 8;
+  const int64_t t = ((blockIdx.x % 8) * per + blockIdx.x / 8) * kBlock + threadIdx.x;
+  const int bb = bs0 * bs1;
+  const int64_t q = bb == 1 ? t : t / bb;
+  if (q >= nq) return;
+  const int ab = static_cast<int>(t - q * bb), a = ab / bs1, b = ab - a * bs1;
+  const int32_t off = (a * row_stride + b) * 64;
+  double sum = 0.0;
+  int32_t k = ptr[q];
+  const int32_t e = ptr[q + 1];
+  for (; k + 3 < e; k += 4) {
+    const int32_t k0 = at[k], k1 = at[k + 1], k2 = at[k + 2], k3 = at[k + 3];
+    const double v0 = ws[k0 + off], v1 = ws[k1 + off], v2 = ws[k2 + off], v3 = ws[k3 + off];
+    sum += v0;
+    sum += v1;
+    sum += v2;
+    sum += v3;
+  }
+  for (; k < e; ++k) sum += ws[at[k] + off];
+  if (bb == 1) {
+    values[q] = sum;
+  } else {
+    const int2 p = pos[q];
+    values[(int64_t)p.x + (int64_t)a * p.y + b] = sum;
+  }
+}
+
 __global__ void block_table_kernel(int32_t* __restrict__ table, const int32_t* __restrict__ ents,
                                    int64_t nents, int stride, int ncell,
                                    const int32_t* __restrict__ dm0, int nd0,
@@ -413,6 +508,33 @@ void k_unroll_cols(int32_t* cols, const int32_t* row_ptr, const int32_t* rpb, co
                    int64_t nrows_b, int bs0, int bs1, hipStream_t s) {
   unroll_kernel<<<grid_for(nrows_b * 32), kBlock, 0, s>>>(cols, row_ptr, rpb, colsb, nrows_b, bs0,
                                                           bs1);
+  MF_HIP(hipGetLastError());
+}
+void k_gather_plan(int32_t* count, int32_t* fill, const int32_t* ents, int64_t nents, int stride,
+                   int ncell, const int32_t* dm0, int nd0, const int32_t* dm1, int nd1, int bs0,
+                   int bs1, const int32_t* rpb, const int32_t* colsb, int32_t* missing,
+                   hipStream_t s) {
+  const int64_t total = nents * (int64_t)ncell * nd0 * ncell * nd1;
+  if (total <= 0) return;
+  gather_plan_kernel<<<grid_for(total, 4), kBlock, 0, s>>>(count, fill, ents, nents, stride, ncell,
+                                                           dm0, nd0, dm1, nd1, bs0, bs1, rpb, colsb,
+                                                           missing);
+  MF_HIP(hipGetLastError());
+}
+void k_gather_sort(int32_t* fill, const int32_t* ptr, int2* pos, int64_t nq, int64_t nrows_b,
+                   const int32_t* rpb, const int32_t* row_ptr, int bs0, int bs1, hipStream_t s) {
+  if (nq <= 0) return;
+  gather_sort_kernel<<<grid_for(nq), kBlock, 0, s>>>(fill, ptr, pos, nq, nrows_b, rpb, row_ptr, bs0,
+                                                     bs1);
+  MF_HIP(hipGetLastError());
+}
+void k_gather(double* values, const double* ws, const int32_t* ptr, const int32_t* at,
+              const int2* pos, int64_t nq, int bs0, int bs1, int row_stride, hipStream_t s) {
+  const int64_t n = nq * bs0 * bs1;
+  if (n <= 0) return;
+  const int64_t blocks = (n + kBlock - 1) / kBlock;
+  gather_kernel<<<static_cast<uint32_t>((blocks + 7) / 8 * 8), kBlock, 0, s>>>(
+      values, ws, ptr, at, pos, nq, bs0, bs1, row_stride);
   MF_HIP(hipGetLastError());
 }
 void k_build_table(int32_t* table, const int32_t* ents, int64_t nents, int stride, int ncell,

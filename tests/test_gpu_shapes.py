@@ -104,3 +104,66 @@ def test_right_hand_side_rows_per_workgroup(n, k):
     b = asm.assemble_vector(cufem.form(L))
     asm.synchronize()
     assert _rel(b.to_host(), cpu.OracleAssembler(L).assemble_vector()) <= TOL
+
+
+@pytest.mark.parametrize("n,k,share", [(1, 1, 0.0), (3, 1, 0.2), (5, 1, 0.1), (1, 2, 0.3), (3, 2, 0.1)])
+def test_gathered_element_tensors(n, k, share):
+    """Forms without an owner kernel: element tensors summed by entry, with a
+    Dirichlet set, against the per-entity kernel and the oracle; overwriting,
+    then adding, then overwriting again; and bit-identical on repeat."""
+    import cudolfinx as cufem
+    from mifem.nonlinear import reference_test_forms
+    print(f"[gpu-test] gathered tensors P{k} n={n} share={share}", flush=True)
+    R = reference_test_forms(create_unit_cube(n, jitter=0.2, seed=1), k)
+    a = R["matrix"][0]
+    V = a.function_spaces[0]
+    R["u"].x[:] = np.random.default_rng(4).uniform(-1, 1, V.size)
+    bc = _some_dofs(V, share, 6)
+    asm = cufem.CUDAAssembler()
+    f = cufem.form(a)
+    A = asm.assemble_matrix(f, bcs=[bc], diagonal=2.0)
+    asm.synchronize()
+    rp, cols, v = A.csr()
+    o = cpu.OracleAssembler(a)
+    orp, ocols, _, _ = o.sparsity()
+    ref = o.assemble_matrix(orp, ocols, [bc], diagonal=2.0)
+    assert np.array_equal(rp, orp) and np.array_equal(cols, ocols) and _rel(v, ref) <= TOL
+    g = cufem.form(a, options={"matrix_kernel": 1})
+    B = asm.assemble_matrix(g, bcs=[bc], diagonal=2.0)
+    asm.synchronize()
+    assert _rel(v, B.csr()[2]) <= TOL
+    asm.assemble_matrix(f, A, bcs=[], zero=False)
+    asm.synchronize()
+    free = o.assemble_matrix(orp, ocols, [])
+    assert _rel(A.csr()[2], ref + free) <= TOL
+    asm.assemble_matrix(f, A, bcs=[bc], diagonal=2.0)
+    asm.synchronize()
+    assert np.array_equal(A.csr()[2], v)
+
+
+def test_gathered_blocks_of_a_vector_form():
+    """bs > 1 and different row and column Dirichlet sets (no owner kernel)."""
+    import cudolfinx as cufem
+    from cudolfinx import _lib
+    V, a, _ = _elasticity(3)
+    f = cufem.form(a)
+    src = f.source()
+    asm = cufem.CUDAAssembler()
+    A = asm.create_matrix(f)
+    b0, b1 = _some_dofs(V, 0.1, 1), _some_dofs(V, 0.2, 2)
+    p0, p1 = asm.pack_bcs([b0]), asm.pack_bcs([b1])
+    f.to_device()
+    asm.pack_coefficients(f)
+    _lib.check(_lib.lib().mf_assemble_matrix(f.handle, A.handle, p0._get_cpp_bcs(V).handle,
+                                             p1._get_cpp_bcs(V).handle, 1.0, 1, None))
+    asm.synchronize()
+    assert "mf_mat_cell_0" in src
+    o = cpu.OracleAssembler(a)
+    rp, cols, _, _ = o.sparsity()
+    full = o.assemble_matrix(rp, cols, [])
+    rows = np.repeat(np.arange(V.size), np.diff(rp))
+    m0, m1 = np.zeros(V.size, bool), np.zeros(V.size, bool)
+    m0[b0.dofs], m1[b1.dofs] = True, True
+    ref = np.where(m0[rows] | m1[cols], 0.0, full)
+    ref[(rows == cols) & m0[rows]] = 1.0
+    assert _rel(A.csr()[2], ref) <= TOL
