@@ -245,6 +245,79 @@ std::shared_ptr<OwnerPlan> vector_plan(mf_form* L, Integral& I) {
   return plan;
 }
 
+// Whether blocks of cells (mf_vblk_*) beat the row-owning kernel (mf_vown_*).
+// The blocks cost a cleared vector (2.3 us of launch) and their atomics; the
+// other repeats cells, which weighs what the body weighs, and the registers it
+// needs tell light from heavy bodies.  Cell integral in us, rows / blocks:
+//   under 100 registers: P1 196 thousand cells 7.7 / 8.7, 750 thousand 19.3 /
+//     14.0; P2 94 thousand 8.1 / 8.5; vector P2 664 thousand 59 / 51;
+//   P3 source (126): 10 thousand cells 15.0 / 15.1, 83 thousand 24.6 / 21.6;
+//   P2 residual with 64 points (242): 1 thousand 37 / 43, 10 thousand 61 / 41,
+//     48 thousand 97 / 48; P1 with 27 points: 3 thousand 17 / 9.
+// Cells of more than 32 nodes have no row-owning kernel: Q3 source on 14
+// thousand hexahedra 50 us, 78 us with one atomic per row.
+static bool blocks_pay(const mf_form& L, Integral& I) {
+  if (!I.k_vown) return true;
+  if (L.options.count("vector_chunk_values") || L.options.count("vector_block")) return false;
+  if (I.vown_regs == 0) {
+    int regs = 0;
+    MF_HIP(hipFuncGetAttribute(&regs, HIP_FUNC_ATTRIBUTE_NUM_REGS, I.k_vown));
+    I.vown_regs = std::max(1, regs);
+  }
+  return I.n >= (I.vown_regs < 100 ? 400000 : I.vown_regs < 160 ? 64000 : 2500);
+}
+
+// Blocks of at most 256 entities (down to 64 where that leaves fewer than
+// three blocks per CU) whose rows fit 64 KB of LDS; null when rows are shared so
+// little that the blocks hold fewer than half their entities.
+static VectorBlocks* vector_blocks(mf_form* L, const Integral& I) {
+  auto it = L->vblocks.find(I.index);
+  if (it != L->vblocks.end()) return it->second.get();
+  const mf_dofmap* d0 = L->dm[0];
+  const int nd = d0->nd, bs = d0->bs;
+  auto B = std::make_unique<VectorBlocks>();
+  while (B->threads > 64 && I.n < 3LL * L->ctx->num_cus * B->threads) B->threads /= 2;
+  const size_t cap = 8192 / bs;                          // nodes per block
+  std::vector<int32_t> ent{0}, ptr{0}, row, place(d0->num_nodes, -1), nodes;
+  std::vector<uint16_t> slot(static_cast<size_t>(I.n) * nd);
+  for (int64_t e = 0; e < I.n;) {
+    const int64_t e0 = e;
+    nodes.clear();
+    for (; e < I.n && e - e0 < (int64_t)B->threads; ++e) {
+      const size_t before = nodes.size();
+      const int32_t* dm = &d0->host[(int64_t)I.h_ents[e] * nd];
+      for (int i = 0; i < nd; ++i)
+        if (place[dm[i]] < 0) {
+          place[dm[i]] = 0;
+          nodes.push_back(dm[i]);
+        }
+      if (nodes.size() > cap) {                          // this entity starts the next block
+        for (size_t k = before; k < nodes.size(); ++k) place[nodes[k]] = -1;
+        nodes.resize(before);
+        break;
+      }
+    }
+    if (e == e0) return (L->vblocks[I.index] = nullptr).get();   // one entity's rows exceed a block
+    std::sort(nodes.begin(), nodes.end());
+    for (size_t k = 0; k < nodes.size(); ++k) place[nodes[k]] = static_cast<int32_t>(k);
+    for (int64_t q = e0; q < e; ++q)
+      for (int i = 0; i < nd; ++i)
+        slot[q * nd + i] = static_cast<uint16_t>(place[d0->host[(int64_t)I.h_ents[q] * nd + i]]);
+    for (int32_t r : nodes) place[r] = -1;
+    row.insert(row.end(), nodes.begin(), nodes.end());
+    ent.push_back(static_cast<int32_t>(e));
+    ptr.push_back(static_cast<int32_t>(row.size()));
+    B->lds = std::max(B->lds, static_cast<uint32_t>(8 * bs * nodes.size()));
+  }
+  B->n = static_cast<int64_t>(ent.size()) - 1;
+  if (B->n * B->threads > 2 * std::max<int64_t>(I.n, B->threads)) return (L->vblocks[I.index] = nullptr).get();
+  B->ent.upload(ent);
+  B->ptr.upload(ptr);
+  B->row.upload(row);
+  B->slot.upload(slot);
+  return (L->vblocks[I.index] = std::move(B)).get();
+}
+
 LiftList build_lift_list(const mf_form& f, const Integral& I, const mf_bc& bc, hipStream_t s) {
   const mf_dofmap* d0 = f.dm[0];
   const mf_dofmap* d1 = f.dm[1];
@@ -802,7 +875,16 @@ void assemble_vector(mf_form* L, double* b, int64_t n, int zero, hipStream_t s) 
   MF_CHECK(mode != 3, MF_EUNSUPPORTED, "cell-owner DG vector kernel unavailable for this form");
   Integral* owner = nullptr;
   std::shared_ptr<OwnerPlan> plan;
-  if (mode != 1)
+  VectorBlocks* blocks = nullptr;
+  if (mode == 0 || mode == 4)
+    for (auto& I : L->ints)
+      if (I->type == MF_CELL && I->n && I->k_vblk) {
+        if (mode == 4 || blocks_pay(*L, *I)) blocks = vector_blocks(L, *I);
+        if (blocks) owner = I.get();
+        break;
+      }
+  MF_CHECK(!(mode == 4 && !blocks), MF_EUNSUPPORTED, "no blocks of cells for this form");
+  if (mode != 1 && !blocks)
     for (auto& I : L->ints)
       if (I->type == MF_CELL && I->k_vown) {
         plan = vector_plan(L, *I);
@@ -810,7 +892,13 @@ void assemble_vector(mf_form* L, double* b, int64_t n, int zero, hipStream_t s) 
         break;
       }
   MF_CHECK(!(mode == 2 && !owner), MF_EUNSUPPORTED, "owner-computes vector kernel unavailable");
-  if (owner) {
+  if (blocks) {
+    if (zero) k_fill(b, n, 0.0, s);
+    launch(owner->k_vblk, static_cast<uint32_t>((blocks->n + 7) / 8 * 8), blocks->threads, blocks->lds,
+           s, static_cast<int32_t>(blocks->n), blocks->ent.ptr, blocks->ptr.ptr, blocks->row.ptr,
+           blocks->slot.ptr, owner->d_ents.ptr, L->mesh->cells.ptr, L->mesh->x.ptr, L->packed.ptr,
+           L->consts.ptr, b);
+  } else if (owner) {
     const int64_t nx = 8, per = (plan->nchunks + nx - 1) / nx;
     launch(owner->k_vown, static_cast<uint32_t>(per * nx),
            static_cast<uint32_t>(L->opt("vector_block", 256)), 0, s,

@@ -252,6 +252,8 @@ struct Integral {
   int index = 0;                      // position in the form
   hipFunction_t k_ten = nullptr;      // element tensors into a workspace
   hipFunction_t k_mat = nullptr, k_vec = nullptr, k_lift = nullptr, k_owner = nullptr;
+  hipFunction_t k_vblk = nullptr;     // rank 1: blocks of consecutive cells
+  int vown_regs = 0;                  // registers of k_vown (0: not queried)
   hipFunction_t k_vown = nullptr, k_slift = nullptr, k_hlift = nullptr, k_prep = nullptr;
   hipFunction_t k_hprep = nullptr, k_howner[3] = {nullptr, nullptr, nullptr};  // FP64, FP32, BF16
   hipFunction_t k_scl = nullptr;      // rank 0: per-block partial sums
@@ -288,6 +290,15 @@ struct GatherPlan {
   DevArray<int2> pos;
   DevArray<double> ws;
 };
+// Blocks of consecutive entities of a cell integral of a linear form: entities
+// ent[k] .. ent[k + 1], the block's distinct nodes row[ptr[k] ..] (ascending)
+// and the place of every (entity, local node) among them.
+struct VectorBlocks {
+  int64_t n = 0;
+  uint32_t threads = 256, lds = 0;    // threads per block, LDS bytes of the largest block
+  DevArray<int32_t> ent, ptr, row;
+  DevArray<uint16_t> slot;
+};
 struct OwnerPlan;   // cooperative owner-computes schedule (matrix.cpp)
 // Cell-owner schedule for forms on discontinuous spaces (matrix.cpp)
 struct DGPlan {
@@ -314,6 +325,7 @@ struct mf_form {
   std::string source;
   std::map<std::string, int64_t> options;
   std::map<int, std::shared_ptr<mf::OwnerPlan>> vplans;   // owner-computes vector schedules
+  std::map<int, std::unique_ptr<mf::VectorBlocks>> vblocks;   // blocks of cell integrals
   hipFunction_t k_dgown = nullptr;    // cell-owner kernel over all integrals (DG spaces)
   std::shared_ptr<mf::DGPlan> dgvplan;                    // its vector schedule
   bool dgvplan_tried = false;

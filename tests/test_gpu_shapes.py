@@ -95,13 +95,39 @@ def test_hexahedral_lifting(degree, n, share, noalloc):
     assert _rel(b.to_host(), ref) <= TOL
 
 
+@pytest.mark.parametrize("kernel", [0, 4])
 @pytest.mark.parametrize("n,k", [(1, 1), (9, 1), (17, 1), (2, 3), (9, 2), (13, 3)])
-def test_right_hand_side_rows_per_workgroup(n, k):
+def test_right_hand_side_rows_per_workgroup(n, k, kernel):
     import cudolfinx as cufem
-    print(f"[gpu-test] right-hand side P{k} n={n}", flush=True)
+    print(f"[gpu-test] right-hand side P{k} n={n} vector_kernel={kernel}", flush=True)
     V, _, L = _poisson(n, k)
     asm = cufem.CUDAAssembler()
-    b = asm.assemble_vector(cufem.form(L))
+    f = cufem.form(L, options={"vector_kernel": kernel})
+    b = asm.assemble_vector(f)
+    asm.synchronize()
+    ref = cpu.OracleAssembler(L).assemble_vector()
+    assert _rel(b.to_host(), ref) <= TOL
+    asm.assemble_vector(f, b, zero=False)
+    asm.synchronize()
+    assert _rel(b.to_host(), 2 * ref) <= TOL
+
+
+@pytest.mark.parametrize("which,n", [("elasticity", 1), ("elasticity", 4), ("hex", 1), ("hex", 5),
+                                     ("shuffled", 4)])
+def test_right_hand_side_in_blocks_of_cells(which, n):
+    """Several components with a facet integral, 64 nodes per cell, and an order
+    of the cells in which a block's cells share no rows."""
+    import cudolfinx as cufem
+    print(f"[gpu-test] right-hand side in blocks: {which} n={n}", flush=True)
+    if which == "elasticity":
+        L = _elasticity(n)[2]
+    elif which == "hex":
+        L = problems.helmholtz_q3(n, seed=2).L
+    else:
+        L = _poisson(n, 2)[2]
+        L.integrals[0].entities = np.random.default_rng(0).permutation(L.integrals[0].entities)
+    asm = cufem.CUDAAssembler()
+    b = asm.assemble_vector(cufem.form(L, options={"vector_kernel": 4}))
     asm.synchronize()
     assert _rel(b.to_host(), cpu.OracleAssembler(L).assemble_vector()) <= TOL
 
