@@ -712,7 +712,9 @@ int mf_spmv(mf_matrix* A, const double* d_x, double* d_y, mf_stream s) {
     MF_CHECK(A->values, MF_ESTATE, "matrix has no values");
     MF_CHECK(d_x != d_y, MF_EINVAL, "x and y must not alias");
     if (A->form) use_device(A->form->ctx);
-    mf::k_spmv(A->nrows, A->nnz, A->row_ptr.ptr, A->cols.ptr, A->values, d_x, d_y, S(s));
+    if (!mf::k_spmv_block(A->bs0, A->bs1, A->nrows_b, A->nnz_b, A->rpb.ptr, A->colsb.ptr, A->values,
+                          d_x, d_y, S(s)))
+      mf::k_spmv(A->nrows, A->nnz, A->row_ptr.ptr, A->cols.ptr, A->values, d_x, d_y, S(s));
   });
 }
 

@@ -113,6 +113,10 @@ void k_scatter_add(double* dst, const double* src, const int32_t* map, int64_t n
 // y = A x (CSR, int32 indices, FP64 values); d = diag(A)
 void k_spmv(int64_t nrows, int64_t nnz, const int32_t* rp, const int32_t* cols, const double* v,
             const double* x, double* y, hipStream_t s);
+// the same for a bs-unrolled CSR from its blocked pattern (2 or 3 components;
+// false: not this shape, nothing launched)
+bool k_spmv_block(int bs0, int bs1, int64_t nrows_b, int64_t nnz_b, const int32_t* rpb,
+                  const int32_t* colsb, const double* v, const double* x, double* y, hipStream_t s);
 void k_diagonal(int64_t nrows, const int32_t* rp, const int32_t* cols, const double* v, double* d,
                 hipStream_t s);
 void k_fill_i32(int32_t* x, int64_t n, int32_t v, hipStream_t s);

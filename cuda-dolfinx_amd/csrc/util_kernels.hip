@@ -376,6 +376,13 @@ __global__ void lift_list_kernel(int32_t* __restrict__ list, int32_t* __restrict
   }
 }
 
+// Workgroups land on the 8 XCDs in turn; with this order (grid a multiple of 8)
+// each XCD takes a contiguous eighth of the rows, so the part of x that they
+// share stays in its own L2.
+__device__ __forceinline__ int64_t xcd_block() {
+  return (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+}
+
 // y = A x for a CSR matrix (int32 row_ptr / cols, FP64 values): G lanes per
 // row (G a power of two <= 64, so a wave holds 64 / G rows); each lane sums a
 // strided part of its row and the lanes of a row combine with shuffles, in a
@@ -386,15 +393,93 @@ __global__ void __launch_bounds__(kBlock) spmv_kernel(int64_t nrows, const int32
                                                       const double* __restrict__ v,
                                                       const double* __restrict__ x,
                                                       double* __restrict__ y) {
-  const int64_t row = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / G;
+  // short rows: the x gathers weigh most (P1 50^3 7.3 -> 5.5 us, DG1 32^3 47.7 ->
+  // 43.5 us in XCD order); long rows stream their values (Q3 24^3: 2% slower)
+  const int64_t wg = G <= 8 ? xcd_block() : (int64_t)blockIdx.x;
+  const int64_t row = (wg * kBlock + threadIdx.x) / G;
   const int lane = threadIdx.x & (G - 1);
   double acc = 0.0;
   if (row < nrows) {
     const int32_t e = rp[row + 1];
-    for (int32_t k = rp[row] + lane; k < e; k += G) acc += v[k] * x[cols[k]];
+    int32_t k = rp[row] + lane;
+    for (; k + G < e; k += 2 * G) {
+      const double v0 = v[k], v1 = v[k + G];
+      const double x0 = x[cols[k]], x1 = x[cols[k + G]];
+      acc += v0 * x0;
+      acc += v1 * x1;
+    }
+    if (k < e) acc += v[k] * x[cols[k]];
   }
   for (int o = G / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, G);
   if (row < nrows && lane == 0) y[row] = acc;
+}
+
+// y = A x for the bs-unrolled CSR of a BS-component space: the BS scalar rows of
+// a blocked row hold the same columns, whole nodes at a time, so G lanes take
+// the blocked row together, each x value is loaded once for BS rows and the
+// columns come from the blocked pattern, 4 bytes per BS x BS values instead of
+// 4 per value.  Bound by memory: (8 + 4 / BS^2) bytes per value.
+template <int BS, int G>
+__global__ void __launch_bounds__(kBlock) spmv_block_kernel(int64_t nrows_b,
+                                                            const int32_t* __restrict__ rpb,
+                                                            const int32_t* __restrict__ colsb,
+                                                            const double* __restrict__ v,
+                                                            const double* __restrict__ x,
+                                                            double* __restrict__ y) {
+  const int64_t row = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / G;
+  const int lane = threadIdx.x & (G - 1);
+  double acc[BS];
+#pragma unroll
+  for (int a = 0; a < BS; ++a) acc[a] = 0.0;
+  if (row < nrows_b) {
+    const int32_t s = rpb[row], n = BS * (rpb[row + 1] - s);
+    const double* vr = v + (int64_t)BS * BS * s;
+    int32_t t = lane;
+    for (; t + G < n; t += 2 * G) {
+      const int32_t u = t + G;
+      const double xt = x[(int64_t)BS * colsb[s + t / BS] + t % BS];
+      const double xu = x[(int64_t)BS * colsb[s + u / BS] + u % BS];
+      double vt[BS], vu[BS];
+#pragma unroll
+      for (int a = 0; a < BS; ++a) {
+        vt[a] = vr[(int64_t)a * n + t];
+        vu[a] = vr[(int64_t)a * n + u];
+      }
+#pragma unroll
+      for (int a = 0; a < BS; ++a) acc[a] = acc[a] + vt[a] * xt + vu[a] * xu;
+    }
+    if (t < n) {
+      const double xt = x[(int64_t)BS * colsb[s + t / BS] + t % BS];
+#pragma unroll
+      for (int a = 0; a < BS; ++a) acc[a] += vr[(int64_t)a * n + t] * xt;
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < BS; ++a)
+    for (int o = G / 2; o > 0; o >>= 1) acc[a] += __shfl_xor(acc[a], o, G);
+  if (row < nrows_b) {
+#pragma unroll
+    for (int a = 0; a < BS; ++a)
+      if (lane == a) y[(int64_t)BS * row + a] = acc[a];
+  }
+}
+
+template <int BS>
+void spmv_block(int64_t nrows_b, int64_t nnz_b, const int32_t* rpb, const int32_t* colsb,
+                const double* v, const double* x, double* y, hipStream_t s) {
+  // lanes per blocked row: about three of its columns each
+  const double mean = (double)BS * nnz_b / (double)nrows_b;
+  const int g = mean > 96 ? 64 : (mean > 48 ? 32 : (mean > 24 ? 16 : 8));
+  const int64_t threads = nrows_b * g;
+  MF_CHECK(threads / kBlock < (1LL << 31) - 16, MF_ESHAPE, "matrix too large for one SpMV launch");
+  const uint32_t grid = static_cast<uint32_t>((threads + kBlock - 1) / kBlock);
+  switch (g) {
+    case 8: spmv_block_kernel<BS, 8><<<grid, kBlock, 0, s>>>(nrows_b, rpb, colsb, v, x, y); break;
+    case 16: spmv_block_kernel<BS, 16><<<grid, kBlock, 0, s>>>(nrows_b, rpb, colsb, v, x, y); break;
+    case 32: spmv_block_kernel<BS, 32><<<grid, kBlock, 0, s>>>(nrows_b, rpb, colsb, v, x, y); break;
+    default: spmv_block_kernel<BS, 64><<<grid, kBlock, 0, s>>>(nrows_b, rpb, colsb, v, x, y); break;
+  }
+  MF_HIP(hipGetLastError());
 }
 
 // d[r] = A[r][r] (0 where the pattern has no diagonal entry); columns sorted.
@@ -599,8 +684,8 @@ void k_spmv(int64_t nrows, int64_t nnz, const int32_t* rp, const int32_t* cols, 
   int g = 2;
   while (g < 64 && g * 3 < mean) g *= 2;
   const int64_t threads = nrows * g;
-  MF_CHECK(threads / kBlock < (1LL << 31), MF_ESHAPE, "matrix too large for one SpMV launch");
-  const uint32_t grid = static_cast<uint32_t>((threads + kBlock - 1) / kBlock);
+  MF_CHECK(threads / kBlock < (1LL << 31) - 16, MF_ESHAPE, "matrix too large for one SpMV launch");
+  const uint32_t grid = static_cast<uint32_t>((threads + kBlock - 1) / kBlock + 7) / 8 * 8;
   switch (g) {
     case 2: spmv_kernel<2><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y); break;
     case 4: spmv_kernel<4><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y); break;
@@ -610,6 +695,15 @@ void k_spmv(int64_t nrows, int64_t nnz, const int32_t* rp, const int32_t* cols, 
     default: spmv_kernel<64><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y); break;
   }
   MF_HIP(hipGetLastError());
+}
+
+bool k_spmv_block(int bs0, int bs1, int64_t nrows_b, int64_t nnz_b, const int32_t* rpb,
+                  const int32_t* colsb, const double* v, const double* x, double* y, hipStream_t s) {
+  if (bs0 != bs1 || (bs0 != 2 && bs0 != 3)) return false;
+  if (nrows_b <= 0) return true;
+  if (bs0 == 2) spmv_block<2>(nrows_b, nnz_b, rpb, colsb, v, x, y, s);
+  else spmv_block<3>(nrows_b, nnz_b, rpb, colsb, v, x, y, s);
+  return true;
 }
 
 void k_diagonal(int64_t nrows, const int32_t* rp, const int32_t* cols, const double* v, double* d,

@@ -193,3 +193,37 @@ def test_gathered_blocks_of_a_vector_form():
     ref = np.where(m0[rows] | m1[cols], 0.0, full)
     ref[(rows == cols) & m0[rows]] = 1.0
     assert _rel(A.csr()[2], ref) <= TOL
+
+
+@pytest.mark.parametrize("which,n", [("elasticity", 1), ("elasticity", 4), ("p1", 1), ("p1", 9), ("p3", 3),
+                                     ("q3", 2), ("dg1", 2), ("two", 1), ("two", 5)])
+def test_product_rows_of_any_length(which, n):
+    """y = A x from the blocked pattern (three components) and row by row."""
+    import scipy.sparse as sp
+    import torch
+    import cudolfinx as cufem
+    print(f"[gpu-test] product {which} n={n}", flush=True)
+    if which == "elasticity":
+        a = _elasticity(n)[1]
+    elif which == "q3":
+        a = problems.helmholtz_q3(n).a
+    elif which == "dg1":
+        a = problems.dg_plaplace(n).a
+    elif which == "two":
+        V = functionspace(create_unit_cube(n), ("P", 1), shape=(2,))
+        name = "tabulate_tensor_integral_two"
+        body = "{\n  for (int i = 0; i < 8; ++i)\n    for (int j = 0; j < 8; ++j) A[8 * i + j] += 1.0 / (1 + i + 2 * j);\n}\n"
+        a = forms.Form(2, [V, V], [forms.Integral("cell", -1, np.arange(V.mesh.num_cells, dtype=np.int32),
+                                                  name, forms._SIG.format(name=name) + "\n" + body)])
+    else:
+        a = _poisson(n, int(which[1]))[1]
+    asm = cufem.CUDAAssembler()
+    A = asm.assemble_matrix(cufem.form(a))
+    asm.synchronize()
+    rp, cols, vals = A.csr()
+    x = np.random.default_rng(1).uniform(-1, 1, A.ncols)
+    y = torch.full((A.nrows,), 7.0, dtype=torch.float64, device="cuda")
+    A.mult(torch.from_numpy(x).cuda(), y)
+    S = sp.csr_matrix((vals, cols, rp), shape=(A.nrows, A.ncols))
+    # at most 400 products per row, each rounded once: 400 eps of the absolute sums
+    assert np.all(np.abs(y.cpu().numpy() - S @ x) <= 400 * 2.2e-16 * (abs(S) @ np.abs(x)) + 1e-300)
