@@ -356,8 +356,11 @@ void compile_form(mf_form* f, int verbose) {
   {
     MF_CHECK(!f->ints.empty(), MF_ESTATE, "form has no integrals");
     use_device(f->ctx);
-    for (auto& I : f->ints)                                           // the kernels below are new
+    for (auto& I : f->ints) {                                         // the kernels below are new
       I->owner_grid = I->owner_grid32 = I->owner_gridp = I->owner_gridp32 = 0;
+      for (auto& g : I->howner_grid) g = 0;
+      I->vown_regs = 0;
+    }
     ++f->gen;                          // schedules built for an earlier compile are stale
     f->vplans.clear();
     if (!f->consts.ptr) {
@@ -387,8 +390,8 @@ void compile_form(mf_form* f, int verbose) {
             const char* names[3] = {"howner64", "howner32", "howner16"};
             for (int v = 0; v < 3; ++v)
               I->k_howner[v] = f->mod->get(mf::kernel_name(names[v], I->type, I->index));
-            I->record_bytes = 464;
-            I->records.alloc(f->mesh->num_cells * I->record_bytes / 8);
+            I->record_bytes = 8;                       // constrained columns as bits
+            I->records.alloc(f->mesh->num_cells);
           }
         } else if (I->type == MF_CELL && !I->staged_src.empty()) {
           if (mf::staged_lift_emitted(*I))

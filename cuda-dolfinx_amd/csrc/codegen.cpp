@@ -400,7 +400,7 @@ int hex_batch(const mf_form& f, const Integral& I, int prec) {
   const int64_t budget = f.opt("owner_lds", 78 * 1024);
   const int64_t fixed = 8 * cap + 4 * (maxr + 1) + 4 * f.opt("owner_pairs", 384) + 64;
   const int64_t nq = (int64_t)nq1 * nq1 * nq1;
-  const int64_t per_cell = 464 + 4 + (prec == 64 ? 8 * (8 * nq + 8) : 4 * 8 * nq);
+  const int64_t per_cell = 8 * 24 + 8 + (prec == 64 ? 8 * (8 * nq + 8) : 4 * 8 * nq);
   int64_t nb = (budget - fixed) / per_cell;
   nb = std::min<int64_t>(nb, f.opt("owner_nb", 16));
   MF_CHECK(nb >= 1, MF_EUNSUPPORTED, "hexahedral owner kernel does not fit the LDS budget");
@@ -493,7 +493,6 @@ extern const char* kOwnerVectorParams;
 extern const char* kStagedLiftTemplate;
 extern const char* kCellRecord;
 extern const char* kPrepTemplate;
-extern const char* kHexRecord;
 extern const char* kHexPrepTemplate;
 extern const char* kHexOwnerTemplate;
 extern const char* kHexLiftTemplate;
@@ -1070,7 +1069,6 @@ std::string generate_form_source(const mf_form& f) {
         }
         if (hex_owner_supported(f, *I)) {
           m["$TAG"] = "H" + std::to_string(I->index);
-          os << subst(kHexRecord, m);
           m["$KNAME"] = kernel_name("hprep", I->type, I->index);
           os << subst(kHexPrepTemplate, m);
           for (int prec : {64, 32, 16}) {

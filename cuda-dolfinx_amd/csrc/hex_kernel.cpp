@@ -31,38 +31,19 @@
 
 namespace mf {
 
-const char* kHexRecord = R"(
-#ifndef MF_HREC_$TAG
-#define MF_HREC_$TAG
-struct __attribute__((aligned(16))) mf_hrec_$TAG {
-  double x[8][3];
-  int32_t d[HX_ND];
-  uint32_t bits[(HX_ND + 31) / 32];
-};
-#endif
-)";
-
+// Constrained columns of every cell as bits (bit j: local node j), for the
+// assembly that follows: one wave per cell, lane = local node.
 const char* kHexPrepTemplate = R"(
 extern "C" __global__ void __launch_bounds__(256)
-$KNAME(const int32_t n, const int32_t* __restrict__ ents, const int32_t* __restrict__ geo,
-       const double* __restrict__ xg, const int32_t* __restrict__ dm0,
-       const uint8_t* __restrict__ nb0, mf_hrec_$TAG* __restrict__ rec)
+$KNAME(const int32_t n, const int32_t* __restrict__ ents, const int32_t* __restrict__ dm0,
+       const uint8_t* __restrict__ nb0, uint64_t* __restrict__ cmask)
 {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  static_assert(HX_ND == 64, "one lane per local node");
+  const int e = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (e >= n) return;
   const int64_t c = ents[e];
-  mf_hrec_$TAG r;
-  for (int v = 0; v < 8; ++v) {
-    const int64_t gv = geo[c * 8 + v];
-    r.x[v][0] = xg[3 * gv]; r.x[v][1] = xg[3 * gv + 1]; r.x[v][2] = xg[3 * gv + 2];
-  }
-  for (int w = 0; w < (HX_ND + 31) / 32; ++w) r.bits[w] = 0;
-  for (int l = 0; l < HX_ND; ++l) {
-    const int32_t node = dm0[c * HX_ND + l];
-    r.d[l] = node;
-    if (nb0 && nb0[node]) r.bits[l >> 5] |= 1u << (l & 31);
-  }
-  rec[c] = r;
+  const uint64_t bits = __ballot(nb0[dm0[c * 64 + (threadIdx.x & 63)]] != 0);
+  if ((threadIdx.x & 63) == 0) cmask[c] = bits;
 }
 )";
 
@@ -245,16 +226,19 @@ static __device__ __forceinline__ short mf_to_bf16(float f)
 
 
 extern "C" __global__ void __launch_bounds__($HBLOCK)
+#if MF_HX_PREC != 64
+__attribute__((amdgpu_waves_per_eu(4)))                // two workgroups of eight waves per CU
+#endif
 $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
-       const int32_t* __restrict__ item_cell, const int32_t* __restrict__ pair_list,
-       const uint16_t* __restrict__ pair_pos, const mf_hrec_$TAG* __restrict__ rec,
+       const int32_t* __restrict__ item_cell, const int32_t* __restrict__ item_geo,
+       const int32_t* __restrict__ pair_list, const uint16_t* __restrict__ pair_pos,
+       const double* __restrict__ xg, const uint64_t* __restrict__ cmask,
        const int32_t* __restrict__ rpb,
        const int32_t* __restrict__ diag_pos, const uint8_t* __restrict__ nb0,
        double* __restrict__ values, const double diag, const int flags)
 {
   constexpr int K1 = HX_K + 1, ND = HX_ND, M1 = HX_NQ1, NQ = M1 * M1 * M1;
   constexpr int NB = $HNB, CAP = $OCAP, MAXR = $OMAXR, MAXP = $OMAXP;
-  constexpr int RW = sizeof(mf_hrec_$TAG) / 16;
   constexpr int DS = 8;                              // D_q record: G00 G01 G02 G11 G12 G22 M pad
 #if MF_HX_PREC == 64
   typedef double real;
@@ -269,7 +253,8 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
 #endif
   __shared__ __attribute__((aligned(16))) double acc[CAP];
   __shared__ int32_t lrp[MAXR + 1];
-  __shared__ mf_hrec_$TAG srec[NB];
+  __shared__ double sx[NB * 24];                     // vertex coordinates of the batch's cells
+  __shared__ uint64_t smask[NB];                     // their constrained columns
   __shared__ __attribute__((aligned(16))) real sD[NB * DCELL];
   __shared__ int32_t spair[MAXP];
   // 1D basis values / derivatives at the 1D points, [q][n], in LDS: the
@@ -277,18 +262,28 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
   // would be a global load (and a wait) per quadrature line
   __shared__ real sTL[M1 * K1], sTD[M1 * K1];
 
-  const int k = mf_xcd_chunk(nchunks);
-  if (k < 0) return;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int lane = tid & 63, wave = tid >> 6, nwave = nt >> 6;
-  const int4 m0 = reinterpret_cast<const int4*>(chunk_meta)[3 * k];
-  const int4 m1 = reinterpret_cast<const int4*>(chunk_meta)[3 * k + 1];
-  const int4 m2 = reinterpret_cast<const int4*>(chunk_meta)[3 * k + 2];
-  const int32_t r0 = m0.x, r1 = m0.y, i0 = m0.z, i1 = m0.w;
-  const int32_t cb0 = m1.x, ncb = m1.y, base = m1.z, seglen = m1.w;
-  const int32_t p0 = m2.x, p1 = m2.y;
-  const int nr = r1 - r0, npc = p1 - p0;
-  for (int p = tid; p < npc; p += nt) spair[p] = pair_list[p0 + p];
+  // Persistent: the grid holds the resident workgroups (a multiple of 8); those
+  // of XCD blockIdx % 8 walk its contiguous eighth of the chunks with stride
+  // gridDim / 8.  Everything the next step (the chunk's next batch of cells, or
+  // the next chunk) reads from memory is loaded into registers while this one
+  // computes, its dependent loads issued a phase apart, and the accumulator is
+  // cleared by the write-out.  24^3 cells, 47 M values, 0.38 GB: 370 us (FP64),
+  // 510 us (FP32) against 390 and 520 us with one workgroup per chunk, and 436
+  // and 518 us when the coordinates and dofs came from 464-byte cell records,
+  // rows were searched in chunks and chunks were filled up.  What is left is the
+  // arithmetic of the 4-5 tiles of a chunk (FP64 about 140 us of issue, FP32
+  // 190 us of MFMA) and the geometry in two workgroups' phases per CU.
+  constexpr int NTH = $HBLOCK;
+  constexpr int PFX = (NB * 24 + NTH - 1) / NTH, PFP = (MAXP + NTH - 1) / NTH;
+  static_assert(MAXR < NTH && NB <= NTH, "one row and one cell per thread");
+  const int tid = threadIdx.x, nt = NTH;
+  const int lane = tid & 63, wave = tid >> 6, nwave = NTH >> 6;
+  const int nx = 8, gx = gridDim.x / nx, per = (nchunks + nx - 1) / nx;
+  const int kend = min(nchunks, ((int)blockIdx.x % nx + 1) * per);
+  int k = ((int)blockIdx.x % nx) * per + (int)blockIdx.x / nx;
+  if (k >= kend) return;
+  const int4* meta = reinterpret_cast<const int4*>(chunk_meta);
+  int4 m0 = meta[3 * k], m1 = meta[3 * k + 1], m2 = meta[3 * k + 2];
   if (tid < M1 * K1) {
 #if MF_HX_PREC == 64
     sTL[tid] = HX_L[tid / K1][tid % K1];
@@ -301,54 +296,103 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
   {
     mf_d2* a2 = reinterpret_cast<mf_d2*>(acc);
     const mf_d2 z = {0.0, 0.0};
-    for (int p = tid; p < (seglen + 1) / 2; p += nt) a2[p] = z;
+    for (int p = tid; p < CAP / 2; p += nt) a2[p] = z;
   }
-  for (int p = tid; p <= nr; p += nt) lrp[p] = rpb[r0 + p] - cb0;
-
-  // cell records of a batch, fetched into registers one batch ahead (the
-  // next batch's loads are in flight while this batch's tiles run)
-  constexpr int NTH = $HBLOCK, PFH = (NB * RW + NTH - 1) / NTH;
-  int4 pfr[PFH];
-  {
+  // registers of the step ahead: vertices (1), then coordinates and constrained
+  // columns (2) of its cells; for a chunk also its pairs and its row (row tid)
+  int pfv[PFX], pfc = 0, pfp[PFP], pfr = 0, pfd = -1;
+  double pfx[PFX];
+  uint64_t pfm = 0;
+  auto fetch1 = [&](const int ib, const int nb, const int tid) {
 #pragma clang loop unroll(full)
-    for (int t = 0; t < PFH; ++t) {
-      // clamped, unconditional loads keep pfr in registers (every chunk has >= 1 item)
-      const int u = min(tid + t * NTH, min(NB, i1 - i0) * RW - 1);
-      const int b = u / RW, w = u - b * RW;
-      pfr[t] = reinterpret_cast<const int4*>(rec)[(int64_t)item_cell[i0 + b] * RW + w];
+    for (int t = 0; t < PFX; ++t)                      // clamped, unconditional loads stay in registers
+      pfv[t] = item_geo[(int64_t)ib * 8 + min(tid + t * NTH, max(nb * 24 - 1, 0)) / 3];
+    pfc = item_cell[ib + min(tid, max(nb - 1, 0))];    // (the lists are padded by one cell and pair)
+  };
+  auto fetch2 = [&](const int nb, const int tid) {
+#pragma clang loop unroll(full)
+    for (int t = 0; t < PFX; ++t)
+      pfx[t] = xg[3 * (int64_t)pfv[t] + min(tid + t * NTH, max(nb * 24 - 1, 0)) % 3];
+    pfm = cmask ? cmask[pfc] : 0;
+  };
+  auto fetch_rows = [&](const int4 c0, const int4 c1, const int4 c2, const int tid) {
+#pragma clang loop unroll(full)
+    for (int t = 0; t < PFP; ++t) pfp[t] = pair_list[max(min(c2.x + tid + t * NTH, c2.y - 1), c2.x)];
+    pfr = rpb[min(c0.x + tid, c0.y)] - c1.x;           // rpb[c0.y] closes the last row
+    // Dirichlet rows: position of their diagonal entry (-1: none)
+    const int row = min(c0.x + tid, c0.y - 1);
+    const int dp = diag_pos[row];
+    const bool on = (flags & 2) && nb0 && nb0[row];
+    pfd = on && c0.x + tid < c0.y ? dp : -1;
+  };
+  auto store_cells = [&](const int nb) {
+#pragma clang loop unroll(full)
+    for (int t = 0; t < PFX; ++t) {
+      const int u = tid + t * NTH;
+      if (u < nb * 24) sx[u] = pfx[t];
     }
-  }
+    if (tid < nb) smask[tid] = pfm;
+  };
+  auto store_rows = [&](const int4 c0, const int4 c2) {
+#pragma clang loop unroll(full)
+    for (int t = 0; t < PFP; ++t) {
+      const int u = tid + t * NTH;
+      if (u < c2.y - c2.x) spair[u] = pfp[t];
+    }
+    if (tid <= c0.y - c0.x) lrp[tid] = pfr;
+    // constrained rows get no contributions (their pairs are masked), so their
+    // diagonal is set up front
+    if (pfd >= 0) acc[pfr + pfd] = diag;
+  };
+  fetch1(m0.z, min(NB, m0.w - m0.z), tid);
+  fetch_rows(m0, m1, m2, tid);
+  fetch2(min(NB, m0.w - m0.z), tid);
+  __syncthreads();                                     // accumulator cleared before a diagonal goes in
+  store_cells(min(NB, m0.w - m0.z));
+  store_rows(m0, m2);
 
+  while (true) {
+  const int32_t i0 = m0.z, i1 = m0.w, base = m1.z, seglen = m1.w, p0 = m2.x;
+  const int npc = m2.y - m2.x;
+  const int kn = k + gx;
+  const bool more = kn < kend;
+  const int4 n0 = meta[3 * (more ? kn : k)], n1 = meta[3 * (more ? kn : k) + 1], n2 = meta[3 * (more ? kn : k) + 2];
   int pb = 0;
-  for (int ib = i0; ib < i1; ib += NB) {
+  for (int ib = i0;; ib += NB) {                       // a chunk without cells takes one empty batch
     const int nb = min(NB, i1 - ib);
-    __syncthreads();                                 // previous batch done with srec / sD
-    // the batch's serial part (record staging, pair range, FP64 geometry)
-    // holds every wave of this workgroup at the next barrier, so it issues at
-    // a raised priority over the other workgroup's matrix-core contraction
-    __builtin_amdgcn_s_setprio(2);
-    {
-      int4* dst = reinterpret_cast<int4*>(srec);
-#pragma clang loop unroll(full)
-      for (int t = 0; t < PFH; ++t) {
-        const int u = tid + t * NTH;
-        if (u < nb * RW) dst[u] = pfr[t];
-      }
+    const bool last = ib + NB >= i1;
+    // the step ahead: its first item and how many cells it takes
+    const int ibx = last ? n0.z : ib + NB, nbx = min(NB, (last ? n0.w : i1) - ibx);
+    if (ib > i0) {
+      __syncthreads();                                 // previous batch done with sx / sD
+      store_cells(nb);
     }
+    __syncthreads();                                   // lists and cells visible
+    // the batch's serial part (pair range, FP64 geometry) holds every wave of
+    // this workgroup at the next barrier, so it issues at a raised priority
+    // over the other workgroup's contraction
+    __builtin_amdgcn_s_setprio(2);
+    int tid_ = tid;
+#if MF_HX_PREC != 64
+    // a thread's quadrature point is the same in every batch: keep the compiler
+    // from holding what depends on it alone (24 basis derivatives) in registers
+    // across the contraction, which would leave room for one workgroup per CU
+    asm volatile("" : "+v"(tid_));
+#endif
+    fetch1(ibx, nbx, tid_);
     int pe;
     {
       int lo2 = pb, hi2 = npc;
       const int lim = ib - i0 + nb;
       while (lo2 < hi2) {
         const int mid = (lo2 + hi2) >> 1;
-        if ((spair[mid] >> 8) < lim) lo2 = mid + 1;
+        if ((spair[mid] >> 16) < lim) lo2 = mid + 1;
         else hi2 = mid;
       }
       pe = lo2;
     }
-    __syncthreads();
     // geometry: D_q for every (cell, quadrature point), FP64
-    for (int u = tid; u < nb * NQ; u += nt) {
+    for (int u = tid_; u < nb * NQ; u += nt) {
       const int b = u / NQ, q = u - b * NQ;
       const int q1 = q % M1, q2 = (q / M1) % M1, q3 = q / (M1 * M1);
       const double X = HX_X1[q1], Y = HX_X1[q2], Z = HX_X1[q3];
@@ -359,7 +403,7 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
         const double gx = a ? 1.0 : -1.0, gy = bb ? 1.0 : -1.0, gz = c ? 1.0 : -1.0;
         const double d0 = gx * fy * fz, d1 = fx * gy * fz, d2 = fx * fy * gz;
         for (int i = 0; i < 3; ++i) {
-          const double xv = srec[b].x[v][i];
+          const double xv = sx[b * 24 + 3 * v + i];
           J[i][0] += xv * d0; J[i][1] += xv * d1; J[i][2] += xv * d2;
         }
       }
@@ -388,17 +432,10 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
       D[6] = (real)(-HX_K2 * wq);
       D[7] = (real)0;
     }
+    if (last) fetch_rows(n0, n1, n2, tid_);
+    fetch2(nbx, tid_);
     __syncthreads();
     __builtin_amdgcn_s_setprio(0);
-    if (ib + NB < i1) {
-      const int ibx = ib + NB, nbx = min(NB, i1 - ib - NB);
-#pragma clang loop unroll(full)
-      for (int t = 0; t < PFH; ++t) {
-        const int u = min(tid + t * NTH, nbx * RW - 1);
-        const int b = u / RW, w = u - b * RW;
-        pfr[t] = reinterpret_cast<const int4*>(rec)[(int64_t)item_cell[ibx + b] * RW + w];
-      }
-    }
     // contraction: one wave per 16-pair tile, all 64 columns (4 tiles of 16)
     const int np = pe - pb;
     const int ntile = (np + 15) / 16;
@@ -407,7 +444,7 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
       const int pr = t * 16 + r;
       const bool valid = pr < np;
       const int pc = pb + (valid ? pr : 0);
-      const int b = (spair[pc] >> 8) - (ib - i0), i = spair[pc] & 255;
+      const int b = (spair[pc] >> 16) - (ib - i0), i = spair[pc] & 63;
       const int ia = i % K1, ib2 = (i / K1) % K1, ic = i / (K1 * K1);
 #if MF_HX_PREC != 64
       const real* Db = &sD[b * DCELL];
@@ -423,15 +460,15 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
       // About 950 multiply-adds per row and lane against 4,350 when every
       // column's quadrature sum runs over all 64 points.
       const int jc = slot;
-      double Lx[4], Gx[4], Ly[4], Gy[4], Zl[4], Zd[4];
+      // row-relative column positions of this pair (precomputed), 32 bytes,
+      // loaded ahead of the arithmetic
+      const uint4* pp = reinterpret_cast<const uint4*>(pair_pos + ((int64_t)p0 + pc) * ND + 16 * jc);
+      const uint4 w0 = pp[0], w1 = pp[1];
+      double Lx[4], Gx[4];
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         Lx[m] = sTL[m * K1 + ia];
         Gx[m] = sTD[m * K1 + ia];
-        Ly[m] = sTL[m * K1 + ib2];
-        Gy[m] = sTD[m * K1 + ib2];
-        Zl[m] = sTL[slot * K1 + m];
-        Zd[m] = sTD[slot * K1 + m];
       }
       const double Lz = sTL[slot * K1 + ic], Gz = sTD[slot * K1 + ic];
       double YL[16], YG[16];
@@ -440,7 +477,8 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
       const double* Ds = &sD[MF_DOFF(b, 16 * slot)];
 #pragma unroll
       for (int q2 = 0; q2 < 4; ++q2) {
-        const double LyLz = Ly[q2] * Lz, GyLz = Gy[q2] * Lz, LyGz = Ly[q2] * Gz;
+        const double Ly = sTL[q2 * K1 + ib2], Gy = sTD[q2 * K1 + ib2];
+        const double LyLz = Ly * Lz, GyLz = Gy * Lz, LyGz = Ly * Gz;
         double wx[4] = {0, 0, 0, 0}, wy[4] = {0, 0, 0, 0}, wz[4] = {0, 0, 0, 0};
 #pragma unroll
         for (int q1 = 0; q1 < 4; ++q1) {
@@ -465,6 +503,12 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
             YG[ja + 4 * jb] += wz[ja] * HX_L[q2][jb];
           }
       }
+      double Zl[4], Zd[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        Zl[m] = sTL[slot * K1 + m];
+        Zd[m] = sTD[slot * K1 + m];
+      }
       double cacc[16];
 #pragma unroll
       for (int k = 0; k < 16; ++k) {
@@ -474,18 +518,11 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
         cacc[k] = mf_swap_add16(mf_swap_add32(z[0], z[2]), mf_swap_add32(z[1], z[3]));
       }
       {
-        const int prr = t * 16 + r;
-        if (prr < np) {
-          const int pcc = pb + prr;
-          const int bq = (spair[pcc] >> 8) - (ib - i0), iq = spair[pcc] & 255;
-          const mf_hrec_$TAG& R = srec[bq];
-          if (!((R.bits[iq >> 5] >> (iq & 31)) & 1u)) {
-            const int lr = R.d[iq] - r0;
-            const int lo = lrp[lr];
-            const uint32_t cbits = (R.bits[jc >> 1] >> (16 * (jc & 1))) & 0xFFFFu;
-            // row-relative column positions of this pair (precomputed), 32 bytes
-            const uint4* pp = reinterpret_cast<const uint4*>(pair_pos + ((int64_t)p0 + pcc) * ND + 16 * jc);
-            const uint4 w0 = pp[0], w1 = pp[1];
+        if (valid) {
+          const uint64_t mask = smask[b];
+          if (!((mask >> i) & 1u)) {                   // not a Dirichlet row
+            const int lo = lrp[(spair[pc] >> 6) & 1023];
+            const uint32_t cbits = (uint32_t)(mask >> (16 * jc)) & 0xFFFFu;
             const uint32_t pw[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
             int pos[16];
 #pragma unroll
@@ -561,7 +598,8 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
         const float Lz = sTL[(q3) * K1 + (ic)], Gz = sTD[(q3) * K1 + (ic)];
         float cz[4];
 #pragma unroll
-        for (int jt = 0; jt < 4; ++jt) cz[jt] = slot == 2 ? sTD[(q3) * K1 + (jt)] : sTL[(q3) * K1 + (jt)];
+        for (int jt = 0; jt < 4; ++jt)
+          cz[jt] = slot == 2 ? sTD[(q3) * K1 + (jt)] : sTL[(q3) * K1 + (jt)];
 #pragma unroll
         for (int q2 = 0; q2 < 4; ++q2) {
           const float Ly = sTL[(q2) * K1 + (ib2)], Gy = sTD[(q2) * K1 + (ib2)];
@@ -595,16 +633,15 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
           const int prr = t * 16 + slot * 4 + rr;
           const bool rv = prr < np;
           const int pcc = pb + (rv ? prr : 0);
-          const int bq = (spair[pcc] >> 8) - (ib - i0), iq = spair[pcc] & 255;
-          const mf_hrec_$TAG& R = srec[bq];
-          const bool rowok = rv && !((R.bits[iq >> 5] >> (iq & 31)) & 1u);   // Dirichlet row
-          const int lr = rv ? R.d[iq] - r0 : 0;
-          const int lo = lrp[lr];
+          const int iq = spair[pcc] & 63;
+          const uint64_t mask = smask[(spair[pcc] >> 16) - (ib - i0)];
+          const bool rowok = rv && !((mask >> iq) & 1u);                  // Dirichlet row
+          const int lo = lrp[(spair[pcc] >> 6) & 1023];
           const uint16_t* pp = pair_pos + ((int64_t)p0 + pcc) * ND;   // precomputed positions
 #pragma unroll
           for (int jt = 0; jt < 4; ++jt) {
             const int j = jt * 16 + (lane & 15);
-            ok[rr][jt] = rowok && !((R.bits[j >> 5] >> (j & 31)) & 1u);     // Dirichlet column
+            ok[rr][jt] = rowok && !((mask >> j) & 1u);                    // Dirichlet column
             pos[rr][jt] = lo + (int)pp[j];
           }
         }
@@ -617,22 +654,41 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
 #endif
     }
     pb = pe;
+    if (last) break;
   }
-  __syncthreads();
-  if ((flags & 2) && nb0) {
-    for (int lr = tid; lr < nr; lr += nt) {
-      const int32_t Rr = r0 + lr;
-      if (!nb0[Rr]) continue;
-      const int pd = diag_pos[Rr];                   // position of (Rr, Rr) in the row
-      if (pd >= 0) acc[lrp[lr] + pd] = diag;
-    }
-    __syncthreads();
-  }
+  __syncthreads();                                     // all contributions in acc
+  __builtin_amdgcn_s_setprio(2);
+  // write the segment and clear what was read
   double* out = values + (int64_t)(uint32_t)base;
   if (flags & 1) {
-    for (int p = tid; p < seglen; p += nt) __builtin_nontemporal_store(acc[p], &out[p]);
+    const int h = base & 1;                            // peel to a 16-byte boundary
+    if (h && tid == 0) {
+      __builtin_nontemporal_store(acc[0], &out[0]);
+      acc[0] = 0.0;
+    }
+    mf_d2* o2 = reinterpret_cast<mf_d2*>(out + h);
+    for (int p = tid; p < (seglen - h) >> 1; p += nt) {
+      const mf_d2 v = {acc[h + 2 * p], acc[h + 2 * p + 1]};
+      __builtin_nontemporal_store(v, &o2[p]);
+      acc[h + 2 * p] = 0.0;
+      acc[h + 2 * p + 1] = 0.0;
+    }
+    if (((seglen - h) & 1) && tid == 0) {
+      __builtin_nontemporal_store(acc[seglen - 1], &out[seglen - 1]);
+      acc[seglen - 1] = 0.0;
+    }
   } else {
-    for (int p = tid; p < seglen; p += nt) out[p] += acc[p];
+    for (int p = tid; p < seglen; p += nt) {
+      out[p] += acc[p];
+      acc[p] = 0.0;
+    }
+  }
+  if (!more) break;
+  if ((flags & 2) && nb0) __syncthreads();             // cleared before a diagonal goes in
+  store_cells(min(NB, n0.w - n0.z));
+  store_rows(n0, n2);
+  m0 = n0; m1 = n1; m2 = n2;
+  k = kn;
   }
 }
 #undef MF_DOFF

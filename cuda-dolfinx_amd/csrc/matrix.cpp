@@ -15,6 +15,7 @@ struct OwnerPlan {
   DevArray<uint32_t> item_mask;
   DevArray<uint8_t> pair_kk;
   DevArray<uint16_t> pair_pos;        // hexahedral kernel: row-relative position of each column
+  DevArray<int32_t> item_geo;         // hexahedral kernel: the 8 vertices of each item's cell
   DevArray<int32_t> diag_pos;         // hexahedral kernel: row-relative position of the diagonal
   int64_t nitems = 0, npairs = 0;
   // host copies used while building matrix schedules
@@ -54,7 +55,7 @@ std::shared_ptr<OwnerPlan> build_items(const std::vector<int32_t>& rows, const I
   }
   for (int64_t c = 0; c < nch; ++c) cnt[c + 1] += cnt[c];
   MF_CHECK(cnt[nch] < INT32_MAX, MF_EUNSUPPORTED, "too many owner items");
-  std::vector<int32_t> icell(std::max<int64_t>(1, cnt[nch]));
+  std::vector<int32_t> icell(cnt[nch] + 1, 0);
   std::vector<uint64_t> imask(std::max<int64_t>(1, cnt[nch]));
   std::vector<int64_t> pos(cnt.begin(), cnt.end() - 1);
   for (int64_t e = 0; e < I.n; ++e) {
@@ -99,24 +100,67 @@ std::shared_ptr<OwnerPlan> build_owner_plan(const mf_form& a, const Integral& I,
   const int nd = d0->nd;
   if (nd > (with_kk ? 32 : 64)) return nullptr;
   if (with_kk && d0->num_cells >= (int64_t(1) << 26)) return nullptr;   // cell << 6 | i in 32 bits
+  if (!with_kk) maxr = std::min(maxr, 1023), maxp = std::min(maxp, 32767);   // fields of pair_list
   const int bs2 = A.bs0 * A.bs1;
   std::vector<int32_t> ncell(A.nrows_b, 0);
   for (int64_t e = 0; e < I.n; ++e)
     for (int l = 0; l < nd; ++l) ncell[d0->host[(int64_t)I.h_ents[e] * nd + l]]++;
   std::vector<int32_t> rows{0};
-  int64_t seg = 0, pairs = 0;
-  int32_t r0 = 0;
-  for (int64_t r = 0; r < A.nrows_b; ++r) {
-    const int64_t len = (int64_t)bs2 * (A.h_rpb[r + 1] - A.h_rpb[r]);
-    if (len > cap || ncell[r] > maxp) return nullptr;   // a single row does not fit
-    if (seg + len > cap || r - r0 >= maxr || pairs + ncell[r] > maxp) {
-      rows.push_back(static_cast<int32_t>(r));
-      r0 = static_cast<int32_t>(r);
-      seg = 0;
-      pairs = 0;
+  if (with_kk) {
+    int64_t seg = 0, pairs = 0;
+    int32_t r0 = 0;
+    for (int64_t r = 0; r < A.nrows_b; ++r) {
+      const int64_t len = (int64_t)bs2 * (A.h_rpb[r + 1] - A.h_rpb[r]);
+      if (len > cap || ncell[r] > maxp) return nullptr;   // a single row does not fit
+      if (seg + len > cap || r - r0 >= maxr || pairs + ncell[r] > maxp) {
+        rows.push_back(static_cast<int32_t>(r));
+        r0 = static_cast<int32_t>(r);
+        seg = 0;
+        pairs = 0;
+      }
+      seg += len;
+      pairs += ncell[r];
     }
-    seg += len;
-    pairs += ncell[r];
+  } else {
+    // The hexahedral kernel forms the geometry of every cell of a chunk at all
+    // its quadrature points, so a chunk ends where it has the fewest cells per
+    // value among the row counts that fill at least 3/4 of it.
+    std::vector<int64_t> start(A.nrows_b + 1, 0);
+    for (int64_t r = 0; r < A.nrows_b; ++r) start[r + 1] = start[r] + ncell[r];
+    std::vector<int32_t> cells(std::max<int64_t>(1, start[A.nrows_b]));
+    {
+      std::vector<int64_t> at(start.begin(), start.end() - 1);
+      for (int64_t e = 0; e < I.n; ++e)
+        for (int l = 0; l < nd; ++l)
+          cells[at[d0->host[(int64_t)I.h_ents[e] * nd + l]]++] = I.h_ents[e];
+    }
+    std::vector<int32_t> seen(d0->num_cells, -1);
+    std::vector<std::pair<int64_t, int64_t>> ends;     // (values, cells) up to each row
+    for (int64_t r0 = 0; r0 < A.nrows_b;) {
+      int64_t seg = 0, pairs = 0, items = 0, r = r0;
+      ends.clear();
+      for (; r < A.nrows_b && r - r0 < maxr; ++r) {
+        const int64_t len = (int64_t)bs2 * (A.h_rpb[r + 1] - A.h_rpb[r]);
+        if (len > cap || ncell[r] > maxp) return nullptr;
+        if (seg + len > cap || pairs + ncell[r] > maxp) break;
+        seg += len;
+        pairs += ncell[r];
+        for (int64_t k = start[r]; k < start[r + 1]; ++k)
+          if (seen[cells[k]] != (int32_t)r0) {
+            seen[cells[k]] = (int32_t)r0;
+            ++items;
+          }
+        ends.emplace_back(seg, items);
+      }
+      size_t best = ends.size() - 1;
+      if (r < A.nrows_b)
+        for (size_t k = 0; k + 1 < ends.size(); ++k)
+          if (4 * ends[k].first >= 3 * seg &&
+              (double)ends[k].second * ends[best].first < (double)ends[best].second * ends[k].first)
+            best = k;
+      r0 += static_cast<int64_t>(best) + 1;
+      if (r0 < A.nrows_b) rows.push_back(static_cast<int32_t>(r0));
+    }
   }
   rows.push_back(static_cast<int32_t>(A.nrows_b));
   auto plan = build_items(rows, I, d0);
@@ -130,7 +174,7 @@ std::shared_ptr<OwnerPlan> build_owner_plan(const mf_form& a, const Integral& I,
     poff[c + 1] = poff[c] + n;
   }
   const int64_t np = poff[nch];
-  std::vector<int32_t> plist(std::max<int64_t>(1, np));
+  std::vector<int32_t> plist(np + 1, 0);
   // column offsets: one 16-byte aligned block of npairs * nd bytes per chunk
   std::vector<int64_t> kkoff(nch + 1, 0);
   for (int64_t c = 0; c < nch; ++c)
@@ -153,10 +197,10 @@ std::shared_ptr<OwnerPlan> build_owner_plan(const mf_form& a, const Integral& I,
           const int i = __builtin_ctzll(msk);
           msk &= msk - 1;
           // simplex kernel (column offsets precomputed): cell id << 6 | local row;
-          // hexahedral kernel: item offset in the chunk << 8 | local row
-          plist[p] = with_kk ? static_cast<int32_t>((static_cast<uint32_t>(cell) << 6) | i)
-                             : ((it - ci[c]) << 8) | i;
+          // hexahedral kernel: item in the chunk << 16 | row in the chunk << 6 | local row
           const int32_t R = d0->host[(int64_t)cell * nd + i];
+          plist[p] = with_kk ? static_cast<int32_t>((static_cast<uint32_t>(cell) << 6) | i)
+                             : ((it - ci[c]) << 16) | ((R - rows[c]) << 6) | i;
           const int32_t* rb = A.h_colsb.data() + A.h_rpb[R];
           const int32_t* re = A.h_colsb.data() + A.h_rpb[R + 1];
           if (!with_kk) {
@@ -205,6 +249,14 @@ std::shared_ptr<OwnerPlan> build_owner_plan(const mf_form& a, const Integral& I,
     mc[6] = static_cast<int32_t>(base); mc[7] = static_cast<int32_t>(bs2 * (cb1 - cb0));
     mc[8] = static_cast<int32_t>(poff[c]); mc[9] = static_cast<int32_t>(poff[c + 1]);
     mc[10] = static_cast<int32_t>(kkoff[c]);
+  }
+  if (!with_kk) {
+    const mf_mesh& M = *a.mesh;
+    std::vector<int32_t> geo(M.num_cells * M.nv), ig((plan->nitems + 1) * M.nv, 0);
+    MF_HIP(hipMemcpy(geo.data(), M.cells.ptr, sizeof(int32_t) * geo.size(), hipMemcpyDeviceToHost));
+    for (int64_t it = 0; it < plan->nitems; ++it)
+      std::copy_n(&geo[(int64_t)plan->h_cell[it] * M.nv], M.nv, &ig[it * M.nv]);
+    plan->item_geo.upload(ig);
   }
   plan->chunk_meta.upload(meta);
   plan->pair_list.upload(plist);
@@ -738,14 +790,22 @@ void assemble_matrix(mf_form* a, mf_matrix* A, const mf_bc* bc0, const mf_bc* bc
       const int64_t prec = a->opt("precision", 64);
       const int v = prec == 64 ? 0 : (prec == 32 ? 1 : 2);
       MF_CHECK(prec == 64 || prec == 32 || prec == 16, MF_EINVAL, "precision must be 64, 32 or 16");
-      launch(owner->k_hprep, static_cast<uint32_t>((owner->n + 255) / 256), 256, 0, s,
-             static_cast<int32_t>(owner->n), owner->d_ents.ptr, a->mesh->cells.ptr,
-             a->mesh->x.ptr, a->dm[0]->dev.ptr, n0, owner->records.ptr);
-      launch(owner->k_howner[v], static_cast<uint32_t>(per * nx),
-             static_cast<uint32_t>(hex_block(*a, static_cast<int>(prec))), 0, s,
+      uint64_t* cmask = n0 ? reinterpret_cast<uint64_t*>(owner->records.ptr) : nullptr;
+      if (cmask)
+        launch(owner->k_hprep, static_cast<uint32_t>((owner->n + 3) / 4), 256, 0, s,
+               static_cast<int32_t>(owner->n), owner->d_ents.ptr, a->dm[0]->dev.ptr, n0, cmask);
+      const uint32_t hblock = static_cast<uint32_t>(hex_block(*a, static_cast<int>(prec)));
+      int64_t& hgrid = owner->howner_grid[v];
+      if (hgrid == 0) {
+        int nblk = 0;
+        MF_HIP(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&nblk, owner->k_howner[v], hblock, 0));
+        hgrid = std::max<int64_t>(nx, (int64_t)std::max(1, nblk) * a->ctx->num_cus / nx * nx);
+      }
+      const int64_t grid = a->opt("owner_persistent", 1) ? std::min(per * nx, hgrid) : per * nx;
+      launch(owner->k_howner[v], static_cast<uint32_t>(grid), hblock, 0, s,
              static_cast<int32_t>(plan->nchunks), plan->chunk_meta.ptr, plan->item_cell.ptr,
-             plan->pair_list.ptr, plan->pair_pos.ptr, owner->records.ptr, A->rpb.ptr,
-             plan->diag_pos.ptr, n0, A->values, diagonal, flags);
+             plan->item_geo.ptr, plan->pair_list.ptr, plan->pair_pos.ptr, a->mesh->x.ptr, cmask,
+             A->rpb.ptr, plan->diag_pos.ptr, n0, A->values, diagonal, flags);
     } else {
     const uint8_t* cf = n0 ? bc0->cell_flags_for(a->dm[0], s) : nullptr;
     launch(owner->k_prep, static_cast<uint32_t>((owner->n + 255) / 256), 256, 0, s,

@@ -260,6 +260,7 @@ struct Integral {
   int vown_regs = 0;                  // registers of k_vown (0: not queried)
   hipFunction_t k_vown = nullptr, k_slift = nullptr, k_hlift = nullptr, k_prep = nullptr;
   hipFunction_t k_hprep = nullptr, k_howner[3] = {nullptr, nullptr, nullptr};  // FP64, FP32, BF16
+  int64_t howner_grid[3] = {0, 0, 0};  // resident workgroups of k_howner (0: not queried)
   hipFunction_t k_scl = nullptr;      // rank 0: per-block partial sums
   int64_t scl_off = 0;                // rank 0: first partial of this integral
   uint32_t scl_grid = 1;              // rank 0: workgroups (one partial each)

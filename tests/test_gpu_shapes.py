@@ -227,3 +227,38 @@ def test_product_rows_of_any_length(which, n):
     S = sp.csr_matrix((vals, cols, rp), shape=(A.nrows, A.ncols))
     # at most 400 products per row, each rounded once: 400 eps of the absolute sums
     assert np.all(np.abs(y.cpu().numpy() - S @ x) <= 400 * 2.2e-16 * (abs(S) @ np.abs(x)) + 1e-300)
+
+
+@pytest.mark.parametrize("prec,tol", [(64, TOL), (32, 1e-6)])
+@pytest.mark.parametrize("n,share,subset", [(1, 0.1, False), (2, 0.0, False), (3, 0.3, True), (5, 0.05, True),
+                                            (7, 0.1, False)])
+def test_hexahedral_owner_chunks(n, share, subset, prec, tol):
+    """Q3 matrices from one cell to more chunks than resident workgroups per XCD,
+    with Dirichlet rows, over all cells or a subdomain (rows and chunks without
+    cells), overwriting and adding."""
+    import dataclasses
+    import cudolfinx as cufem
+    print(f"[gpu-test] Q3 owner chunks n={n} share={share} subset={subset} precision={prec}", flush=True)
+    P = problems.helmholtz_q3(n, seed=8)
+    a = P.a
+    if subset:
+        I = a.integrals[0]
+        keep = np.sort(np.random.default_rng(n).choice(n ** 3, size=n ** 3 // 3, replace=False)).astype(np.int32)
+        a = dataclasses.replace(a, integrals=[dataclasses.replace(I, entities=keep)])
+    bc = _some_dofs(P.V, share, 3)
+    asm = cufem.CUDAAssembler()
+    f = cufem.form(a, options={"matrix_kernel": 2, "precision": prec})
+    A = asm.assemble_matrix(f, bcs=[bc], diagonal=1.5)
+    asm.synchronize()
+    rp, cols, v = A.csr()
+    o = cpu.OracleAssembler(a)
+    orp, ocols, _, _ = o.sparsity()
+    ref = o.assemble_matrix(orp, ocols, [bc], diagonal=1.5)
+    assert np.array_equal(rp, orp) and np.array_equal(cols, ocols)
+    # FP32 element arithmetic keeps its 1e-6; the diagonal entries are exact
+    scale = np.linalg.norm(o.assemble_matrix(orp, ocols, []))
+    assert np.linalg.norm(v - ref) <= tol * max(scale, np.linalg.norm(ref))
+    asm.assemble_matrix(f, A, bcs=[bc], diagonal=1.5, zero=False)
+    asm.synchronize()
+    ref = o.assemble_matrix(orp, ocols, [bc], diagonal=1.5, values=ref.copy())
+    assert np.linalg.norm(A.csr()[2] - ref) <= 2 * tol * max(scale, np.linalg.norm(ref))
