@@ -415,7 +415,10 @@ void compile_form(mf_form* f, int verbose) {
         I->k_scl = f->mod->get(mf::kernel_name("scl", I->type, I->index));
       } else {
         I->k_vec = f->mod->get(mf::kernel_name("vec", I->type, I->index));
-        if (I->type == MF_CELL) I->k_vblk = f->mod->get(mf::kernel_name("vblk", I->type, I->index));
+        if (mf::hex_source_emitted(*f, *I))
+          I->k_hsrc = f->mod->get(mf::kernel_name("hsrc", I->type, I->index));
+        else if (I->type == MF_CELL)
+          I->k_vblk = f->mod->get(mf::kernel_name("vblk", I->type, I->index));
         if (I->type == MF_CELL && f->dm[0]->nd <= 32)
           I->k_vown = f->mod->get(mf::kernel_name("vown", I->type, I->index));
       }

@@ -387,6 +387,18 @@ bool hex_lift_emitted(const mf_form& f, const Integral& I) {
          f.dm[0]->nd == k1 * k1 * k1 && staged_define(I.staged_src, "HX_ND") == f.dm[0]->nd;
 }
 
+// The source kernel takes any degree whose stages and rows fit its LDS, and
+// one integral of a form (the tables are not renamed).
+bool hex_source_emitted(const mf_form& f, const Integral& I) {
+  if (I.type != MF_CELL || f.rank != 1 || f.mesh->nv != 8 ||
+      I.staged_src.find("#define HS_C ") == std::string::npos)
+    return false;
+  for (auto& J : f.ints)
+    if (J->index < I.index && J->type == MF_CELL && !J->staged_src.empty()) return false;
+  const int k1 = staged_define(I.staged_src, "HX_K") + 1, m1 = staged_define(I.staged_src, "HX_NQ1");
+  return k1 >= 1 && k1 <= 6 && m1 >= 1 && m1 <= 6 && f.dm[0]->bs == 1 && f.dm[0]->nd == k1 * k1 * k1;
+}
+
 // Threads per workgroup of the hex matrix-core kernel: 512 for the FP32 / BF16
 // operand paths (more waves to overlap the MFMA chains with the operand
 // loads), 256 for FP64; option hex_block overrides both.
@@ -496,6 +508,7 @@ extern const char* kPrepTemplate;
 extern const char* kHexPrepTemplate;
 extern const char* kHexOwnerTemplate;
 extern const char* kHexLiftTemplate;
+extern const char* kHexSourceTemplate;
 extern const char* kDGOwnerMatrix;        // dg_kernel.cpp
 extern const char* kDGOwnerVector;
 extern const char* kDGCaseCellMat;
@@ -1145,7 +1158,12 @@ std::string generate_form_source(const mf_form& f) {
     } else if (f.rank == 1) {
       m["$KNAME"] = kernel_name("vec", I->type, I->index);
       os << subst(subst(kVector, {{"$GATHER", gather}}), m);
-      if (I->type == MF_CELL) {
+      if (hex_source_emitted(f, *I)) {
+        os << "\n" << I->staged_src << "\n";
+        m["$KNAME"] = kernel_name("hsrc", I->type, I->index);
+        m["$HSC"] = std::to_string(kHexSourceCells);
+        os << subst(kHexSourceTemplate, m);
+      } else if (I->type == MF_CELL) {
         m["$KNAME"] = kernel_name("vblk", I->type, I->index);
         os << subst(subst(kVectorBlocks, {{"$GATHER", gather}}), m);
       }

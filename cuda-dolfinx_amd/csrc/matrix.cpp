@@ -307,9 +307,10 @@ std::shared_ptr<OwnerPlan> vector_plan(mf_form* L, Integral& I) {
 //   P2 residual with 64 points (242): 1 thousand 37 / 43, 10 thousand 61 / 41,
 //     48 thousand 97 / 48; P1 with 27 points: 3 thousand 17 / 9.
 // Cells of more than 32 nodes have no row-owning kernel: Q3 source on 14
-// thousand hexahedra 50 us, 78 us with one atomic per row.
+// thousand hexahedra 50 us, 78 us with one atomic per row, 14 us with a wave per
+// cell (mf_hsrc_*).
 static bool blocks_pay(const mf_form& L, Integral& I) {
-  if (!I.k_vown) return true;
+  if (I.k_hsrc || !I.k_vown) return true;
   if (L.options.count("vector_chunk_values") || L.options.count("vector_block")) return false;
   if (I.vown_regs == 0) {
     int regs = 0;
@@ -321,21 +322,24 @@ static bool blocks_pay(const mf_form& L, Integral& I) {
 
 // Blocks of at most 256 entities (down to 64 where that leaves fewer than
 // three blocks per CU) whose rows fit 64 KB of LDS; null when rows are shared so
-// little that the blocks hold fewer than half their entities.
+// little that the blocks hold fewer than half their entities.  With a wave per
+// cell 32 cells (down to 4) and 32 KB, in blocks of 256 threads.
 static VectorBlocks* vector_blocks(mf_form* L, const Integral& I) {
   auto it = L->vblocks.find(I.index);
   if (it != L->vblocks.end()) return it->second.get();
   const mf_dofmap* d0 = L->dm[0];
   const int nd = d0->nd, bs = d0->bs;
   auto B = std::make_unique<VectorBlocks>();
-  while (B->threads > 64 && I.n < 3LL * L->ctx->num_cus * B->threads) B->threads /= 2;
-  const size_t cap = 8192 / bs;                          // nodes per block
+  int most = I.k_hsrc ? kHexSourceCells : 256;
+  while (most > (I.k_hsrc ? 4 : 64) && I.n < 3LL * L->ctx->num_cus * most) most /= 2;
+  B->threads = I.k_hsrc ? 256 : most;
+  const size_t cap = (I.k_hsrc ? 4096 : 8192) / bs;      // nodes per block
   std::vector<int32_t> ent{0}, ptr{0}, row, place(d0->num_nodes, -1), nodes;
   std::vector<uint16_t> slot(static_cast<size_t>(I.n) * nd);
   for (int64_t e = 0; e < I.n;) {
     const int64_t e0 = e;
     nodes.clear();
-    for (; e < I.n && e - e0 < (int64_t)B->threads; ++e) {
+    for (; e < I.n && e - e0 < most; ++e) {
       const size_t before = nodes.size();
       const int32_t* dm = &d0->host[(int64_t)I.h_ents[e] * nd];
       for (int i = 0; i < nd; ++i)
@@ -362,7 +366,7 @@ static VectorBlocks* vector_blocks(mf_form* L, const Integral& I) {
     B->lds = std::max(B->lds, static_cast<uint32_t>(8 * bs * nodes.size()));
   }
   B->n = static_cast<int64_t>(ent.size()) - 1;
-  if (B->n * B->threads > 2 * std::max<int64_t>(I.n, B->threads)) return (L->vblocks[I.index] = nullptr).get();
+  if (!I.k_hsrc && B->n * most > 2 * std::max<int64_t>(I.n, most)) return (L->vblocks[I.index] = nullptr).get();
   B->ent.upload(ent);
   B->ptr.upload(ptr);
   B->row.upload(row);
@@ -938,7 +942,7 @@ void assemble_vector(mf_form* L, double* b, int64_t n, int zero, hipStream_t s) 
   VectorBlocks* blocks = nullptr;
   if (mode == 0 || mode == 4)
     for (auto& I : L->ints)
-      if (I->type == MF_CELL && I->n && I->k_vblk) {
+      if (I->type == MF_CELL && I->n && (I->k_vblk || I->k_hsrc)) {
         if (mode == 4 || blocks_pay(*L, *I)) blocks = vector_blocks(L, *I);
         if (blocks) owner = I.get();
         break;
@@ -954,7 +958,7 @@ void assemble_vector(mf_form* L, double* b, int64_t n, int zero, hipStream_t s) 
   MF_CHECK(!(mode == 2 && !owner), MF_EUNSUPPORTED, "owner-computes vector kernel unavailable");
   if (blocks) {
     if (zero) k_fill(b, n, 0.0, s);
-    launch(owner->k_vblk, static_cast<uint32_t>((blocks->n + 7) / 8 * 8), blocks->threads, blocks->lds,
+    launch(owner->k_hsrc ? owner->k_hsrc : owner->k_vblk, static_cast<uint32_t>((blocks->n + 7) / 8 * 8), blocks->threads, blocks->lds,
            s, static_cast<int32_t>(blocks->n), blocks->ent.ptr, blocks->ptr.ptr, blocks->row.ptr,
            blocks->slot.ptr, owner->d_ents.ptr, L->mesh->cells.ptr, L->mesh->x.ptr, L->packed.ptr,
            L->consts.ptr, b);

@@ -256,7 +256,8 @@ struct Integral {
   int index = 0;                      // position in the form
   hipFunction_t k_ten = nullptr;      // element tensors into a workspace
   hipFunction_t k_mat = nullptr, k_vec = nullptr, k_lift = nullptr, k_owner = nullptr;
-  hipFunction_t k_vblk = nullptr;     // rank 1: blocks of consecutive cells
+  hipFunction_t k_vblk = nullptr;     // rank 1: blocks of consecutive cells, a thread per cell
+  hipFunction_t k_hsrc = nullptr;     // the same with a wave per cell (hexahedral source)
   int vown_regs = 0;                  // registers of k_vown (0: not queried)
   hipFunction_t k_vown = nullptr, k_slift = nullptr, k_hlift = nullptr, k_prep = nullptr;
   hipFunction_t k_hprep = nullptr, k_howner[3] = {nullptr, nullptr, nullptr};  // FP64, FP32, BF16
@@ -434,6 +435,8 @@ bool staged_trace(const Integral& I);
 bool staged_lift_emitted(const Integral& I);
 bool hex_owner_supported(const mf_form& f, const Integral& I);
 bool hex_lift_emitted(const mf_form& f, const Integral& I);
+bool hex_source_emitted(const mf_form& f, const Integral& I);
+constexpr int kHexSourceCells = 32;   // most cells in a block of the hexahedral source kernel
 int hex_batch(const mf_form& f, const Integral& I, int prec);
 int hex_block(const mf_form& f, int prec);
 struct OwnerShape { int nb = 0, maxp = 0; };

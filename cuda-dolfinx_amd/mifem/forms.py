@@ -487,7 +487,8 @@ def linear_sum(a: Form, b: Form) -> Form:
                 spec[key] = ("w", val[1] + coffs_a)
             elif isinstance(val, tuple) and val[0] == "c":
                 spec[key] = ("c", val[1] + consts_a)
-        new_b.append(Integral(I.type, I.id, I.entities, I.name, src, I.staged, spec))
+        staged = I.staged.shifted(consts_a) if hasattr(I.staged, "shifted") else I.staged
+        new_b.append(Integral(I.type, I.id, I.entities, I.name, src, staged, spec))
     order = {CELL: 0, EXTERIOR_FACET: 1, INTERIOR_FACET: 2}
     ints = sorted(a.integrals + new_b, key=lambda I: order[I.type])
     return Form(a.rank, a.function_spaces, ints, a.coefficients + b.coefficients,

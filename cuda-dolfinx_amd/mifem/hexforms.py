@@ -76,6 +76,24 @@ class HexContraction:
     kappa: float
 
 
+def _tensor_tables(k: int, m: int) -> str:
+    """1D GLL Lagrange values and derivatives of degree k at m Gauss points."""
+    x, w = E._gauss_legendre01(m)
+    el1 = E.gll_points(k)
+    C1 = np.linalg.inv(np.vander(el1, k + 1, increasing=True))
+    V = np.vander(x, k + 1, increasing=True) @ C1               # (m, k+1)
+    D = np.zeros((m, k + 1))
+    for j in range(1, k + 1):
+        D += j * np.outer(x ** (j - 1), C1[j])
+    return (f"#define HX_K {k}\n#define HX_NQ1 {m}\n#define HX_ND {(k + 1) ** 3}\n"
+            + _carr("HX_L", V, "__constant__ double")
+            + _carr("HX_DL", D, "__constant__ double")
+            + _carr("HX_LF", V, "__constant__ float")
+            + _carr("HX_DLF", D, "__constant__ float")
+            + _carr("HX_X1", x, "__constant__ double")
+            + _carr("HX_W1", w, "__constant__ double"))
+
+
 @dataclass
 class HexStaged:
     """Staged description of kappa grad.grad - k^2 mass on Q_k hexahedra.
@@ -91,22 +109,23 @@ class HexStaged:
     kappa: float
 
     def source(self) -> str:
-        k, m = self.degree, self.m
-        x, w = E._gauss_legendre01(m)
-        el1 = E.gll_points(k)
-        C1 = np.linalg.inv(np.vander(el1, k + 1, increasing=True))
-        V = np.vander(x, k + 1, increasing=True) @ C1               # (m, k+1)
-        D = np.zeros((m, k + 1))
-        for j in range(1, k + 1):
-            D += j * np.outer(x ** (j - 1), C1[j])
-        return (f"#define HX_K {k}\n#define HX_NQ1 {m}\n#define HX_ND {(k + 1) ** 3}\n"
-                f"#define HX_K2 {self.k2!r}\n#define HX_KAPPA {self.kappa!r}\n"
-                + _carr("HX_L", V, "__constant__ double")
-                + _carr("HX_DL", D, "__constant__ double")
-                + _carr("HX_LF", V, "__constant__ float")
-                + _carr("HX_DLF", D, "__constant__ float")
-                + _carr("HX_X1", x, "__constant__ double")
-                + _carr("HX_W1", w, "__constant__ double"))
+        return (f"#define HX_K2 {self.k2!r}\n#define HX_KAPPA {self.kappa!r}\n"
+                + _tensor_tables(self.degree, self.m))
+
+
+@dataclass
+class HexSource:
+    """Staged description of the source c[constant] v on scalar Q_k hexahedra:
+    the 1D tables of HexStaged and the place of the constant."""
+    degree: int
+    m: int
+    constant: int = 0
+
+    def shifted(self, constants: int) -> "HexSource":
+        return HexSource(self.degree, self.m, self.constant + constants)
+
+    def source(self) -> str:
+        return f"#define HS_C {self.constant}\n" + _tensor_tables(self.degree, self.m)
 
 
 def helmholtz(V: FunctionSpace, k: float, kappa=None, qpoints_per_dir: Optional[int] = None) -> Form:
@@ -189,4 +208,5 @@ def hex_source(V: FunctionSpace, f: Constant, qpoints_per_dir: Optional[int] = N
     cells = np.arange(V.mesh.num_cells, dtype=np.int32)
     spec = dict(kind="source", cell=1, degree=el.degree, bs=1, rank=1, qm=m, f=("c", 0),
                 f_degree=0)
-    return Form(1, [V], [Integral(CELL, -1, cells, name, src, None, spec)], [], [f], "hex_source")
+    return Form(1, [V], [Integral(CELL, -1, cells, name, src, HexSource(el.degree, m), spec)], [], [f],
+                "hex_source")

@@ -262,3 +262,40 @@ def test_hexahedral_owner_chunks(n, share, subset, prec, tol):
     asm.synchronize()
     ref = o.assemble_matrix(orp, ocols, [bc], diagonal=1.5, values=ref.copy())
     assert np.linalg.norm(A.csr()[2] - ref) <= 2 * tol * max(scale, np.linalg.norm(ref))
+
+
+@pytest.mark.parametrize("k,m,n,subset", [(1, 2, 1, False), (1, 3, 9, True), (2, 2, 3, False), (3, 4, 1, False),
+                                          (3, 4, 5, True), (3, 4, 13, False), (4, 6, 3, False), (5, 5, 2, True),
+                                          (6, 7, 1, False)])
+def test_hexahedral_source(k, m, n, subset):
+    """Q_k sources on hexahedra against the per-entity kernel, and the oracle where it
+    takes the degree: more and fewer points than nodes per direction, a partial last
+    block, a subdomain, a degree past the kernel's, a sum of two sources, and its
+    second one alone, whose constant is not the form's first."""
+    import dataclasses
+    import cudolfinx as cufem
+    from mifem import forms
+    from mifem.fem import Constant, functionspace
+    from mifem.mesh import create_unit_cube
+    print(f"[gpu-test] Q{k} source m={m} n={n} subset={subset}", flush=True)
+    V = functionspace(create_unit_cube(n, "hexahedron", jitter=0.2, seed=3), ("P", k))
+    L = forms.hex_source(V, Constant(1.7), qpoints_per_dir=m)
+    M = forms.hex_source(V, Constant(-0.3), qpoints_per_dir=m - 1)
+    if subset:
+        keep = np.sort(np.random.default_rng(n).choice(n ** 3, size=n ** 3 // 2, replace=False)).astype(np.int32)
+        L = dataclasses.replace(L, integrals=[dataclasses.replace(L.integrals[0], entities=keep)])
+    S = forms.linear_sum(M, L)
+    asm = cufem.CUDAAssembler()
+    for F in (L, S, dataclasses.replace(S, integrals=S.integrals[1:])):
+        f = cufem.form(F)
+        b = asm.assemble_vector(f)
+        asm.synchronize()
+        per_entity = asm.assemble_vector(cufem.form(F, options={"vector_kernel": 1}))
+        asm.synchronize()
+        ref = per_entity.to_host()
+        assert _rel(b.to_host(), ref) <= TOL
+        if k <= 3 and m <= 4:
+            assert _rel(b.to_host(), cpu.OracleAssembler(F).assemble_vector()) <= TOL
+        asm.assemble_vector(f, b, zero=False)
+        asm.synchronize()
+        assert _rel(b.to_host(), 2 * ref) <= TOL
