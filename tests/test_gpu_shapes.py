@@ -299,3 +299,29 @@ def test_hexahedral_source(k, m, n, subset):
         asm.assemble_vector(f, b, zero=False)
         asm.synchronize()
         assert _rel(b.to_host(), 2 * ref) <= TOL
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5])
+def test_fused_system_adds_with_dirichlet_rows(n):
+    """J, F and E of DG1 in blocks of 64 cells (partial, exact and several, segments
+    that start at odd values' alignment): overwriting, then adding, with Dirichlet rows."""
+    import torch
+    import cudolfinx as cufem
+    from mifem.dgforms import sipg_energy
+    print(f"[gpu-test] DG1 system n={n}", flush=True)
+    P = problems.dg_plaplace(n)
+    P.extras["u"].x[:] = np.random.default_rng(n).uniform(-1, 1, P.V.size)
+    bc = _some_dofs(P.V, 0.2, 5)
+    J, F, E_ = cufem.form(P.a), cufem.form(P.L), cufem.form(sipg_energy(P.V, P.extras["u"]))
+    asm = cufem.CUDAAssembler()
+    A, b = asm.create_matrix(J), asm.create_vector(F)
+    system, ev = cufem.CUDASystem(J, F, E_), torch.zeros(1, dtype=torch.float64, device="cuda")
+    o = cpu.OracleAssembler(P.a)
+    rp, cols, _, _ = o.sparsity()
+    ref, rhs = o.assemble_matrix(rp, cols, [bc], diagonal=2.5), cpu.OracleAssembler(P.L).assemble_vector()
+    for times in (1, 2):
+        system.assemble(asm, A, b, ev, bcs=asm.pack_bcs([bc]), diagonal=2.5, zero=times == 1)
+        asm.synchronize()
+        assert _rel(A.csr()[2], ref) <= TOL
+        assert _rel(b.to_host(), times * rhs) <= TOL
+        ref = o.assemble_matrix(rp, cols, [bc], diagonal=2.5, values=ref.copy())
