@@ -767,9 +767,14 @@ static bool owner_f32(const mf_form& f, const Integral& I) {
   return staged_trace(I) && f.opt("precision", 64) == 32;
 }
 
+// MF_RST of the owner kernel: numbers of size sz between rows of the reference tensors
+static int64_t ref_stride(int64_t nd, int64_t sz) {
+  return nd * 6 + (8 - nd * 6 * (sz / 4) % 8 + 4) % 8 / (sz / 4);
+}
+
 static std::vector<LdsSlice> owner_lds_slices(const mf_form& f, const Integral& I) {
   auto r16 = [](int64_t b) { return (b + 15) / 16 * 16; };
-  const int64_t nd = staged_define(I.staged_src, "SK_ND"), bs = staged_define(I.staged_src, "SK_BS");
+  const int64_t nd = staged_define(I.staged_src, "SK_ND");
   const int64_t cap = f.opt("chunk_values", 4096), maxr = f.opt("chunk_rows", 64);
   const int64_t maxp = owner_shape(f, I).maxp;
   const bool f32 = owner_f32(f, I), f32acc = f32 && f.opt("owner_f32acc", 0);
@@ -777,11 +782,10 @@ static std::vector<LdsSlice> owner_lds_slices(const mf_form& f, const Integral& 
   const int64_t as = f32 ? 4 : 8;
   std::vector<LdsSlice> v = {{"acc", f32acc ? "float" : "double", r16((f32acc ? 4 : 8) * cap)},
                              {"lrp", "int32_t", r16(4 * (maxr + 1))},
-                             {"snb", "uint8_t", r16(maxr)},
-                             {"lcols", "int32_t", r16(4 * (cap / (bs * bs) + 1))},
+                             {"snb", "int32_t", r16(4 * maxr)},
                              {"spair", "int32_t", r16(4 * maxp)},
                              {"skk", "uint8_t", r16((maxp * nd + 15) / 16 * 16)}};
-  if (staged_trace(I)) v.push_back({"sRS", at, r16(as * nd * nd * 6)});
+  if (staged_trace(I)) v.push_back({"sRS", at, r16(as * nd * ref_stride(nd, as))});
   else if (staged_fullrt(I)) v.push_back({"sRT", "double", r16(8 * nd * nd * 9)});
   else v.push_back({"sDPHI", "double", r16(8 * staged_define(I.staged_src, "SK_NQ") * nd * 3)});
   return v;
@@ -915,10 +919,10 @@ std::string generate_batch_source(const std::vector<const mf_form*>& forms,
                 a + "pair_list, const uint8_t* __restrict__ " + a + "pair_kk, const mf_rec_" + tag +
                 "* __restrict__ " + a + "rec, const double* __restrict__ " + a +
                 "consts, const int32_t* __restrict__ " + a + "rpb, const int32_t* __restrict__ " + a +
-                "colsb, const uint8_t* __restrict__ " + a + "nb0, double* __restrict__ " + a + "values";
+                "dpos, const uint8_t* __restrict__ " + a + "nb0, double* __restrict__ " + a + "values";
       calls += "  mf_owner_body_g" + std::to_string(g) + "(" + a + "nchunks, " + a + "chunk_meta, " +
                a + "item_cell, " + a + "pair_list, " + a + "pair_kk, " + a + "rec, " + a + "consts, " +
-               a + "rpb, " + a + "colsb, " + a + "nb0, " + a + "values, diag, flags" + sargs +
+               a + "rpb, " + a + "dpos, " + a + "nb0, " + a + "values, diag, flags" + sargs +
                ");\n  __syncthreads();\n";
     }
   }

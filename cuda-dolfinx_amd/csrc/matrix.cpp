@@ -264,7 +264,7 @@ std::shared_ptr<OwnerPlan> build_owner_plan(const mf_form& a, const Integral& I,
   plan->pair_pos.upload(ppos);
   {
     // position of the diagonal block in each blocked row (-1: none): the
-    // Dirichlet diagonal of the hexahedral and warp-specialised kernels
+    // Dirichlet diagonal of the owner kernels
     std::vector<int32_t> dp(std::max<int64_t>(1, A.nrows_b), -1);
     for (int64_t R = 0; R < A.nrows_b; ++R) {
       const int32_t* rb = A.h_colsb.data() + A.h_rpb[R];
@@ -854,7 +854,7 @@ void assemble_matrix(mf_form* a, mf_matrix* A, const mf_bc* bc0, const mf_bc* bc
     launch(kown, static_cast<uint32_t>(grid), oblock, 0, s,
            static_cast<int32_t>(plan->nchunks), plan->chunk_meta.ptr, plan->item_cell.ptr,
            plan->pair_list.ptr, plan->pair_kk.ptr, owner->records.ptr, a->consts.ptr, A->rpb.ptr,
-           A->colsb.ptr, n0, A->values, diagonal, flags);
+           plan->diag_pos.ptr, n0, A->values, diagonal, flags);
     }
     }
   }
@@ -1047,7 +1047,7 @@ void assemble_batch(mf_batch* B, mf_matrix* const* As, const mf_bc* const* bcs, 
                     int zero, hipStream_t s) {
   struct Args {   // one group's kernel arguments (see the pointer list below)
     const void* chunk_meta; const void* item_cell; const void* pair_list; const void* pair_kk;
-    const void* rec; const void* consts; const void* rpb; const void* colsb; const void* nb0;
+    const void* rec; const void* consts; const void* rpb; const void* dpos; const void* nb0;
     void* values; int32_t nchunks; int32_t pad;
   };
   static_assert(sizeof(Args) == 88, "batch argument layout");
@@ -1080,7 +1080,7 @@ void assemble_batch(mf_batch* B, mf_matrix* const* As, const mf_bc* const* bcs, 
            static_cast<int32_t>(I->n), I->d_ents.ptr, a->mesh->cells.ptr, a->mesh->x.ptr,
            a->packed.ptr, a->dm[0]->dev.ptr, n0, cf, I->records.ptr);
     h[g] = Args{plan->chunk_meta.ptr, plan->item_cell.ptr, plan->pair_list.ptr, plan->pair_kk.ptr,
-                I->records.ptr, a->consts.ptr, A->rpb.ptr, A->colsb.ptr, n0, A->values,
+                I->records.ptr, a->consts.ptr, A->rpb.ptr, plan->diag_pos.ptr, n0, A->values,
                 static_cast<int32_t>(plan->nchunks), 0};
   }
   // kernel arguments, per group in the order of kOwnerParams (nchunks,
@@ -1095,7 +1095,7 @@ void assemble_batch(mf_batch* B, mf_matrix* const* As, const mf_bc* const* bcs, 
                     static_cast<void*>(&x.item_cell), static_cast<void*>(&x.pair_list),
                     static_cast<void*>(&x.pair_kk), static_cast<void*>(&x.rec),
                     static_cast<void*>(&x.consts), static_cast<void*>(&x.rpb),
-                    static_cast<void*>(&x.colsb), static_cast<void*>(&x.nb0),
+                    static_cast<void*>(&x.dpos), static_cast<void*>(&x.nb0),
                     static_cast<void*>(&x.values)})
       ptrs.push_back(p);
   }

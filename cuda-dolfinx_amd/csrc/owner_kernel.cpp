@@ -14,8 +14,10 @@
 // Element math comes from the form's staged description: reference
 // gradients SK_DPHI[q][i][d], weights SK_W[q] and sk_combine(G, w, c, out)
 // mapping G_ij = sum_q w_q |det J| g_i(q) (x) g_j(q) to the bs x bs block of
-// entry (i, j).  Column positions are found by binary search in the chunk's
-// blocked column list staged in LDS.
+// entry (i, j).  Column positions come with the schedule, one byte per column of
+// a (cell, row) pair, and the position of a row's diagonal block, read under a
+// Dirichlet condition only; the column list itself is not read (4 bytes per
+// block, and 8 KB of LDS in the scalar kernels, which went with it).
 //
 // Vector kernel.  Same ownership over a row range of b: one thread per
 // (cell, chunk) item evaluates the UFCx tabulate_tensor body, adds the rows
@@ -43,6 +45,12 @@ typedef float mf_f2 __attribute__((ext_vector_type(2)));
 // each entry with FP32 arithmetic; 1 also accumulates in an FP32 LDS array, 2
 // in the FP64 one.  Geometry stays FP64 and the CSR values are written as FP64
 #define MF_OWNER_F32 0
+// Row i of the reference tensors, nd * 6 numbers, at a stride of 4 words more or
+// less than a multiple of 8: rows are then 16 places of four banks apart (a
+// wave's lanes read different rows; P3's 120 doubles alone would give 4 places).
+// With the column list gone too: P3 24^3 93 -> 73 us, a batch of 48 P1-P3
+// instances in FP32 159 -> 110 us, vector P2 48^3 818 -> 778 us.
+#define MF_RST(nd, sz) ((nd) * 6 + (8 - (nd) * 6 * ((sz) / 4) % 8 + 4) % 8 / ((sz) / 4))
 static __device__ __forceinline__ int mf_lds_lower_bound(const int32_t* a, int lo, int hi, int32_t key)
 {
   while (lo < hi) {
@@ -71,7 +79,7 @@ const char* kOwnerParams =
     "const int32_t* __restrict__ item_cell, const int32_t* __restrict__ pair_list, "
     "const uint8_t* __restrict__ pair_kk, const mf_rec_$TAG* __restrict__ rec, "
     "const double* __restrict__ consts, const int32_t* __restrict__ rpb, "
-    "const int32_t* __restrict__ colsb, const uint8_t* __restrict__ nb0, "
+    "const int32_t* __restrict__ dpos, const uint8_t* __restrict__ nb0, "
     "double* __restrict__ values, const double diag, const int flags";
 
 // Several forms (one element group each) in ONE persistent launch: every
@@ -216,10 +224,9 @@ $OHEAD($OPARAMS)
   // ceil(nchunks / 8) every workgroup owns exactly one chunk.
   constexpr int ND = SK_ND, BS = SK_BS, NQ = SK_NQ;
   constexpr int CAP = $OCAP, MAXR = $OMAXR, MAXP = $OMAXP, NT = $OBLOCK;
-  constexpr int CAPB = CAP / (BS * BS) + 1;
   constexpr int KK4 = (MAXP * ND + 15) / 16;         // column-offset words (16 bytes)
   constexpr int PF_P = (MAXP + NT - 1) / NT, PF_K = (KK4 + NT - 1) / NT;
-  constexpr int PF_R = (MAXR + 1 + NT - 1) / NT, PF_C = (CAPB + NT - 1) / NT;
+  constexpr int PF_R = (MAXR + 1 + NT - 1) / NT;
   constexpr int PF_B = (MAXR + NT - 1) / NT;
 #if MF_OWNER_F32 == 1
   typedef float mf_acc_t;
@@ -234,22 +241,24 @@ $OHEAD($OPARAMS)
   static_assert(CAP * sizeof(mf_acc_t) % 16 == 0, "chunk_values: the accumulator is zeroed in 16-byte words");
   MF_SHARED(mf_acc_t, acc, CAP);
   MF_SHARED(int32_t, lrp, MAXR + 1);
-  MF_SHARED(uint8_t, snb, MAXR);                     // Dirichlet bits of the chunk's rows
-  MF_SHARED(int32_t, lcols, CAPB);
+  // the chunk's rows: Dirichlet bits | position of the diagonal block + 1 << 8
+  // (0: none), read only under a Dirichlet condition
+  MF_SHARED(int32_t, snb, MAXR);
   MF_SHARED(int32_t, spair, MAXP);
   MF_SHARED(uint8_t, skk, KK4 * 16);
 #ifdef SK_TRACE
   // reference tensors R_ij (symmetrised, 6 per entry), loaded once per workgroup
-  MF_SHARED(mf_rt_t, sRS, ND * ND * 6);
+  constexpr int RST = MF_RST(ND, sizeof(mf_rt_t));
+  MF_SHARED(mf_rt_t, sRS, ND * RST);
 #if (SK_ND % 4 == 0) && MF_OWNER_F32
-  // FP32, ND a multiple of 4: row i's tensors transposed, sRS[(i * 6 + k) * ND + j],
+  // FP32, ND a multiple of 4: row i's tensors transposed, sRS[i * RST + k * ND + j],
   // so one 16-byte LDS read gives component k of four consecutive columns
   for (int p = threadIdx.x; p < ND * ND * 6; p += NT) {
     const int i = p / (6 * ND), k = (p / ND) % 6, j = p % ND;
-    sRS[p] = (mf_rt_t)SK_RS[i][j][k];
+    sRS[i * RST + k * ND + j] = (mf_rt_t)SK_RS[i][j][k];
   }
 #else
-  for (int p = threadIdx.x; p < ND * ND * 6; p += NT) sRS[p] = (mf_rt_t)(&SK_RS[0][0][0])[p];
+  for (int p = threadIdx.x; p < ND * ND * 6; p += NT) sRS[p / (ND * 6) * RST + p % (ND * 6)] = (mf_rt_t)(&SK_RS[0][0][0])[p];
 #endif
 #elif defined(SK_FULLRT)
   // full reference tensors R_ij[3 r + s] (9 per entry), loaded once per workgroup
@@ -286,8 +295,8 @@ $OHEAD($OPARAMS)
     for (int p = tid; p < CAP * (int)sizeof(mf_acc_t) / 16; p += nt) a4[p] = make_int4(0, 0, 0, 0);
   }
   for (int p = tid; p <= m0.y - m0.x; p += nt) lrp[p] = rpb[m0.x + p] - m1.x;
-  for (int p = tid; p < m0.y - m0.x; p += nt) snb[p] = nb0 ? nb0[m0.x + p] : 0;
-  for (int p = tid; p < m1.y; p += nt) lcols[p] = colsb[m1.x + p];
+  for (int p = tid; p < m0.y - m0.x; p += nt)
+    snb[p] = nb0 ? nb0[m0.x + p] | (dpos[m0.x + p] + 1) << 8 : 0;
 
   // pair index of this thread's first (pair, column range) unit in a chunk
   // of np pairs (same mapping as the unit loop below), -1 if it has none
@@ -342,14 +351,12 @@ $OHEAD($OPARAMS)
       // Dirichlet rows: the diagonal entries of constrained components receive
       // no contributions (their rows are masked), so they are set up front
       for (int lr = tid; lr < nr; lr += nt) {
-        const int32_t R = r0 + lr;
-        const uint32_t rbits = snb[lr];
-        if (!rbits) continue;
+        const uint32_t rbits = snb[lr] & 0xFF;
+        const int p = (snb[lr] >> 8) - 1;
+        if (!rbits || p < 0) continue;
         const int lo = lrp[lr], hi = lrp[lr + 1];
-        const int p = mf_lds_lower_bound(lcols, lo, hi, R);
-        if (p < hi && lcols[p] == R)
-          for (int a = 0; a < BS; ++a)
-            if (rbits & (1u << a)) acc[BS * BS * lo + a * BS * (hi - lo) + BS * (p - lo) + a] = diag;
+        for (int a = 0; a < BS; ++a)
+          if (rbits & (1u << a)) acc[BS * BS * lo + a * BS * (hi - lo) + BS * p + a] = diag;
       }
     }
     // prefetch the next chunk's lists into registers (issued before the
@@ -358,7 +365,7 @@ $OHEAD($OPARAMS)
     const bool more = jn < per && kn < nchunks;
     int4 n0 = {0, 0, 0, 0}, n1 = {0, 0, 0, 0}, n2 = {0, 0, 0, 0};
     uint32_t pvn = 0xFFFFFFFFu;
-    int pf_p[PF_P], pf_r[PF_R], pf_c[PF_C], pf_b[PF_B];
+    int pf_p[PF_P], pf_r[PF_R], pf_b[PF_B];
     int4 pf_k[PF_K];
     if (more) {
       n0 = reinterpret_cast<const int4*>(chunk_meta)[3 * kn];
@@ -382,14 +389,9 @@ $OHEAD($OPARAMS)
         pf_r[t] = p <= n0.y - n0.x ? rpb[n0.x + p] : 0;
       }
 #pragma unroll
-      for (int t = 0; t < PF_C; ++t) {
-        const int p = tid + t * NT;
-        pf_c[t] = p < n1.y ? colsb[n1.x + p] : 0;
-      }
-#pragma unroll
       for (int t = 0; t < PF_B; ++t) {
         const int p = tid + t * NT;
-        pf_b[t] = p < n0.y - n0.x && nb0 ? nb0[n0.x + p] : 0;
+        pf_b[t] = p < n0.y - n0.x && nb0 ? nb0[n0.x + p] | (dpos[n0.x + p] + 1) << 8 : 0;
       }
       // pair of this thread's first unit in the next chunk (its record is
       // loaded after the compute phase, while this chunk is written out)
@@ -534,14 +536,9 @@ $UNIT
         if (p <= n0.y - n0.x) lrp[p] = pf_r[t] - n1.x;
       }
 #pragma unroll
-      for (int t = 0; t < PF_C; ++t) {
-        const int p = tid + t * NT;
-        if (p < n1.y) lcols[p] = pf_c[t];
-      }
-#pragma unroll
       for (int t = 0; t < PF_B; ++t) {
         const int p = tid + t * NT;
-        if (p < n0.y - n0.x) snb[p] = (uint8_t)pf_b[t];
+        if (p < n0.y - n0.x) snb[p] = pf_b[t];
       }
     }
     m0 = n0; m1 = n1; m2 = n2;
@@ -861,14 +858,15 @@ $OHEAD($OPARAMS)
   __shared__ __attribute__((aligned(16))) int32_t lrp2[2][MAXR + 1];
   __shared__ __attribute__((aligned(16))) uint8_t snb2[2][MAXR];
 #ifdef SK_TRACE
-  __shared__ __attribute__((aligned(16))) mf_rt_t sRS[ND * ND * 6];
+  constexpr int RST = MF_RST(ND, sizeof(mf_rt_t));
+  __shared__ __attribute__((aligned(16))) mf_rt_t sRS[ND * RST];
 #if (SK_ND % 4 == 0) && MF_OWNER_F32
   for (int p = threadIdx.x; p < ND * ND * 6; p += NT + 64) {
     const int i = p / (6 * ND), k = (p / ND) % 6, j = p % ND;
-    sRS[p] = (mf_rt_t)SK_RS[i][j][k];
+    sRS[i * RST + k * ND + j] = (mf_rt_t)SK_RS[i][j][k];
   }
 #else
-  for (int p = threadIdx.x; p < ND * ND * 6; p += NT + 64) sRS[p] = (mf_rt_t)(&SK_RS[0][0][0])[p];
+  for (int p = threadIdx.x; p < ND * ND * 6; p += NT + 64) sRS[p / (ND * 6) * RST + p % (ND * 6)] = (mf_rt_t)(&SK_RS[0][0][0])[p];
 #endif
 #elif defined(SK_FULLRT)
   __shared__ __attribute__((aligned(16))) double sRT[ND * ND * 9];
@@ -1207,7 +1205,7 @@ const char* kOwnerUnit = R"(
         };
         // tr G_ij from the tensors in their row-major layout
         auto trace = [&](const int j) {
-          const mf_rt_t* R = &sRS[(i * ND + j) * 6];
+          const mf_rt_t* R = &sRS[i * RST + j * 6];
 #if MF_OWNER_F32
           return (double)(f00 * R[0] + f11 * R[1] + f22 * R[2] + f01 * R[3] + f02 * R[4] + f12 * R[5]);
 #else
@@ -1223,7 +1221,7 @@ const char* kOwnerUnit = R"(
 #if (SK_ND % 4 == 0) && MF_OWNER_F32
             // the transposed FP32 tensors: six 16-byte reads for four columns
             typedef float mf_f4 __attribute__((ext_vector_type(4)));
-            const mf_f4* R4 = reinterpret_cast<const mf_f4*>(&sRS[i * 6 * ND + jw]);
+            const mf_f4* R4 = reinterpret_cast<const mf_f4*>(&sRS[i * RST + jw]);
             const mf_f4 r0 = R4[0], r1 = R4[ND / 4], r2 = R4[2 * ND / 4];
             const mf_f4 r3 = R4[3 * ND / 4], r4 = R4[4 * ND / 4], r5 = R4[5 * ND / 4];
             const mf_f4 tg = f00 * r0 + f11 * r1 + f22 * r2 + f01 * r3 + f02 * r4 + f12 * r5;
