@@ -351,10 +351,9 @@ int staged_define(const std::string& src, const std::string& name) {
 
 int64_t record_bytes(const mf_form& f, const Integral& I) {
   // layout of kCellRecord: {K[9], det} or, for scalar reference-tensor forms,
-  // the metric M[6]; then w[max(1, W)], d[nd], bits; 16-byte aligned
-  const int nd = staged_define(I.staged_src, "SK_ND");
+  // the metric M[6]; then w[max(1, W)], bits; 16-byte aligned
   const int64_t geo = staged_trace(I) ? 48 : 72 + 8;
-  const int64_t raw = geo + 8LL * std::max(1, f.W) + 4LL * nd + 4;
+  const int64_t raw = geo + 8LL * std::max(1, f.W) + 4;
   return (raw + 15) / 16 * 16;
 }
 
@@ -915,13 +914,13 @@ std::string generate_batch_source(const std::vector<const mf_form*>& forms,
       // parameters in the order of kOwnerParams (and of the host's argument list)
       const std::string a = "g" + std::to_string(g) + "_";
       params += std::string(g ? ",\n    " : "") + "const int32_t " + a + "nchunks, const int32_t* __restrict__ " +
-                a + "chunk_meta, const int32_t* __restrict__ " + a + "item_cell, const int32_t* __restrict__ " +
-                a + "pair_list, const uint8_t* __restrict__ " + a + "pair_kk, const mf_rec_" + tag +
+                a + "chunk_meta, const int32_t* __restrict__ " + a + "pair_list, const uint16_t* __restrict__ " +
+                a + "pair_row, const uint8_t* __restrict__ " + a + "pair_kk, const mf_rec_" + tag +
                 "* __restrict__ " + a + "rec, const double* __restrict__ " + a +
                 "consts, const int32_t* __restrict__ " + a + "rpb, const int32_t* __restrict__ " + a +
                 "dpos, const uint8_t* __restrict__ " + a + "nb0, double* __restrict__ " + a + "values";
       calls += "  mf_owner_body_g" + std::to_string(g) + "(" + a + "nchunks, " + a + "chunk_meta, " +
-               a + "item_cell, " + a + "pair_list, " + a + "pair_kk, " + a + "rec, " + a + "consts, " +
+               a + "pair_list, " + a + "pair_row, " + a + "pair_kk, " + a + "rec, " + a + "consts, " +
                a + "rpb, " + a + "dpos, " + a + "nb0, " + a + "values, diag, flags" + sargs +
                ");\n  __syncthreads();\n";
     }

@@ -14,6 +14,7 @@ struct OwnerPlan {
   DevArray<int32_t> chunk_rows, chunk_items, item_cell, chunk_meta, pair_list;
   DevArray<uint32_t> item_mask;
   DevArray<uint8_t> pair_kk;
+  DevArray<uint16_t> pair_row;        // simplex kernels: each pair's row in its chunk
   DevArray<uint16_t> pair_pos;        // hexahedral kernel: row-relative position of each column
   DevArray<int32_t> item_geo;         // hexahedral kernel: the 8 vertices of each item's cell
   DevArray<int32_t> diag_pos;         // hexahedral kernel: row-relative position of the diagonal
@@ -175,6 +176,7 @@ std::shared_ptr<OwnerPlan> build_owner_plan(const mf_form& a, const Integral& I,
   }
   const int64_t np = poff[nch];
   std::vector<int32_t> plist(np + 1, 0);
+  std::vector<uint16_t> prow(with_kk ? np + 1 : 1, 0);
   // column offsets: one 16-byte aligned block of npairs * nd bytes per chunk
   std::vector<int64_t> kkoff(nch + 1, 0);
   for (int64_t c = 0; c < nch; ++c)
@@ -201,6 +203,7 @@ std::shared_ptr<OwnerPlan> build_owner_plan(const mf_form& a, const Integral& I,
           const int32_t R = d0->host[(int64_t)cell * nd + i];
           plist[p] = with_kk ? static_cast<int32_t>((static_cast<uint32_t>(cell) << 6) | i)
                              : ((it - ci[c]) << 16) | ((R - rows[c]) << 6) | i;
+          if (with_kk) prow[p] = static_cast<uint16_t>(R - rows[c]);
           const int32_t* rb = A.h_colsb.data() + A.h_rpb[R];
           const int32_t* re = A.h_colsb.data() + A.h_rpb[R + 1];
           if (!with_kk) {
@@ -261,6 +264,7 @@ std::shared_ptr<OwnerPlan> build_owner_plan(const mf_form& a, const Integral& I,
   plan->chunk_meta.upload(meta);
   plan->pair_list.upload(plist);
   plan->pair_kk.upload(pkk);
+  plan->pair_row.upload(prow);
   plan->pair_pos.upload(ppos);
   {
     // position of the diagonal block in each blocked row (-1: none): the
@@ -836,7 +840,7 @@ void assemble_matrix(mf_form* a, mf_matrix* A, const mf_bc* bc0, const mf_bc* bc
         pgrid = std::max<int64_t>(nx, (int64_t)std::max(1, nblk) * a->ctx->num_cus / nx * nx);
       }
       launch(kpipe, static_cast<uint32_t>(std::min<int64_t>(per * nx, pgrid)), pblock, 0, s,
-             static_cast<int32_t>(plan->nchunks), plan->chunk_meta.ptr, plan->pair_list.ptr,
+             static_cast<int32_t>(plan->nchunks), plan->chunk_meta.ptr, plan->pair_list.ptr, plan->pair_row.ptr,
              plan->pair_kk.ptr, owner->records.ptr, a->consts.ptr, A->rpb.ptr, plan->diag_pos.ptr,
              n0, A->values, diagonal, flags);
     } else {
@@ -852,8 +856,8 @@ void assemble_matrix(mf_form* a, mf_matrix* A, const mf_bc* bc0, const mf_bc* bc
       grid = std::min<int64_t>(grid, ogrid * a->opt("owner_waves", 1));
     }
     launch(kown, static_cast<uint32_t>(grid), oblock, 0, s,
-           static_cast<int32_t>(plan->nchunks), plan->chunk_meta.ptr, plan->item_cell.ptr,
-           plan->pair_list.ptr, plan->pair_kk.ptr, owner->records.ptr, a->consts.ptr, A->rpb.ptr,
+           static_cast<int32_t>(plan->nchunks), plan->chunk_meta.ptr, plan->pair_list.ptr,
+           plan->pair_row.ptr, plan->pair_kk.ptr, owner->records.ptr, a->consts.ptr, A->rpb.ptr,
            plan->diag_pos.ptr, n0, A->values, diagonal, flags);
     }
     }
@@ -1046,7 +1050,7 @@ void assemble_vbatch(mf_batch* B, double* const* d_b, const int64_t* n_b, int ze
 void assemble_batch(mf_batch* B, mf_matrix* const* As, const mf_bc* const* bcs, double diag,
                     int zero, hipStream_t s) {
   struct Args {   // one group's kernel arguments (see the pointer list below)
-    const void* chunk_meta; const void* item_cell; const void* pair_list; const void* pair_kk;
+    const void* chunk_meta; const void* pair_list; const void* pair_row; const void* pair_kk;
     const void* rec; const void* consts; const void* rpb; const void* dpos; const void* nb0;
     void* values; int32_t nchunks; int32_t pad;
   };
@@ -1079,7 +1083,7 @@ void assemble_batch(mf_batch* B, mf_matrix* const* As, const mf_bc* const* bcs, 
     launch(B->preps[g], static_cast<uint32_t>((I->n + 255) / 256), 256, 0, s,
            static_cast<int32_t>(I->n), I->d_ents.ptr, a->mesh->cells.ptr, a->mesh->x.ptr,
            a->packed.ptr, a->dm[0]->dev.ptr, n0, cf, I->records.ptr);
-    h[g] = Args{plan->chunk_meta.ptr, plan->item_cell.ptr, plan->pair_list.ptr, plan->pair_kk.ptr,
+    h[g] = Args{plan->chunk_meta.ptr, plan->pair_list.ptr, plan->pair_row.ptr, plan->pair_kk.ptr,
                 I->records.ptr, a->consts.ptr, A->rpb.ptr, plan->diag_pos.ptr, n0, A->values,
                 static_cast<int32_t>(plan->nchunks), 0};
   }
@@ -1092,7 +1096,7 @@ void assemble_batch(mf_batch* B, mf_matrix* const* As, const mf_bc* const* bcs, 
   for (size_t g = 0; g < ng; ++g) {
     Args& x = h[g];
     for (void* p : {static_cast<void*>(&x.nchunks), static_cast<void*>(&x.chunk_meta),
-                    static_cast<void*>(&x.item_cell), static_cast<void*>(&x.pair_list),
+                    static_cast<void*>(&x.pair_list), static_cast<void*>(&x.pair_row),
                     static_cast<void*>(&x.pair_kk), static_cast<void*>(&x.rec),
                     static_cast<void*>(&x.consts), static_cast<void*>(&x.rpb),
                     static_cast<void*>(&x.dpos), static_cast<void*>(&x.nb0),

@@ -76,7 +76,7 @@ static __device__ __forceinline__ int mf_xcd_chunk(int nchunks)
 // Parameters of one form's owner-computes body.
 const char* kOwnerParams =
     "const int32_t nchunks, const int32_t* __restrict__ chunk_meta, "
-    "const int32_t* __restrict__ item_cell, const int32_t* __restrict__ pair_list, "
+    "const int32_t* __restrict__ pair_list, const uint16_t* __restrict__ pair_row, "
     "const uint8_t* __restrict__ pair_kk, const mf_rec_$TAG* __restrict__ rec, "
     "const double* __restrict__ consts, const int32_t* __restrict__ rpb, "
     "const int32_t* __restrict__ dpos, const uint8_t* __restrict__ nb0, "
@@ -100,9 +100,14 @@ $CALLS}
 )";
 
 // Per-cell record consumed by the owner kernel (square forms): geometry
-// factors, packed coefficients, row dofs and their Dirichlet bits, written
+// factors, packed coefficients and the Dirichlet bits of its dofs, written
 // once per assembly by mf_prep_* in cell order.
-//   double K[9], |det J|, w[W]; int32 dofs[ND]; uint32 bits (BS*ND <= 32)
+//   double K[9], |det J|, w[W]; uint32 bits (BS*ND <= 32)
+// The lanes of a wave read as many records, each load a cache line per lane, so
+// what the schedule can hold (a pair's row) is not in here: 64 bytes for scalar
+// forms with one coefficient (80 to 144 with the dofs in it): the
+// pass that writes them 20 -> 16 us on 750 thousand P1 cells, 31 -> 22 us on 664
+// thousand vector P2 cells, a batch of 48 P1-P3 instances 31 -> 23 us in all.
 const char* kCellRecord = R"(
 #ifndef MF_REC_$TAG
 #define MF_REC_$TAG
@@ -114,7 +119,6 @@ struct __attribute__((aligned(16))) mf_rec_$TAG {
   double det;
 #endif
   double w[$WW];
-  int32_t d[SK_ND];
   uint32_t bits;
 };
 #endif
@@ -176,11 +180,8 @@ $KNAME(const int32_t n, const int32_t* __restrict__ ents, const int32_t* __restr
     for (int l = 0; l < $WW; ++l) r.w[l] = l < W ? coeffs[c * W + l] : 0.0;
     uint32_t bits = 0;
     const bool gather = nb0 && cflag[c];
-    for (int l = 0; l < ND; ++l) {
-      const int32_t node = dm0[c * ND + l];
-      r.d[l] = node;
-      if (gather) bits |= (uint32_t)nb0[node] << (BS * l);
-    }
+    if (gather)
+      for (int l = 0; l < ND; ++l) bits |= (uint32_t)nb0[dm0[c * ND + l]] << (BS * l);
     r.bits = bits;
     if (staged)
       reinterpret_cast<mf_rec_$TAG*>(srec)[threadIdx.x] = r;
@@ -208,7 +209,7 @@ $OHEAD($OPARAMS)
   // chunk_meta[12k ..]: r0, r1, i0, i1, cb0 (= rpb[r0]), ncb, base (CSR offset),
   //   seglen, p0, p1 (pair range), kko (byte offset of the chunk's column
   //   offsets, 16-byte aligned), 0.
-  // pair_list[p] = cell << 6 | local row i; pair_kk[kko + (p-p0)*ND + j] = position of
+  // pair_list[p] = cell << 6 | local row i, pair_row[p] = its row in the chunk; pair_kk[kko + (p-p0)*ND + j] = position of
   //   column node j within the blocked row of node i.  Each (pair, column range)
   //   thread reads its cell's record straight from memory (neighbouring chunks
   //   share cells, so these reads mostly hit L2): no staging batches, no barriers
@@ -316,12 +317,13 @@ $OHEAD($OPARAMS)
   // this thread's first unit: pair value and the record fields it needs,
   // loaded one chunk ahead so the compute phase starts with them in registers
   uint32_t u_pv = 0, u_bits = 0;
-  int32_t u_di = 0;
+  int32_t u_lr = 0;
   double u_K[9], u_det = 0.0, u_w[$WW];
   for (int x = 0; x < 9; ++x) u_K[x] = 0.0;
   for (int x = 0; x < $WW; ++x) u_w[x] = 0.0;
   auto mf_load_unit = [&](uint32_t pv) {
-    const mf_rec_$TAG& r = rec[pv >> 6];
+    mf_rec_$TAG r;                                     // in 16-byte loads
+    __builtin_memcpy(&r, __builtin_assume_aligned(&rec[pv >> 6], 16), sizeof(r));
 #ifdef SK_TRACE
     for (int x = 0; x < 6; ++x) u_K[x] = r.M[x];       // the metric, see the record
 #else
@@ -329,13 +331,13 @@ $OHEAD($OPARAMS)
     u_det = r.det;
 #endif
     for (int x = 0; x < $WW; ++x) u_w[x] = r.w[x];
-    u_di = r.d[pv & 63];
     u_bits = r.bits;
   };
   {
     const int pr0 = mf_first_pair(m2.y - m2.x);
     if (pr0 >= 0) {
       u_pv = (uint32_t)pair_list[m2.x + pr0];
+      u_lr = pair_row[m2.x + pr0];
       mf_load_unit(u_pv);
     }
   }
@@ -344,7 +346,7 @@ $OHEAD($OPARAMS)
     const int32_t r0 = m0.x, r1 = m0.y;
     const int32_t base = m1.z, seglen = m1.w;
     const int nr = r1 - r0;
-    const int npc = m2.y - m2.x;
+    const int npc = m2.y - m2.x, p0 = m2.x;
 
     __syncthreads();                                   // lists and zeroed acc visible
     if ((flags & 2) && nb0) {
@@ -365,6 +367,7 @@ $OHEAD($OPARAMS)
     const bool more = jn < per && kn < nchunks;
     int4 n0 = {0, 0, 0, 0}, n1 = {0, 0, 0, 0}, n2 = {0, 0, 0, 0};
     uint32_t pvn = 0xFFFFFFFFu;
+    int32_t lrn = 0;
     int pf_p[PF_P], pf_r[PF_R], pf_b[PF_B];
     int4 pf_k[PF_K];
     if (more) {
@@ -396,7 +399,10 @@ $OHEAD($OPARAMS)
       // pair of this thread's first unit in the next chunk (its record is
       // loaded after the compute phase, while this chunk is written out)
       const int prn = mf_first_pair(n2.y - n2.x);
-      if (prn >= 0) pvn = (uint32_t)pair_list[n2.x + prn];
+      if (prn >= 0) {
+        pvn = (uint32_t)pair_list[n2.x + prn];
+        lrn = pair_row[n2.x + prn];
+      }
     }
     __builtin_amdgcn_s_setprio(0);
     {
@@ -423,6 +429,7 @@ $OHEAD($OPARAMS)
         const int pc = pr;                             // pair index within the chunk
         if (reload) {                                  // later segments: load directly
           u_pv = (uint32_t)spair[pc];
+          u_lr = pair_row[p0 + pc];
           mf_load_unit(u_pv);
         }
         const int u_j0 = jb, u_j1 = je;
@@ -444,6 +451,7 @@ $UNIT
         const int pc = pr;                             // pair index within the chunk
         if (u != tid) {                                // later units: load directly
           u_pv = (uint32_t)spair[pc];
+          u_lr = pair_row[p0 + pc];
           mf_load_unit(u_pv);
         }
         const int u_j0 = part * jw, u_j1 = min(ND, u_j0 + jw);
@@ -454,6 +462,7 @@ $UNIT
     __syncthreads();                                   // all contributions in acc
     if (pvn != 0xFFFFFFFFu) {
       u_pv = pvn;
+      u_lr = lrn;
       mf_load_unit(pvn);
     }
 
@@ -545,7 +554,6 @@ $UNIT
     jj = jn;
     k = kn;
   }
-  (void)item_cell;
 }
 )";
 
@@ -818,7 +826,8 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
 // Parameters of the warp-specialised owner-computes kernel.
 const char* kOwnerPipeParams =
     "const int32_t nchunks, const int32_t* __restrict__ chunk_meta, "
-    "const int32_t* __restrict__ pair_list, const uint8_t* __restrict__ pair_kk, "
+    "const int32_t* __restrict__ pair_list, const uint16_t* __restrict__ pair_row, "
+    "const uint8_t* __restrict__ pair_kk, "
     "const mf_rec_$TAG* __restrict__ rec, const double* __restrict__ consts, "
     "const int32_t* __restrict__ rpb, const int32_t* __restrict__ dpos, "
     "const uint8_t* __restrict__ nb0, double* __restrict__ values, const double diag, "
@@ -890,12 +899,13 @@ $OHEAD($OPARAMS)
   const int4* meta4 = reinterpret_cast<const int4*>(chunk_meta);
   int4 m0 = {0, 0, 0, 0}, m1 = {0, 0, 0, 0}, m2 = {0, 0, 0, 0};
   uint32_t u_pv = 0, u_bits = 0;
-  int32_t u_di = 0;
+  int32_t u_lr = 0;
   double u_K[9], u_det = 0.0, u_w[$WW];
   for (int x = 0; x < 9; ++x) u_K[x] = 0.0;
   for (int x = 0; x < $WW; ++x) u_w[x] = 0.0;
   auto mf_load_unit = [&](uint32_t pv) {
-    const mf_rec_$TAG& r = rec[pv >> 6];
+    mf_rec_$TAG r;                                     // in 16-byte loads
+    __builtin_memcpy(&r, __builtin_assume_aligned(&rec[pv >> 6], 16), sizeof(r));
 #ifdef SK_TRACE
     for (int x = 0; x < 6; ++x) u_K[x] = r.M[x];       // the metric, see the record
 #else
@@ -903,7 +913,6 @@ $OHEAD($OPARAMS)
     u_det = r.det;
 #endif
     for (int x = 0; x < $WW; ++x) u_w[x] = r.w[x];
-    u_di = r.d[pv & 63];
     u_bits = r.bits;
   };
   // pair index of this thread's first (pair, column range) unit in a chunk
@@ -963,6 +972,7 @@ $OHEAD($OPARAMS)
     const int pr0 = mf_first_pair(m2.y - m2.x);
     if (pr0 >= 0) {
       u_pv = (uint32_t)pair_list[m2.x + pr0];
+      u_lr = pair_row[m2.x + pr0];
       mf_load_unit(u_pv);
     }
   }
@@ -997,6 +1007,7 @@ $OHEAD($OPARAMS)
       }
       // the next chunk's lists into registers (latency hidden by the units)
       uint32_t pvn = 0xFFFFFFFFu;
+      int32_t lrn = 0;
       int pf_p[PF_P], pf_r[PF_R], pf_b[PF_B];
       int4 pf_k[PF_K];
       if (more) {
@@ -1026,7 +1037,10 @@ $OHEAD($OPARAMS)
           pf_b[t] = p < n0.y - n0.x && nb0 ? nb0[n0.x + p] : 0;
         }
         const int prn = mf_first_pair(nnp);
-        if (prn >= 0) pvn = (uint32_t)pair_list[n2.x + prn];
+        if (prn >= 0) {
+          pvn = (uint32_t)pair_list[n2.x + prn];
+          lrn = pair_row[n2.x + prn];
+        }
       }
       {
         // one thread per (pair, column range); lanes of a wave share the
@@ -1044,6 +1058,7 @@ $OHEAD($OPARAMS)
           const int pc = pr;                           // pair index within the chunk
           if (u != tid) {                              // later units: load directly
             u_pv = (uint32_t)spair[pc];
+            u_lr = pair_row[m2.x + pc];
             mf_load_unit(u_pv);
           }
           const int u_j0 = part * jw, u_j1 = min(ND, u_j0 + jw);
@@ -1076,6 +1091,7 @@ $UNIT
         }
         if (pvn != 0xFFFFFFFFu) {
           u_pv = pvn;
+          u_lr = lrn;
           mf_load_unit(pvn);
         }
       }
@@ -1130,7 +1146,7 @@ const char* kOwnerUnit = R"(
 #endif
         const uint32_t bits = u_bits;
         const uint32_t rb0 = (bits >> (BS * i)) & ((1u << BS) - 1);
-        const int lr = u_di - r0;
+        const int lr = u_lr;
         const int lo = lrp[lr], hi = lrp[lr + 1];
         const int rowlen = BS * (hi - lo);
         const int rbase = BS * BS * lo;
