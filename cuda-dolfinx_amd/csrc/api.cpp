@@ -1151,6 +1151,7 @@ int mf_autotune_matrix(mf_form* a, mf_matrix* A, const mf_bc* bc, int reps, mf_s
         {{"chunk_values", 4608}, {"owner_pairs", 384}, {"owner_block", 256}, {"owner_lds", 73728}},
     };
     const auto base = a->options;
+    const bool base_default = a->shape_default;
     auto drop_plans = [&] {
       for (auto it = A->plans.begin(); it != A->plans.end();)
         it = it->first.first == a->uid ? A->plans.erase(it) : std::next(it);
@@ -1164,6 +1165,7 @@ int mf_autotune_matrix(mf_form* a, mf_matrix* A, const mf_bc* bc, int reps, mf_s
       a->options = base;
       for (auto& kv : cands[k]) a->options[kv.first] = kv.second;
       a->options["matrix_kernel"] = 2;
+      a->shape_default = false;
       try {
         compile_form(a, 0);
         drop_plans();
@@ -1186,6 +1188,7 @@ int mf_autotune_matrix(mf_form* a, mf_matrix* A, const mf_bc* bc, int reps, mf_s
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     a->options = base;
+    a->shape_default = best_k < 0 && base_default;
     std::string desc;
     if (best_k >= 0)
       for (auto& kv : cands[best_k]) {

@@ -330,6 +330,7 @@ struct mf_form {
   std::unique_ptr<mf::Module> mod;
   std::string source;
   std::map<std::string, int64_t> options;
+  bool shape_default = false;         // chunk_values and owner_pairs are the library's choice
   std::map<int, std::shared_ptr<mf::OwnerPlan>> vplans;   // owner-computes vector schedules
   std::map<int, std::unique_ptr<mf::VectorBlocks>> vblocks;   // blocks of cell integrals
   hipFunction_t k_dgown = nullptr;    // cell-owner kernel over all integrals (DG spaces)

@@ -325,3 +325,25 @@ def test_fused_system_adds_with_dirichlet_rows(n):
         assert _rel(A.csr()[2], ref) <= TOL
         assert _rel(b.to_host(), times * rhs) <= TOL
         ref = o.assemble_matrix(rp, cols, [bc], diagonal=2.5, values=ref.copy())
+
+
+@pytest.mark.parametrize("which,times", [("vector", 1), ("vector", 7), ("vector", 8), ("vector", 17),
+                                         (2, 10), (2, 12), (3, 11), (3, 17)])
+def test_matrix_rows_with_many_cells(which, times):
+    """Rows around the numbers of (cell, row) pairs at which the owner kernel's shape
+    changes (160 vector, 256 scalar) and past its largest (384): every cell of a cube
+    listed several times, so that its inner node has 24 cells as often."""
+    import dataclasses
+    import cudolfinx as cufem
+    print(f"[gpu-test] matrix {which} with cells listed {times} times", flush=True)
+    V, a, _ = _elasticity(2) if which == "vector" else _poisson(2, which)
+    ents = np.repeat(np.arange(V.mesh.num_cells, dtype=np.int32), times)
+    a = dataclasses.replace(a, integrals=[dataclasses.replace(a.integrals[0], entities=ents)])
+    bc = _some_dofs(V, 0.1, 3)
+    asm = cufem.CUDAAssembler()
+    A = asm.assemble_matrix(cufem.form(a), bcs=[bc])
+    asm.synchronize()
+    o = cpu.OracleAssembler(a)
+    rp, cols, _, _ = o.sparsity()
+    ref = o.assemble_matrix(rp, cols, [bc])
+    assert _rel(A.csr()[2], ref) <= TOL
