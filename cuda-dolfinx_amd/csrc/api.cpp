@@ -444,12 +444,12 @@ void compile_form(mf_form* f, int verbose) {
 
 // packs every coefficient that has values (all of them after set_coefficient)
 void pack_all(mf_form* f, hipStream_t s) {
+  std::vector<mf::PackItem> items;
   for (auto& c : f->coefs) {
     const double* v = c.ext ? c.ext : c.own.ptr;
-    if (!v) continue;
-    mf::k_pack(f->packed.ptr, f->mesh->num_cells, f->W, c.offset, v, c.dm->dev.ptr, c.dm->nd,
-               c.dm->bs, s);
+    if (v) items.push_back({v, c.dm->dev.ptr, c.dm->nd, c.dm->bs, c.offset});
   }
+  mf::k_pack(f->packed.ptr, f->mesh->num_cells, f->W, items.data(), static_cast<int>(items.size()), s);
 }
 }  // namespace
 
@@ -476,16 +476,19 @@ int mf_form_pack_coefficients(mf_form* f, const int* idx, int n, mf_stream s) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     MF_HIP(hipStreamIsCapturing(S(s), &cap));
     const bool capturing = cap != hipStreamCaptureStatusNone;
+    std::vector<mf::PackItem> items;
     for (int j : sel) {
       MF_CHECK(j >= 0 && j < (int)f->coefs.size(), MF_EINVAL, "coefficient index out of range");
       auto& c = f->coefs[j];
       const double* v = c.ext ? c.ext : c.own.ptr;
       MF_CHECK(v, MF_ESTATE, "coefficient " + std::to_string(j) + " has no values");
       if (!c.ext && !c.dirty && !capturing) continue;
-      mf::k_pack(f->packed.ptr, f->mesh->num_cells, f->W, c.offset, v, c.dm->dev.ptr, c.dm->nd,
-                 c.dm->bs, S(s));
-      if (!c.ext && !capturing) c.dirty = false;
+      items.push_back({v, c.dm->dev.ptr, c.dm->nd, c.dm->bs, c.offset});
     }
+    mf::k_pack(f->packed.ptr, f->mesh->num_cells, f->W, items.data(), static_cast<int>(items.size()),
+               S(s));
+    if (!capturing)
+      for (int j : sel) f->coefs[j].dirty &= f->coefs[j].ext != nullptr;
   });
 }
 

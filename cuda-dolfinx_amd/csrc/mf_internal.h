@@ -139,8 +139,12 @@ void k_node_bits(uint8_t* bits, const int8_t* markers, int64_t nnodes, int bs, h
 // flags[c] = 1 if any node of cell c (dofmap dm, nd nodes per cell) has bits
 void k_cell_flags(uint8_t* flags, const int32_t* dm, int64_t ncells, int nd, const uint8_t* bits,
                   hipStream_t s);
-void k_pack(double* packed, int64_t ncells, int W, int off, const double* values,
-            const int32_t* dofmap, int nd, int bs, hipStream_t s);
+struct PackItem {                      // one coefficient of a form
+  const double* values;
+  const int32_t* dofmap;
+  int nd, bs, off;
+};
+void k_pack(double* packed, int64_t ncells, int W, const PackItem* items, int n, hipStream_t s);
 struct SetBcGroup {
   double* b;
   const int32_t* dofs;

@@ -106,17 +106,43 @@ __global__ void node_bits_kernel(uint8_t* __restrict__ bits, const int8_t* __res
   }
 }
 
-// packed[c*W + off + k*bs + j] = values[bs*dofmap[c*nd + k] + j]
-__global__ void pack_kernel(double* __restrict__ packed, int64_t ncells, int W, int off,
-                            const double* __restrict__ values, const int32_t* __restrict__ dofmap,
-                            int nd, int bs) {
-  const int64_t total = ncells * nd * bs;
-  int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; l < total; l += stride) {
-    int64_t c = l / (nd * bs);
-    int r = static_cast<int>(l - c * nd * bs);
-    int k = r / bs, j = r - k * bs;
-    packed[c * W + off + r] = values[(int64_t)bs * dofmap[c * nd + k] + j];
+// packed[c*W + off + k*bs + j] = values[bs*dofmap[c*nd + k] + j] for up to kPack
+// coefficients of a form at once.  Threads run over the packed entries (cum: first
+// entry of each coefficient among those packed), so a wave writes consecutive
+// addresses whatever the widths, and a form's coefficients cost one launch.  N:
+// number of coefficients, selected by compares; I: 32-bit indices where they do.
+// Bound by launches at these sizes (4 to 7 us each): two P2 coefficients on 48
+// thousand cells 10.6 -> 5.4 us.
+constexpr int kPack = 8;
+struct PackArgs {
+  const double* values[kPack];
+  const int32_t* dofmap[kPack];
+  int32_t nd[kPack], bs[kPack], off[kPack], cum[kPack + 1];
+};
+
+template <int N, class I>
+__global__ void pack_kernel(double* __restrict__ packed, int64_t ncells, int W, const PackArgs a) {
+  const I width = a.cum[N], total = static_cast<I>(ncells) * width;
+  const I stride = static_cast<I>(gridDim.x) * blockDim.x;
+  for (I l = static_cast<I>(blockIdx.x) * blockDim.x + threadIdx.x; l < total; l += stride) {
+    const I c = l / width;
+    const int rr = static_cast<int>(l - c * width);
+    const double* values = a.values[0];
+    const int32_t* dofmap = a.dofmap[0];
+    int nd = a.nd[0], bs = a.bs[0], off = a.off[0], first = 0;
+#pragma unroll
+    for (int g = 1; g < N; ++g)
+      if (rr >= a.cum[g]) {
+        values = a.values[g];
+        dofmap = a.dofmap[g];
+        nd = a.nd[g];
+        bs = a.bs[g];
+        off = a.off[g];
+        first = a.cum[g];
+      }
+    const int r = rr - first, k = bs == 1 ? r : r / bs, j = r - k * bs;
+    packed[static_cast<int64_t>(c) * W + off + r] =
+        values[static_cast<int64_t>(bs) * dofmap[static_cast<int64_t>(c) * nd + k] + j];
   }
 }
 
@@ -554,12 +580,38 @@ void k_node_bits(uint8_t* bits, const int8_t* m, int64_t nnodes, int bs, hipStre
   node_bits_kernel<<<grid_for(nnodes), kBlock, 0, s>>>(bits, m, nnodes, bs);
   MF_HIP(hipGetLastError());
 }
-void k_pack(double* packed, int64_t ncells, int W, int off, const double* values,
-            const int32_t* dofmap, int nd, int bs, hipStream_t s) {
+template <class I>
+static void pack_launch(double* packed, int64_t ncells, int W, const PackArgs& a, int n, hipStream_t s) {
+  const int grid = grid_for(ncells * a.cum[n]);
+  switch (n) {
+    case 1: pack_kernel<1, I><<<grid, kBlock, 0, s>>>(packed, ncells, W, a); break;
+    case 2: pack_kernel<2, I><<<grid, kBlock, 0, s>>>(packed, ncells, W, a); break;
+    case 3: pack_kernel<3, I><<<grid, kBlock, 0, s>>>(packed, ncells, W, a); break;
+    case 4: pack_kernel<4, I><<<grid, kBlock, 0, s>>>(packed, ncells, W, a); break;
+    default: pack_kernel<kPack, I><<<grid, kBlock, 0, s>>>(packed, ncells, W, a);
+  }
+}
+void k_pack(double* packed, int64_t ncells, int W, const PackItem* items, int n, hipStream_t s) {
   if (ncells <= 0) return;
-  pack_kernel<<<grid_for(ncells * nd * bs), kBlock, 0, s>>>(packed, ncells, W, off, values, dofmap,
-                                                             nd, bs);
-  MF_HIP(hipGetLastError());
+  for (int i0 = 0; i0 < n; i0 += kPack) {
+    const int m = std::min(n - i0, kPack);
+    PackArgs a{};
+    for (int g = 0; g < kPack; ++g) {
+      if (g < m) {
+        const PackItem& q = items[i0 + g];
+        a.values[g] = q.values;
+        a.dofmap[g] = q.dofmap;
+        a.nd[g] = q.nd;
+        a.bs[g] = q.bs;
+        a.off[g] = q.off;
+      }
+      a.cum[g + 1] = a.cum[g] + (g < m ? a.nd[g] * a.bs[g] : 0);
+    }
+    // the last of a thread's entries is below total + the grid's threads
+    if (ncells * a.cum[m] < (int64_t(1) << 31)) pack_launch<uint32_t>(packed, ncells, W, a, m, s);
+    else pack_launch<int64_t>(packed, ncells, W, a, m, s);
+    MF_HIP(hipGetLastError());
+  }
 }
 void k_set_bc_batch(const SetBcGroup* groups, int ngroups, double scale, hipStream_t s) {
   MF_CHECK(ngroups >= 0 && ngroups <= 32, MF_EINVAL, "at most 32 vectors per set_bc batch");

@@ -347,3 +347,53 @@ def test_matrix_rows_with_many_cells(which, times):
     rp, cols, _, _ = o.sparsity()
     ref = o.assemble_matrix(rp, cols, [bc])
     assert _rel(A.csr()[2], ref) <= TOL
+
+
+@pytest.mark.parametrize("n,count", [(1, 1), (3, 2), (2, 3), (4, 4), (3, 5), (2, 8), (3, 9), (2, 17)])
+def test_packed_coefficients_of_one_form(n, count):
+    """Coefficients of widths 1, 4, 10 and 12 packed together, more of them than one
+    launch takes; then some of them changed: b_i = (i + 1) sum_k (k + 1) w_k."""
+    import cudolfinx as cufem
+    from mifem.forms import _SIG, CELL, Form, Integral
+    print(f"[gpu-test] {count} coefficients on n={n}", flush=True)
+    mesh = create_unit_cube(n, jitter=0.1, seed=2)
+    V = functionspace(mesh, ("P", 1))
+    spaces = [functionspace(mesh, ("DG", 0)), V, functionspace(mesh, ("P", 2)), functionspace(mesh, ("P", 1), (3,))]
+    w = [Function(spaces[k % 4]) for k in range(count)]
+    rng = np.random.default_rng(count)
+    for f in w:
+        f.x[:] = rng.uniform(-1, 1, f.x.size)
+    width = sum(f.function_space.element.ndofs * f.function_space.bs for f in w)
+    name = f"tabulate_tensor_integral_packs_{count}"
+    src = _SIG.format(name=name) + f"""
+{{
+  double s = 0.0;
+  for (int k = 0; k < {width}; ++k) s += (k + 1) * w[k];
+  for (int i = 0; i < 4; ++i) A[i] += (i + 1) * s;
+}}
+"""
+    cells = np.arange(mesh.num_cells, dtype=np.int32)
+    L = Form(1, [V], [Integral(CELL, -1, cells, name, src, None, {})], w, [], "packs")
+
+    def reference():
+        packed = []
+        for f in w:
+            S = f.function_space
+            dofs = S.bs * np.repeat(S.dofmap, S.bs, axis=1) + np.tile(np.arange(S.bs), S.element.ndofs)
+            packed.append(f.x[dofs])
+        s = np.concatenate(packed, axis=1) @ np.arange(1.0, width + 1)
+        b = np.zeros(V.size)
+        np.add.at(b, V.dofmap, s[:, None] * np.arange(1.0, 5.0))
+        return b
+
+    asm = cufem.CUDAAssembler()
+    form = cufem.form(L)
+    b = asm.assemble_vector(form)
+    asm.synchronize()
+    assert _rel(b.to_host(), reference()) <= TOL
+    for f in w[::2]:
+        f.x[:] = rng.uniform(-1, 1, f.x.size)
+    form.to_device()
+    b = asm.assemble_vector(form, b)
+    asm.synchronize()
+    assert _rel(b.to_host(), reference()) <= TOL
