@@ -2,7 +2,9 @@
 // per-integral launches (CUDAAssembler::assemble_matrix,
 // cpp/cudolfinx/fem/CUDAAssembler.h:683-740, and set_diagonal :878-958).
 #include <algorithm>
+#include <array>
 #include <cstdio>
+#include <numeric>
 #include <thread>
 
 #include "mf_internal.h"
@@ -188,50 +190,102 @@ std::shared_ptr<OwnerPlan> build_owner_plan(const mf_form& a, const Integral& I,
   std::vector<uint16_t> ppos(with_kk ? 8 : std::max<int64_t>(8, np * nd), 0);
   std::vector<int> bad(16, 0);
   unsigned nt = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
+  // Order of a simplex chunk's pairs.  The lanes of a wave add an entry of the same
+  // column j of their pairs into LDS at once, 16 lanes at a time (groups of 8, 32
+  // and 64 were slower), and adds that meet in a bank (32 of 8 bytes) or at one
+  // address wait for each other.  So the pairs are dealt to groups of 16 one by one,
+  // each to the group where its addresses meet the fewest so far: first one pair of
+  // every row, then the next, a row's local indices in turn.  Vector P2 48^3
+  // matrix 742 us with the pairs in the order of the cells, 627 dealt in turn
+  // without regard to banks, 610 so; 13^3 30 -> 24 us, P2 25^3 29 -> 27, P3 24^3
+  // 74.5 -> 73.5.  P1, 24 pairs to a row, stays in the order of the cells: there it
+  // is the records that are scattered then (50^3 48 -> 58 us).
+  constexpr int kGroup = 16;
+  struct Pair {
+    int32_t cell, i, row, turn;
+    uint8_t kk[32];
+  };
+  auto order_pairs = [&](std::vector<Pair>& P, int64_t c, std::vector<int32_t>& place) {
+    const int np = static_cast<int>(P.size()), nb = (np + kGroup - 1) / kGroup, bs = A.bs0;
+    const int64_t cb0 = A.h_rpb[rows[c]];
+    std::vector<std::array<int32_t, 4>> order(np);      // turn, row, local row, pair
+    for (int k = 0; k < np; ++k) order[k] = {P[k].row, P[k].turn, P[k].i, k};
+    std::sort(order.begin(), order.end());
+    std::vector<int32_t> count(rows[c + 1] - rows[c], 0);
+    for (auto& q : order) q = {count[q[0]]++, q[0], 0, q[3]};
+    std::sort(order.begin(), order.end());
+    place.resize(np);
+    if (nb == 1) {
+      for (int k = 0; k < np; ++k) place[order[k][3]] = k;
+      return;
+    }
+    std::vector<uint8_t> load(static_cast<size_t>(nb) * nd * bs * 32, 0);
+    std::vector<int> fill(nb, 0);
+    std::vector<int> bank(nd * bs);
+    for (auto& q : order) {
+      const Pair& x = P[q[3]];
+      const int64_t R = rows[c] + x.row, len = A.h_rpb[R + 1] - A.h_rpb[R];
+      const int64_t lo = (int64_t)bs2 * (A.h_rpb[R] - cb0);
+      for (int j = 0; j < nd; ++j)
+        for (int e = 0; e < bs; ++e)
+          bank[j * bs + e] = (j * bs + e) * 32 + static_cast<int>((lo + e * A.bs1 * len + A.bs1 * x.kk[j]) & 31);
+      int best = -1, least = INT32_MAX;
+      for (int h = 0; h < nb; ++h) {
+        if (fill[h] == std::min(kGroup, np - kGroup * h)) continue;
+        const uint8_t* l = &load[(size_t)h * nd * bs * 32];
+        int meet = 0;
+        for (int k : bank) meet += l[k];
+        if (meet < least) {
+          least = meet;
+          best = h;
+        }
+      }
+      for (int k : bank) ++load[(size_t)best * nd * bs * 32 + k];
+      place[q[3]] = kGroup * best + fill[best]++;
+    }
+  };
   auto work = [&](unsigned t) {
+    std::vector<Pair> P;
+    std::vector<int32_t> place, turn;
     for (int64_t c = t; c < nch; c += nt) {
+      P.clear();
+      turn.assign(with_kk ? static_cast<size_t>(rows[c + 1] - rows[c]) * nd : 0, 0);
       int64_t p = poff[c];
-      uint8_t* kkc = pkk.data() + kkoff[c] - poff[c] * nd;   // pair p of chunk c at kkc[p * nd]
       for (int32_t it = ci[c]; it < ci[c + 1]; ++it) {
         const int32_t cell = plan->h_cell[it];
-        uint64_t msk = plan->h_mask[it];
-        while (msk) {
+        for (uint64_t msk = plan->h_mask[it]; msk; msk &= msk - 1) {
           const int i = __builtin_ctzll(msk);
-          msk &= msk - 1;
-          // simplex kernel (column offsets precomputed): cell id << 6 | local row;
-          // hexahedral kernel: item in the chunk << 16 | row in the chunk << 6 | local row
           const int32_t R = d0->host[(int64_t)cell * nd + i];
-          plist[p] = with_kk ? static_cast<int32_t>((static_cast<uint32_t>(cell) << 6) | i)
-                             : ((it - ci[c]) << 16) | ((R - rows[c]) << 6) | i;
-          if (with_kk) prow[p] = static_cast<uint16_t>(R - rows[c]);
           const int32_t* rb = A.h_colsb.data() + A.h_rpb[R];
           const int32_t* re = A.h_colsb.data() + A.h_rpb[R + 1];
-          if (!with_kk) {
-            for (int j = 0; j < nd; ++j) {
-              const int32_t Cn = d1->host[(int64_t)cell * nd + j];
-              const int32_t* f = std::lower_bound(rb, re, Cn);
-              if (f == re || *f != Cn || f - rb > 65535) {
-                bad[t % 16] = 1;
-                ppos[p * nd + j] = 0;
-              } else {
-                ppos[p * nd + j] = static_cast<uint16_t>(f - rb);
-              }
-            }
-            ++p;
-            continue;
-          }
+          const int64_t longest = with_kk ? 255 : 65535;
+          if (with_kk) P.push_back({cell, i, R - rows[c], turn[(size_t)(R - rows[c]) * nd + i]++, {}});
           for (int j = 0; j < nd; ++j) {
             const int32_t Cn = d1->host[(int64_t)cell * nd + j];
             const int32_t* f = std::lower_bound(rb, re, Cn);
-            if (f == re || *f != Cn || f - rb > 255) {
-              bad[t % 16] = 1;
-              kkc[p * nd + j] = 0;
-            } else {
-              kkc[p * nd + j] = static_cast<uint8_t>(f - rb);
-            }
+            const bool ok = f != re && *f == Cn && f - rb <= longest;
+            if (!ok) bad[t % 16] = 1;
+            if (with_kk) P.back().kk[j] = ok ? static_cast<uint8_t>(f - rb) : 0;
+            else ppos[p * nd + j] = ok ? static_cast<uint16_t>(f - rb) : 0;
           }
-          ++p;
+          // hexahedral kernel: item in the chunk << 16 | row in the chunk << 6 | local row
+          if (!with_kk) plist[p++] = ((it - ci[c]) << 16) | ((R - rows[c]) << 6) | i;
         }
+      }
+      if (!with_kk) continue;
+      if (nd > 4) {
+        order_pairs(P, c, place);
+      } else {
+        place.resize(P.size());
+        std::iota(place.begin(), place.end(), 0);
+      }
+      uint8_t* kkc = pkk.data() + kkoff[c];
+      for (size_t k = 0; k < P.size(); ++k) {
+        // simplex kernel (column offsets precomputed): cell id << 6 | local row
+        const int64_t q = place[k];
+        plist[poff[c] + q] = static_cast<int32_t>((static_cast<uint32_t>(P[k].cell) << 6) | P[k].i);
+        prow[poff[c] + q] = static_cast<uint16_t>(P[k].row);
+        std::copy_n(P[k].kk, nd, &kkc[q * nd]);
       }
     }
   };

@@ -51,15 +51,6 @@ typedef float mf_f2 __attribute__((ext_vector_type(2)));
 // With the column list gone too: P3 24^3 93 -> 73 us, a batch of 48 P1-P3
 // instances in FP32 159 -> 110 us, vector P2 48^3 818 -> 778 us.
 #define MF_RST(nd, sz) ((nd) * 6 + (8 - (nd) * 6 * ((sz) / 4) % 8 + 4) % 8 / ((sz) / 4))
-static __device__ __forceinline__ int mf_lds_lower_bound(const int32_t* a, int lo, int hi, int32_t key)
-{
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (a[mid] < key) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo;
-}
 // XCD-aware chunk order: consecutive workgroups land on different XCDs, so
 // each XCD gets a contiguous run of chunks (neighbouring chunks share cells).
 static __device__ __forceinline__ int mf_xcd_chunk(int nchunks)
