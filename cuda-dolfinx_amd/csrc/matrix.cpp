@@ -365,9 +365,9 @@ std::shared_ptr<OwnerPlan> vector_plan(mf_form* L, Integral& I) {
 // The blocks cost a cleared vector (2.3 us of launch) and their atomics; the
 // other repeats cells, which weighs what the body weighs, and the registers it
 // needs tell light from heavy bodies.  Cell integral in us, rows / blocks:
-//   under 100 registers: P1 196 thousand cells 7.7 / 8.7, 750 thousand 19.3 /
-//     14.0; P2 94 thousand 8.1 / 8.5; vector P2 664 thousand 59 / 51;
-//   P3 source (126): 10 thousand cells 15.0 / 15.1, 83 thousand 24.6 / 21.6;
+//   under 100 registers: P1 196 thousand cells 8.2 / 9.2, 750 thousand 19.0 /
+//     14.1; P2 94 thousand 7.5 / 9.1; vector P2 664 thousand 59 / 51;
+//   P3 source (104): 10 thousand cells 12.2 / 9.0, 83 thousand 23.3 / 13.9;
 //   P2 residual with 64 points (242): 1 thousand 37 / 43, 10 thousand 61 / 41,
 //     48 thousand 97 / 48; P1 with 27 points: 3 thousand 17 / 9.
 // Cells of more than 32 nodes have no row-owning kernel: Q3 source on 14
@@ -381,7 +381,7 @@ static bool blocks_pay(const mf_form& L, Integral& I) {
     MF_HIP(hipFuncGetAttribute(&regs, HIP_FUNC_ATTRIBUTE_NUM_REGS, I.k_vown));
     I.vown_regs = std::max(1, regs);
   }
-  return I.n >= (I.vown_regs < 100 ? 400000 : I.vown_regs < 160 ? 64000 : 2500);
+  return I.n >= (I.vown_regs < 100 ? 400000 : I.vown_regs < 160 ? 8000 : 2500);
 }
 
 // Blocks of at most 256 entities (down to 64 where that leaves fewer than

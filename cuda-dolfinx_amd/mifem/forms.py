@@ -396,27 +396,27 @@ def source(V: FunctionSpace, f, qdegree: Optional[int] = None) -> Form:
         raise TypeError("f must be a Constant or Function")
     q = E.tet_rule(qd)
     phi = el.tabulate(q.points, 0)[0]                              # (nq, nd)
-    parts = [_carr("FE_w", q.weights), _carr("FE_phi", phi)]
+    # |det J| is the same at every point of an affine cell, so the quadrature sums
+    # over the reference cell are taken here: b_i = |det J| sum_k M_ik w_k with
+    # M_ik = sum_q w_q phi_i psi_k (64 points at P3: 400 multiply-adds, not 2,560)
+    uid = _uid("source", el, bs, q.points.tobytes(), mode,
+               f.function_space.element if mode == "func" else "", "sums")
+    name = f"tabulate_tensor_integral_{uid}"
     if mode == "func":
-        fel = f.function_space.element
-        nf = fel.ndofs
-        parts.append(_carr("FE_psi", fel.tabulate(q.points, 0)[0]))
-        fval = f"""    double fv[{bs}] = {{0}};
-    for (int k = 0; k < {nf}; ++k)
-      for (int a = 0; a < {bs}; ++a) fv[a] += FE_psi[iq][k] * w[k * {bs} + a];
+        psi = f.function_space.element.tabulate(q.points, 0)[0]
+        nf = psi.shape[1]
+        body = _carr("FE_M", np.einsum("q,qi,qk->ik", q.weights, phi, psi)) + _AFFINE_GEOM + f"""
+  for (int i = 0; i < {nd}; ++i)
+    for (int a = 0; a < {bs}; ++a) {{
+      double s = 0.0;
+      for (int k = 0; k < {nf}; ++k) s += FE_M[i][k] * w[k * {bs} + a];
+      A[i * {bs} + a] += adet * s;
+    }}
 """
     else:
-        fval = f"    double fv[{bs}];\n    for (int a = 0; a < {bs}; ++a) fv[a] = c[a];\n"
-    uid = _uid("source", el, bs, q.points.tobytes(), mode,
-               f.function_space.element if mode == "func" else "")
-    name = f"tabulate_tensor_integral_{uid}"
-    body = "".join(parts) + _AFFINE_GEOM + f"""
-  for (int iq = 0; iq < {q.weights.size}; ++iq) {{
-{fval}    const double fw = FE_w[iq] * adet;
-    for (int i = 0; i < {nd}; ++i)
-      for (int a = 0; a < {bs}; ++a)
-        A[i * {bs} + a] += fw * FE_phi[iq][i] * fv[a];
-  }}
+        body = _carr("FE_M", q.weights @ phi) + _AFFINE_GEOM + f"""
+  for (int i = 0; i < {nd}; ++i)
+    for (int a = 0; a < {bs}; ++a) A[i * {bs} + a] += adet * FE_M[i] * c[a];
 """
     src = _SIG.format(name=name) + "\n{\n" + body + "}\n"
     cells = np.arange(V.mesh.num_cells, dtype=np.int32)
