@@ -466,29 +466,34 @@ int mf_form_pack_coefficients(mf_form* f, const int* idx, int n, mf_stream s) {
   return guard([&] {
     MF_CHECK(f, MF_EINVAL, "null form");
     use_device(f->ctx);
-    std::vector<int> sel;
-    if (idx) sel.assign(idx, idx + n);
-    else
-      for (int j = 0; j < (int)f->coefs.size(); ++j) sel.push_back(j);
     // values uploaded through mf_form_set_coefficient are packed again only
     // after they change; under graph capture every pack is recorded, since the
     // graph replays after later uploads
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     MF_HIP(hipStreamIsCapturing(S(s), &cap));
     const bool capturing = cap != hipStreamCaptureStatusNone;
-    std::vector<mf::PackItem> items;
-    for (int j : sel) {
+    const int count = idx ? n : static_cast<int>(f->coefs.size());
+    mf::PackItem items[mf::kPackItems];
+    int m = 0;
+    auto flush = [&] {
+      mf::k_pack(f->packed.ptr, f->mesh->num_cells, f->W, items, m, S(s));
+      m = 0;
+    };
+    for (int k = 0; k < count; ++k) {
+      const int j = idx ? idx[k] : k;
       MF_CHECK(j >= 0 && j < (int)f->coefs.size(), MF_EINVAL, "coefficient index out of range");
-      auto& c = f->coefs[j];
-      const double* v = c.ext ? c.ext : c.own.ptr;
-      MF_CHECK(v, MF_ESTATE, "coefficient " + std::to_string(j) + " has no values");
-      if (!c.ext && !c.dirty && !capturing) continue;
-      items.push_back({v, c.dm->dev.ptr, c.dm->nd, c.dm->bs, c.offset});
+      MF_CHECK(f->coefs[j].ext || f->coefs[j].own.ptr, MF_ESTATE,
+               "coefficient " + std::to_string(j) + " has no values");
     }
-    mf::k_pack(f->packed.ptr, f->mesh->num_cells, f->W, items.data(), static_cast<int>(items.size()),
-               S(s));
-    if (!capturing)
-      for (int j : sel) f->coefs[j].dirty &= f->coefs[j].ext != nullptr;
+    for (int k = 0; k < count; ++k) {
+      auto& c = f->coefs[idx ? idx[k] : k];
+      const double* v = c.ext ? c.ext : c.own.ptr;
+      if (!c.ext && !c.dirty && !capturing) continue;
+      items[m++] = {v, c.dm->dev.ptr, c.dm->nd, c.dm->bs, c.offset};
+      if (m == mf::kPackItems) flush();
+      if (!c.ext && !capturing) c.dirty = false;
+    }
+    flush();
   });
 }
 

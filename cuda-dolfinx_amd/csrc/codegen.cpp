@@ -362,7 +362,8 @@ bool staged_fullrt(const Integral& I) {
 }
 
 bool staged_trace(const Integral& I) {
-  return I.staged_src.find("#define SK_TRACE ") != std::string::npos;
+  if (I.trace < 0) I.trace = I.staged_src.find("#define SK_TRACE ") != std::string::npos;
+  return I.trace > 0;
 }
 
 bool is_hex_staged(const Integral& I) {

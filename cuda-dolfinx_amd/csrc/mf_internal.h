@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <atomic>
 #include <map>
 #include <memory>
 #include <stdexcept>
@@ -139,6 +140,7 @@ void k_node_bits(uint8_t* bits, const int8_t* markers, int64_t nnodes, int bs, h
 // flags[c] = 1 if any node of cell c (dofmap dm, nd nodes per cell) has bits
 void k_cell_flags(uint8_t* flags, const int32_t* dm, int64_t ncells, int nd, const uint8_t* bits,
                   hipStream_t s);
+constexpr int kPackItems = 8;         // coefficients of one launch
 struct PackItem {                      // one coefficient of a form
   const double* values;
   const int32_t* dofmap;
@@ -254,6 +256,7 @@ struct LiftList {
 struct Integral {
   int type = 0, id = -1;
   std::string tab_name, tab_src, staged_src;
+  mutable std::atomic<int8_t> trace{-1};   // staged_trace (-1: not looked up)
   std::vector<int32_t> h_ents;
   DevArray<int32_t> d_ents;
   int64_t n = 0;
@@ -333,7 +336,7 @@ struct mf_form {
   bool compiled = false;
   std::unique_ptr<mf::Module> mod;
   std::string source;
-  std::map<std::string, int64_t> options;
+  std::map<std::string, int64_t, std::less<>> options;
   bool shape_default = false;         // chunk_values and owner_pairs are the library's choice
   std::map<int, std::shared_ptr<mf::OwnerPlan>> vplans;   // owner-computes vector schedules
   std::map<int, std::unique_ptr<mf::VectorBlocks>> vblocks;   // blocks of cell integrals
@@ -352,7 +355,7 @@ struct mf_form {
   mf::DevArray<double> scalar_out;    // rank 0: device result of the host-returning entry
   uint64_t uid = 0;
   uint64_t gen = 0;                   // compile generation (bumped by every compile)
-  int64_t opt(const std::string& k, int64_t dflt) const {
+  int64_t opt(const char* k, int64_t dflt) const {   // (looked up without making a string)
     auto it = options.find(k);
     return it == options.end() ? dflt : it->second;
   }

@@ -113,15 +113,16 @@ __global__ void node_bits_kernel(uint8_t* __restrict__ bits, const int8_t* __res
 // number of coefficients, selected by compares; I: 32-bit indices where they do.
 // Bound by launches at these sizes (4 to 7 us each): two P2 coefficients on 48
 // thousand cells 10.6 -> 5.4 us.
-constexpr int kPack = 8;
+constexpr int kPack = kPackItems;
+template <int N>
 struct PackArgs {
-  const double* values[kPack];
-  const int32_t* dofmap[kPack];
-  int32_t nd[kPack], bs[kPack], off[kPack], cum[kPack + 1];
+  const double* values[N];
+  const int32_t* dofmap[N];
+  int32_t nd[N], bs[N], off[N], cum[N + 1];
 };
 
 template <int N, class I>
-__global__ void pack_kernel(double* __restrict__ packed, int64_t ncells, int W, const PackArgs a) {
+__global__ void pack_kernel(double* __restrict__ packed, int64_t ncells, int W, const PackArgs<N> a) {
   const I width = a.cum[N], total = static_cast<I>(ncells) * width;
   const I stride = static_cast<I>(gridDim.x) * blockDim.x;
   for (I l = static_cast<I>(blockIdx.x) * blockDim.x + threadIdx.x; l < total; l += stride) {
@@ -580,37 +581,37 @@ void k_node_bits(uint8_t* bits, const int8_t* m, int64_t nnodes, int bs, hipStre
   node_bits_kernel<<<grid_for(nnodes), kBlock, 0, s>>>(bits, m, nnodes, bs);
   MF_HIP(hipGetLastError());
 }
-template <class I>
-static void pack_launch(double* packed, int64_t ncells, int W, const PackArgs& a, int n, hipStream_t s) {
-  const int grid = grid_for(ncells * a.cum[n]);
-  switch (n) {
-    case 1: pack_kernel<1, I><<<grid, kBlock, 0, s>>>(packed, ncells, W, a); break;
-    case 2: pack_kernel<2, I><<<grid, kBlock, 0, s>>>(packed, ncells, W, a); break;
-    case 3: pack_kernel<3, I><<<grid, kBlock, 0, s>>>(packed, ncells, W, a); break;
-    case 4: pack_kernel<4, I><<<grid, kBlock, 0, s>>>(packed, ncells, W, a); break;
-    default: pack_kernel<kPack, I><<<grid, kBlock, 0, s>>>(packed, ncells, W, a);
+// N: room for coefficients, m of them given
+template <int N>
+static void pack_launch(double* packed, int64_t ncells, int W, const PackItem* items, int m, hipStream_t s) {
+  PackArgs<N> a;
+  a.cum[0] = 0;
+  for (int g = 0; g < N; ++g) {
+    const PackItem q = g < m ? items[g] : PackItem{nullptr, nullptr, 0, 1, 0};
+    a.values[g] = q.values;
+    a.dofmap[g] = q.dofmap;
+    a.nd[g] = q.nd;
+    a.bs[g] = q.bs;
+    a.off[g] = q.off;
+    a.cum[g + 1] = a.cum[g] + q.nd * q.bs;
   }
+  const int64_t total = ncells * a.cum[N];
+  // (a thread's index past the last entry stays below total + the grid's threads)
+  if (total < (int64_t(1) << 31)) pack_kernel<N, uint32_t><<<grid_for(total), kBlock, 0, s>>>(packed, ncells, W, a);
+  else pack_kernel<N, int64_t><<<grid_for(total), kBlock, 0, s>>>(packed, ncells, W, a);
+  MF_HIP(hipGetLastError());
 }
 void k_pack(double* packed, int64_t ncells, int W, const PackItem* items, int n, hipStream_t s) {
   if (ncells <= 0) return;
   for (int i0 = 0; i0 < n; i0 += kPack) {
     const int m = std::min(n - i0, kPack);
-    PackArgs a{};
-    for (int g = 0; g < kPack; ++g) {
-      if (g < m) {
-        const PackItem& q = items[i0 + g];
-        a.values[g] = q.values;
-        a.dofmap[g] = q.dofmap;
-        a.nd[g] = q.nd;
-        a.bs[g] = q.bs;
-        a.off[g] = q.off;
-      }
-      a.cum[g + 1] = a.cum[g] + (g < m ? a.nd[g] * a.bs[g] : 0);
+    switch (m) {
+      case 1: pack_launch<1>(packed, ncells, W, items + i0, m, s); break;
+      case 2: pack_launch<2>(packed, ncells, W, items + i0, m, s); break;
+      case 3: pack_launch<3>(packed, ncells, W, items + i0, m, s); break;
+      case 4: pack_launch<4>(packed, ncells, W, items + i0, m, s); break;
+      default: pack_launch<kPack>(packed, ncells, W, items + i0, m, s);
     }
-    // the last of a thread's entries is below total + the grid's threads
-    if (ncells * a.cum[m] < (int64_t(1) << 31)) pack_launch<uint32_t>(packed, ncells, W, a, m, s);
-    else pack_launch<int64_t>(packed, ncells, W, a, m, s);
-    MF_HIP(hipGetLastError());
   }
 }
 void k_set_bc_batch(const SetBcGroup* groups, int ngroups, double scale, hipStream_t s) {

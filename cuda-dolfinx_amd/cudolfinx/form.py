@@ -198,6 +198,8 @@ class CUDAForm:
                 check(lib().mf_form_set_coefficient(self._handle, j, x.ctypes.data_as(C.c_void_p),
                                                     x.size, 0))
                 self._coef_versions[j] = f.version
+        if not force and not self._form.constants and self._consts is not None and not self._consts.size:
+            return                            # nothing to compare (2 us of numpy calls)
         c = np.ascontiguousarray(self._form.constant_values(), dtype=np.float64)
         if force or self._consts is None or not np.array_equal(c, self._consts):
             check(lib().mf_form_set_constants(self._handle,
