@@ -24,13 +24,13 @@ from pathlib import Path
 from .form import CUDAForm
 
 DEFAULT_CANDIDATES = [
+    {"chunk_values": 4608, "owner_pairs": 160, "owner_block": 256},
     {"chunk_values": 4096, "owner_pairs": 256, "owner_block": 256},
     {"chunk_values": 4096, "owner_pairs": 256, "owner_block": 256, "owner_wpe": 4},
     {"chunk_values": 4096, "owner_pairs": 384, "owner_block": 256},
     {"chunk_values": 4608, "owner_pairs": 384, "owner_block": 256, "owner_lds": 73728},
     {"chunk_values": 5120, "owner_pairs": 384, "owner_block": 256, "owner_lds": 81920},
     {"chunk_values": 3072, "owner_pairs": 256, "owner_block": 256},
-    {"chunk_values": 6144, "owner_pairs": 512, "owner_block": 256, "owner_lds": 98304},
     # warp-specialised variant: three compute waves and one store wave,
     # double-buffered accumulators
     {"chunk_values": 2304, "owner_pairs": 192, "owner_pipe": 1, "owner_cwaves": 3,
@@ -41,7 +41,8 @@ DEFAULT_CANDIDATES = [
 # (nd x nd x 6) table shares LDS with the accumulator
 TRACE_CANDIDATES = [
     {"chunk_values": 2048, "owner_pairs": 384, "owner_block": 256},
-    {"chunk_values": 1536, "owner_pairs": 384, "owner_block": 256},
+    {"chunk_values": 2048, "owner_pairs": 256, "owner_block": 256},
+    {"chunk_values": 3040, "owner_pairs": 256, "owner_block": 256},
     {"chunk_values": 3072, "owner_pairs": 384, "owner_block": 256, "owner_lds": 98304},
     {"chunk_values": 2048, "owner_pairs": 256, "owner_block": 128},
     {"chunk_values": 2048, "owner_pairs": 384, "owner_pipe": 1, "owner_cwaves": 3,
@@ -187,10 +188,10 @@ def autotune_matrix_native(a, asm, A, bcs=(), reps: int = 5):
 # member shapes of a CUDABatch: value chunk (rows per workgroup) and pairs
 # per chunk; the batch kernel's threads per workgroup are shared by all members
 BATCH_CANDIDATES = [
+    {"chunk_values": 2048, "owner_pairs": 256},
+    {"chunk_values": 3040, "owner_pairs": 256},
     {"chunk_values": 2048, "owner_pairs": 384},
-    {"chunk_values": 1536, "owner_pairs": 256},
     {"chunk_values": 3072, "owner_pairs": 384, "owner_lds": 98304},
-    {"chunk_values": 4096, "owner_pairs": 384, "owner_lds": 98304},
 ]
 
 
