@@ -20,7 +20,8 @@
 // (same tiles and pair packing; on MI355X the FP64 vector and matrix peaks
 // are equal, 78.6 TFLOP/s, so FP64 matrix cores offer no higher ceiling, and
 // the vector ALUs can contract over x, y and z in turn, 4.6 times fewer
-// multiply-adds than the dense contraction: Q3 on 24^3 cubes 1,215 -> 435 us).
+// multiply-adds than the dense contraction: Q3 on 24^3 cubes 1,215 -> 435 us,
+// 370 with what the kernel's comment below names).
 // Geometry (J, det, K), D_q, and the CSR accumulation are FP64 in all three.
 //
 // Operand layouts (16x16xK, lane l): A[row l%16][k-slot l/16], B[k-slot
@@ -352,9 +353,10 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
   // the next chunk) reads from memory is loaded into registers while this one
   // computes, its dependent loads issued a phase apart, and the accumulator is
   // cleared by the write-out.  24^3 cells, 47 M values, 0.38 GB: 370 us (FP64),
-  // 510 us (FP32) against 390 and 520 us with one workgroup per chunk, and 436
-  // and 518 us when the coordinates and dofs came from 464-byte cell records,
-  // rows were searched in chunks and chunks were filled up.  What is left is the
+  // 510 us (FP32; 470 with chunks that end at full rounds of tiles) against 390
+  // and 520 us with one workgroup per chunk, and 436 and 518 us when the
+  // coordinates and dofs came from 464-byte cell records, rows were searched in
+  // chunks and chunks were filled up.  What is left is the
   // arithmetic of the 4-5 tiles of a chunk (FP64 about 140 us of issue, FP32
   // 190 us of MFMA) and the geometry in two workgroups' phases per CU.
   constexpr int NTH = $HBLOCK;
