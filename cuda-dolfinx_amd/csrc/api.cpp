@@ -1154,7 +1154,7 @@ int mf_autotune_matrix(mf_form* a, mf_matrix* A, const mf_bc* bc, int reps, mf_s
         {{"chunk_values", 4096}, {"owner_pairs", 384}, {"owner_block", 256}},
         {{"chunk_values", 5120}, {"owner_pairs", 384}, {"owner_block", 256}, {"owner_lds", 81920}},
         {{"chunk_values", 3072}, {"owner_pairs", 256}, {"owner_block", 256}},
-        {{"chunk_values", 4608}, {"owner_pairs", 160}, {"owner_block", 256}},
+        {{"chunk_values", 4640}, {"owner_pairs", 128}, {"owner_block", 256}},
         {{"chunk_values", 2048}, {"owner_pairs", 256}, {"owner_block", 256}},
         {{"chunk_values", 4608}, {"owner_pairs", 384}, {"owner_block", 256}, {"owner_lds", 73728}},
     };

@@ -943,9 +943,10 @@ std::string compile_source(mf_form& f) {
   // nd x nd x 6 table in LDS: 2048 values, and for P3 3040, which its 64 rows
   // fill (four workgroups per CU in FP32); 256 pairs at P2 and P3, one per thread (P2 25^3 33.6 us at 384, 32.6 at
   // 256; P3 24^3 83 us at 2048 / 384, 75 at 3040 / 256), 384 at P1, whose rows
-  // have 24 each.  Vector forms 4608 values (the fastest of the tuned shapes at
-  // vector P2) and 160 pairs, at which four workgroups share a CU (48^3: 757 us at
-  // 384, 742 at 160).  Fewer pairs than a node has cells would send the form to
+  // have 24 each.  Vector forms 4640 values and 128 pairs, two full groups
+  // of lanes, at which four workgroups share a CU (vector P2 48^3: 4608 values and
+  // 384 pairs 757 us, 160 pairs 742; with the pairs dealt by bank 160 pairs 606,
+  // 4640 values and 128 pairs 597; 13^3 24.3 and 22.7 us).  Fewer pairs than a node has cells would send the form to
   // another kernel, so then it is 384.  Hexahedra 4096.
   bool trace = false, hex = false;
   for (auto& I : f.ints) {
@@ -958,7 +959,7 @@ std::string compile_source(mf_form& f) {
   f.shape_default |= !given;
   const int nd = f.rank == 2 ? f.dm[0]->nd : 0;
   if (f.shape_default && f.rank == 2) {
-    f.options["chunk_values"] = trace ? (nd > 10 ? 3040 : 2048) : (hex ? 4096 : 4608);
+    f.options["chunk_values"] = trace ? (nd > 10 ? 3040 : 2048) : (hex ? 4096 : 4640);
     if (!hex) {
       int most = 0;                                     // cells of a node
       for (auto& I : f.ints) {
@@ -967,7 +968,7 @@ std::string compile_source(mf_form& f) {
         for (int32_t c : I->h_ents)
           for (int i = 0; i < nd; ++i) most = std::max(most, ++cells[f.dm[0]->host[(int64_t)c * nd + i]]);
       }
-      f.options["owner_pairs"] = trace ? (nd > 4 && most <= 256 ? 256 : 384) : (most <= 160 ? 160 : 384);
+      f.options["owner_pairs"] = trace ? (nd > 4 && most <= 256 ? 256 : 384) : (most <= 128 ? 128 : 384);
     }
   }
   const int64_t cap = f.opt("chunk_values", trace ? 2048 : (hex ? 4096 : 4608));

@@ -24,7 +24,7 @@ from pathlib import Path
 from .form import CUDAForm
 
 DEFAULT_CANDIDATES = [
-    {"chunk_values": 4608, "owner_pairs": 160, "owner_block": 256},
+    {"chunk_values": 4640, "owner_pairs": 128, "owner_block": 256},
     {"chunk_values": 4096, "owner_pairs": 256, "owner_block": 256},
     {"chunk_values": 4096, "owner_pairs": 256, "owner_block": 256, "owner_wpe": 4},
     {"chunk_values": 4096, "owner_pairs": 384, "owner_block": 256},

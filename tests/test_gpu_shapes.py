@@ -327,11 +327,11 @@ def test_fused_system_adds_with_dirichlet_rows(n):
         ref = o.assemble_matrix(rp, cols, [bc], diagonal=2.5, values=ref.copy())
 
 
-@pytest.mark.parametrize("which,times", [("vector", 1), ("vector", 7), ("vector", 8), ("vector", 17),
+@pytest.mark.parametrize("which,times", [("vector", 1), ("vector", 5), ("vector", 6), ("vector", 8), ("vector", 17),
                                          (2, 10), (2, 12), (3, 11), (3, 17)])
 def test_matrix_rows_with_many_cells(which, times):
     """Rows around the numbers of (cell, row) pairs at which the owner kernel's shape
-    changes (160 vector, 256 scalar) and past its largest (384): every cell of a cube
+    changes (128 vector, 256 scalar) and past its largest (384): every cell of a cube
     listed several times, so that its inner node has 24 cells as often."""
     import dataclasses
     import cudolfinx as cufem
