@@ -336,7 +336,7 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
   constexpr int DCELL = NQ * DS;
 #define MF_DOFF(b, q) ((b) * DCELL + (q) * DS)
 #endif
-  __shared__ __attribute__((aligned(16))) double acc[CAP];
+  __shared__ __attribute__((aligned(16))) double acc[(CAP + 1) / 2 * 2];
   __shared__ int32_t lrp[MAXR + 1];
   __shared__ double sx[NB * 24];                     // vertex coordinates of the batch's cells
   __shared__ uint64_t smask[NB];                     // their constrained columns
@@ -382,7 +382,7 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
   {
     mf_d2* a2 = reinterpret_cast<mf_d2*>(acc);
     const mf_d2 z = {0.0, 0.0};
-    for (int p = tid; p < CAP / 2; p += nt) a2[p] = z;
+    for (int p = tid; p < (CAP + 1) / 2; p += nt) a2[p] = z;
   }
   // registers of the step ahead: vertices (1), then coordinates and constrained
   // columns (2) of its cells; for a chunk also its pairs and its row (row tid)

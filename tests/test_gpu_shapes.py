@@ -397,3 +397,25 @@ def test_packed_coefficients_of_one_form(n, count):
     b = asm.assemble_vector(form, b)
     asm.synchronize()
     assert _rel(b.to_host(), reference()) <= TOL
+
+
+@pytest.mark.parametrize("prec,tol", [(64, TOL), (32, 1e-6), (16, 2e-2)])
+def test_hexahedral_accumulator_of_odd_length(prec, tol):
+    """chunk_values = 343, which the row of an inner vertex (7^3 columns) fills to
+    the last value, after a kernel that leaves sums in LDS."""
+    import cudolfinx as cufem
+    print(f"[gpu-test] Q3 owner chunks of 343 values, precision={prec}", flush=True)
+    P = problems.helmholtz_q3(4, seed=8)
+    asm = cufem.CUDAAssembler()
+    f = cufem.form(P.a, options={"matrix_kernel": 2, "precision": prec, "chunk_values": 343})
+    A = asm.create_matrix(f)
+    o = cpu.OracleAssembler(P.a)
+    rp, cols, _, _ = o.sparsity()
+    ref = o.assemble_matrix(rp, cols, [])
+    assert np.diff(rp).max() == 343
+    fill = cufem.form(_elasticity(9)[2], options={"vector_kernel": 4})
+    for _ in range(4):
+        asm.assemble_vector(fill)
+        asm.assemble_matrix(f, A)
+        asm.synchronize()
+        assert _rel(A.csr()[2], ref) <= tol
