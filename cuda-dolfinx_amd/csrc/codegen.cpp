@@ -403,7 +403,10 @@ bool hex_source_emitted(const mf_form& f, const Integral& I) {
 // operand paths (more waves to overlap the MFMA chains with the operand
 // loads), 256 for FP64; option hex_block overrides both.
 int hex_block(const mf_form& f, int prec) {
-  return static_cast<int>(f.opt("hex_block", prec == 64 ? 256 : 512));
+  const int64_t n = f.opt("hex_block", prec == 64 ? 256 : 512);
+  MF_CHECK(n >= 64 && n <= 1024 && n % 64 == 0, MF_EINVAL,
+           "hex_block must be whole waves of 64 threads, at most 1024");
+  return static_cast<int>(n);
 }
 
 int hex_batch(const mf_form& f, const Integral& I, int prec) {

@@ -361,7 +361,7 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
   // 190 us of MFMA) and the geometry in two workgroups' phases per CU.
   constexpr int NTH = $HBLOCK;
   constexpr int PFX = (NB * 24 + NTH - 1) / NTH, PFP = (MAXP + NTH - 1) / NTH;
-  static_assert(MAXR < NTH && NB <= NTH, "one row and one cell per thread");
+  constexpr int PFB = (NB + NTH - 1) / NTH, PFR = (MAXR + NTH) / NTH;   // one each unless a caller's shape has more
   const int tid = threadIdx.x, nt = NTH;
   const int lane = tid & 63, wave = tid >> 6, nwave = NTH >> 6;
   const int nx = 8, gx = gridDim.x / nx, per = (nchunks + nx - 1) / nx;
@@ -370,7 +370,7 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
   if (k >= kend) return;
   const int4* meta = reinterpret_cast<const int4*>(chunk_meta);
   int4 m0 = meta[3 * k], m1 = meta[3 * k + 1], m2 = meta[3 * k + 2];
-  if (tid < M1 * K1) {
+  if (tid < M1 * K1) {                                 // 16 of at least 64 threads
 #if MF_HX_PREC == 64
     sTL[tid] = HX_L[tid / K1][tid % K1];
     sTD[tid] = HX_DL[tid / K1][tid % K1];
@@ -385,31 +385,38 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
     for (int p = tid; p < (CAP + 1) / 2; p += nt) a2[p] = z;
   }
   // registers of the step ahead: vertices (1), then coordinates and constrained
-  // columns (2) of its cells; for a chunk also its pairs and its row (row tid)
-  int pfv[PFX], pfc = 0, pfp[PFP], pfr = 0, pfd = -1;
+  // columns (2) of its cells; for a chunk also its pairs and its rows (row tid, ...)
+  int pfv[PFX], pfc[PFB], pfp[PFP], pfr[PFR], pfd[PFR];
   double pfx[PFX];
-  uint64_t pfm = 0;
+  uint64_t pfm[PFB];
   auto fetch1 = [&](const int ib, const int nb, const int tid) {
 #pragma clang loop unroll(full)
     for (int t = 0; t < PFX; ++t)                      // clamped, unconditional loads stay in registers
       pfv[t] = item_geo[(int64_t)ib * 8 + min(tid + t * NTH, max(nb * 24 - 1, 0)) / 3];
-    pfc = item_cell[ib + min(tid, max(nb - 1, 0))];    // (the lists are padded by one cell and pair)
+#pragma clang loop unroll(full)
+    for (int t = 0; t < PFB; ++t)                      // (the lists are padded by one cell and pair)
+      pfc[t] = item_cell[ib + min(tid + t * NTH, max(nb - 1, 0))];
   };
   auto fetch2 = [&](const int nb, const int tid) {
 #pragma clang loop unroll(full)
     for (int t = 0; t < PFX; ++t)
       pfx[t] = xg[3 * (int64_t)pfv[t] + min(tid + t * NTH, max(nb * 24 - 1, 0)) % 3];
-    pfm = cmask ? cmask[pfc] : 0;
+#pragma clang loop unroll(full)
+    for (int t = 0; t < PFB; ++t) pfm[t] = cmask ? cmask[pfc[t]] : 0;
   };
   auto fetch_rows = [&](const int4 c0, const int4 c1, const int4 c2, const int tid) {
 #pragma clang loop unroll(full)
     for (int t = 0; t < PFP; ++t) pfp[t] = pair_list[max(min(c2.x + tid + t * NTH, c2.y - 1), c2.x)];
-    pfr = rpb[min(c0.x + tid, c0.y)] - c1.x;           // rpb[c0.y] closes the last row
-    // Dirichlet rows: position of their diagonal entry (-1: none)
-    const int row = min(c0.x + tid, c0.y - 1);
-    const int dp = diag_pos[row];
-    const bool on = (flags & 2) && nb0 && nb0[row];
-    pfd = on && c0.x + tid < c0.y ? dp : -1;
+#pragma clang loop unroll(full)
+    for (int t = 0; t < PFR; ++t) {
+      const int u = c0.x + tid + t * NTH;
+      pfr[t] = rpb[min(u, c0.y)] - c1.x;               // rpb[c0.y] closes the last row
+      // Dirichlet rows: position of their diagonal entry (-1: none)
+      const int row = min(u, c0.y - 1);
+      const int dp = diag_pos[row];
+      const bool on = (flags & 2) && nb0 && nb0[row];
+      pfd[t] = on && u < c0.y ? dp : -1;
+    }
   };
   auto store_cells = [&](const int nb) {
 #pragma clang loop unroll(full)
@@ -417,7 +424,9 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
       const int u = tid + t * NTH;
       if (u < nb * 24) sx[u] = pfx[t];
     }
-    if (tid < nb) smask[tid] = pfm;
+#pragma clang loop unroll(full)
+    for (int t = 0; t < PFB; ++t)
+      if (tid + t * NTH < nb) smask[tid + t * NTH] = pfm[t];
   };
   auto store_rows = [&](const int4 c0, const int4 c2) {
 #pragma clang loop unroll(full)
@@ -425,10 +434,14 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
       const int u = tid + t * NTH;
       if (u < c2.y - c2.x) spair[u] = pfp[t];
     }
-    if (tid <= c0.y - c0.x) lrp[tid] = pfr;
-    // constrained rows get no contributions (their pairs are masked), so their
-    // diagonal is set up front
-    if (pfd >= 0) acc[pfr + pfd] = diag;
+#pragma clang loop unroll(full)
+    for (int t = 0; t < PFR; ++t) {
+      const int u = tid + t * NTH;
+      if (u <= c0.y - c0.x) lrp[u] = pfr[t];
+      // constrained rows get no contributions (their pairs are masked), so their
+      // diagonal is set up front
+      if (pfd[t] >= 0) acc[pfr[t] + pfd[t]] = diag;
+    }
   };
   fetch1(m0.z, min(NB, m0.w - m0.z), tid);
   fetch_rows(m0, m1, m2, tid);

@@ -419,3 +419,27 @@ def test_hexahedral_accumulator_of_odd_length(prec, tol):
         asm.assemble_matrix(f, A)
         asm.synchronize()
         assert _rel(A.csr()[2], ref) <= tol
+
+
+@pytest.mark.parametrize("options", [{"hex_block": 64}, {"chunk_rows": 256}, {"chunk_rows": 1500, "chunk_values": 6000},
+                                     {"hex_block": 64, "owner_nb": 70, "owner_lds": 160000}])
+@pytest.mark.parametrize("prec,tol", [(64, TOL), (32, 1e-6)])
+def test_hexahedral_chunks_of_more_rows_than_threads(options, prec, tol):
+    """Workgroups of fewer threads than a chunk has rows or a batch has cells,
+    over a subdomain (rows without cells fill chunks with hundreds of rows)."""
+    import dataclasses
+    import cudolfinx as cufem
+    print(f"[gpu-test] Q3 owner chunks {options} precision={prec}", flush=True)
+    P = problems.helmholtz_q3(5, seed=8)
+    I = P.a.integrals[0]
+    a = dataclasses.replace(P.a, integrals=[dataclasses.replace(I, entities=np.arange(0, 125, 3, dtype=np.int32))])
+    bc = _some_dofs(P.V, 0.1, 3)
+    asm = cufem.CUDAAssembler()
+    f = cufem.form(a, options={"matrix_kernel": 2, "precision": prec, **options})
+    A = asm.assemble_matrix(f, bcs=[bc], diagonal=1.5)
+    asm.synchronize()
+    o = cpu.OracleAssembler(a)
+    rp, cols, _, _ = o.sparsity()
+    ref = o.assemble_matrix(rp, cols, [bc], diagonal=1.5)
+    scale = np.linalg.norm(o.assemble_matrix(rp, cols, []))
+    assert np.linalg.norm(A.csr()[2] - ref) <= tol * max(scale, np.linalg.norm(ref))

@@ -1,0 +1,55 @@
+"""Kernel shape options without a GPU: every shape that the library accepts
+compiles for gfx950 within the 160 KB of LDS, and the rest is refused with a
+message of the library's, not the compiler's."""
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from mifem import problems
+from test_codegen_cpu import _READELF, _describe, _kernels
+
+ROOT = Path(__file__).resolve().parent.parent
+
+
+@pytest.fixture(scope="module")
+def driver(tmp_path_factory):
+    build = ROOT / "cuda-dolfinx_amd" / "_build"
+    objs = [build / f"{n}.o" for n in ("codegen", "runtime", "owner_kernel", "hex_kernel",
+                                       "dg_kernel", "sparsity", "util_kernels", "matrix")]
+    if not shutil.which("hipcc") or not _READELF.exists() or not all(o.exists() for o in objs):
+        pytest.skip("hipcc / llvm-readelf / library objects not available")
+    d = tmp_path_factory.mktemp("shapes")
+    subprocess.run(["hipcc", "-c", "--offload-arch=gfx950", "-fPIC", "-std=c++17", "-O1",
+                    f"-I{ROOT / 'cuda-dolfinx_amd' / 'csrc'}", f"-I{ROOT / 'include'}",
+                    str(ROOT / "tests" / "shape_check.cpp"), "-o", str(d / "check.o")], check=True)
+    subprocess.run(["hipcc", str(d / "check.o"), *map(str, objs), "-lhiprtc", "-o", str(d / "check")],
+                   check=True)
+
+    def run(form, **options):
+        """(kernels of the code object or None, message)"""
+        _describe(form, d / "form.txt")
+        r = subprocess.run([str(d / "check"), str(d / "form.txt"), str(d / "form.co"),
+                            *[f"{k}={v}" for k, v in options.items()]],
+                           stdout=subprocess.PIPE, stderr=subprocess.DEVNULL, text=True, timeout=300)
+        return (_kernels(d / "form.co") if r.stdout.startswith("OK") else None), r.stdout
+
+    return run
+
+
+@pytest.mark.parametrize("options", [
+    {}, {"hex_block": 64}, {"chunk_rows": 255}, {"chunk_rows": 256}, {"chunk_rows": 600, "hex_block": 512},
+    {"chunk_rows": 2000}, {"hex_block": 64, "owner_nb": 70, "owner_lds": 160000},
+    {"chunk_values": 343}, {"hex_block": 1024}])
+def test_hexahedral_shapes_compile(driver, options):
+    K, msg = driver(problems.helmholtz_q3(2).a, **options)
+    assert K is not None, msg[:2000]
+    for k in ("mf_howner64_cell_0", "mf_howner32_cell_0", "mf_howner16_cell_0"):
+        assert K[k][2] <= 160 * 1024
+
+
+@pytest.mark.parametrize("block", [0, 32, 100, 1088])
+def test_hexahedral_block_of_whole_waves(driver, block):
+    K, msg = driver(problems.helmholtz_q3(2).a, hex_block=block)
+    assert K is None and "hex_block" in msg and "error:" not in msg
