@@ -685,6 +685,7 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
   for (int p = tid; p < rows * BS; p += NT) sacc[p] = 0.0;
 #ifdef SK_TRACE
   __shared__ double sv[ND * 64];                       // values to lift: [column][cell]
+  __shared__ bool son[ND * 64];                        // constrained columns
   const int li = blockIdx.x * 64 + (tid & 63);
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool live = li < nl;
@@ -696,24 +697,32 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
 #endif
   const int64_t c = live ? ents[list[li]] : 0;
   const uint64_t mask = live && slot ? lmask[li] : 0;
-  // 0 at unconstrained columns
-  auto value = [&](const int k, const int64_t col) -> double {
-    const bool on = slot ? (mask >> (k & 63)) & 1 : bc1[col] != 0;
-    return on ? scale * (g[col] - (x0 ? x0[col] : 0.0)) : 0.0;
-  };
+  // A column takes part by being constrained, not by its value: a zero times a
+  // tensor that is not finite is not a zero.
+  auto on = [&](const int k, const int64_t col) { return live && (slot ? (mask >> (k & 63)) & 1 : bc1[col] != 0); };
+  auto value = [&](const int64_t col) { return scale * (g[col] - (x0 ? x0[col] : 0.0)); };
 #ifdef SK_TRACE
 #pragma unroll
   for (int j0 = 0; j0 < ND; j0 += 4) {
     const int j = j0 + wave;
-    if (j < ND) sv[j * 64 + (tid & 63)] = live ? value(j, dm1[c * ND + j]) : 0.0;
+    if (j >= ND) continue;
+    const int64_t col = dm1[c * ND + j];
+    const bool o = on(j, col);
+    son[j * 64 + (tid & 63)] = o;
+    sv[j * 64 + (tid & 63)] = o ? value(col) : 0.0;
   }
 #else
   double v[ND * BS];
+  uint64_t non[(ND + 63) / 64] = {};                   // nodes with a constrained component
 #pragma unroll
   for (int j = 0; j < ND; ++j) {
     const int64_t n1 = dm1[c * ND + j];
 #pragma unroll
-    for (int bb = 0; bb < BS; ++bb) v[j * BS + bb] = live ? value(j * BS + bb, BS * n1 + bb) : 0.0;
+    for (int bb = 0; bb < BS; ++bb) {
+      const bool o = on(j * BS + bb, BS * n1 + bb);
+      non[j / 64] |= (uint64_t)o << (j % 64);
+      v[j * BS + bb] = o ? value(BS * n1 + bb) : 0.0;
+    }
   }
 #endif
   double x[NV][3];
@@ -747,7 +756,8 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
   __syncthreads();                                     // sv and sacc written
   for (int j = 0; j < ND; ++j) {
     const double vj = sv[j * 64 + (tid & 63)];
-    if (!__any(vj != 0.0)) continue;
+    const bool o = son[j * 64 + (tid & 63)];
+    if (!__any(o)) continue;
 #pragma unroll
     for (int r = 0; r < RI; ++r) {
       const int i = min(wave * RI + r, ND - 1);
@@ -757,7 +767,7 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
       G[0] = M00 * R[0] + M11 * R[1] + M22 * R[2] + M01 * R[3] + M02 * R[4] + M12 * R[5];
       double blk[1];
       sk_combine(G, w, consts, blk);
-      if (vj != 0.0) be[r] -= blk[0] * vj;
+      if (o) be[r] -= blk[0] * vj;
     }
   }
 #pragma unroll
@@ -776,9 +786,7 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
   for (int a = 0; a < BS; ++a) be[a] = 0.0;
 #pragma unroll
   for (int j = 0; j < ND; ++j) {
-    bool any = false;
-    for (int bb = 0; bb < BS; ++bb) any |= v[j * BS + bb] != 0.0;
-    if (!any) continue;
+    if (!((non[j / 64] >> (j % 64)) & 1)) continue;
     double G[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     for (int q = 0; q < NQ; ++q) {
       double gj[3];

@@ -443,3 +443,43 @@ def test_hexahedral_chunks_of_more_rows_than_threads(options, prec, tol):
     ref = o.assemble_matrix(rp, cols, [bc], diagonal=1.5)
     scale = np.linalg.norm(o.assemble_matrix(rp, cols, []))
     assert np.linalg.norm(A.csr()[2] - ref) <= tol * max(scale, np.linalg.norm(ref))
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("form", [(1,), (2,), (3,), ()])
+def test_lifting_of_zero_values_keeps_nan(form, noalloc):
+    """A constrained value of zero lifts the NaN of a cell's tensor, as any other
+    value does (only one constrained dof, in another cell, is not zero)."""
+    import ctypes as C
+    import cudolfinx as cufem
+    from cudolfinx import _lib
+    print(f"[gpu-test] NaN coefficient under lifting: {'P%d' % form if form else 'vector P2'} "
+          f"noalloc={noalloc}", flush=True)
+    V, a, L = _poisson(4, *form) if form else _elasticity(4)
+    a.coefficients[0].x[7] = np.nan
+    cells = V.dofmap
+    bs = V.bs
+    dofs = np.unique(np.concatenate([bs * cells[7][:2], bs * cells[-1][-2:]])).astype(np.int32)
+    far = int(bs * cells[-1][-1])
+    assert far // bs not in cells[7]
+    g = np.zeros(V.size)
+    g[far] = 1.0
+    bc = DirichletBC(V, dofs, g)
+    af, Lf = cufem.form(a), cufem.form(L)
+    asm = cufem.CUDAAssembler()
+    dbc = asm.pack_bcs([bc])
+    b = asm.create_vector(Lf)
+    asm.pack_coefficients(af)
+    if noalloc:
+        _lib.check(_lib.lib().mf_apply_lifting_noalloc(
+            (C.c_void_p * 1)(af.handle.value), 1, b.ptr, b.size,
+            (C.c_void_p * 1)(dbc._get_cpp_bcs(V).handle.value), None, 1.0, None))
+    else:
+        asm.apply_lifting(b, [af], [dbc])
+    asm.synchronize()
+    got, ref = b.to_host(), np.zeros(V.size)
+    cpu.OracleAssembler(a).apply_lifting(ref, [bc])
+    nan = np.isnan(ref)
+    assert nan.any() and not nan.all()
+    assert np.array_equal(np.isnan(got), nan)
+    assert _rel(got[~nan], ref[~nan]) <= TOL
