@@ -646,7 +646,9 @@ $VK
 // scalar columns come as a mask (lmask), so all its values load at once
 // instead of node, marker and value one after the other per column.  Without
 // slots (null: the list was built on the device, length *nlist_dev) every
-// column's marker is read and each row goes straight to memory.
+// column's marker is read, each row goes straight to memory, and workgroups
+// past the list's end, most of them where only a boundary is constrained, leave
+// at once (P1 on 50^3: 73 -> 60 us with the list).
 //
 // Forms with a reference tensor: a workgroup takes 64 listed cells, lane = cell,
 // and each of its four waves a quarter of the local rows, so the tensor entries
@@ -655,7 +657,8 @@ $VK
 // (one thread per (cell, row), sorted by row, was 27 us: it gathers every
 // cell's geometry 20 times); P1 on 50^3: 18 -> 8 us.
 // Other forms: one thread per (cell, local row), sorted by row (pairs), 128 to
-// a workgroup.  Vector P2, one face of 48^3 cubes: 32 -> 19 us.
+// a workgroup.  Vector P2, one face of 8^3 and 20^3 cubes: 11.3 -> 7.5 and 28 ->
+// 10.5 us.
 const char* kStagedLiftTemplate = R"(
 #ifdef SK_TRACE
 #define MF_LIFT_BLOCK 256
@@ -680,6 +683,11 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
   // device in the same stream (the grid then covers the largest possible list)
   const int nl = nlist_dev ? *nlist_dev : nlist;
   const int tid = threadIdx.x;
+#ifdef SK_TRACE
+  if ((int)blockIdx.x * 64 >= nl) return;              // whole workgroups past the list
+#else
+  if ((int)blockIdx.x * NT >= nl * ND) return;
+#endif
   __shared__ double sacc[MF_LIFT_ROWS * BS];
   const int rows = slot ? blk_ptr[blockIdx.x + 1] - blk_ptr[blockIdx.x] : 0;
   for (int p = tid; p < rows * BS; p += NT) sacc[p] = 0.0;
@@ -697,39 +705,53 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
 #endif
   const int64_t c = live ? ents[list[li]] : 0;
   const uint64_t mask = live && slot ? lmask[li] : 0;
+  // The chains cell -> vertices -> coordinates and cell -> nodes -> markers and
+  // values run side by side, and no load waits for a branch on a marker.
   // A column takes part by being constrained, not by its value: a zero times a
   // tensor that is not finite is not a zero.
-  auto on = [&](const int k, const int64_t col) { return live && (slot ? (mask >> (k & 63)) & 1 : bc1[col] != 0); };
-  auto value = [&](const int64_t col) { return scale * (g[col] - (x0 ? x0[col] : 0.0)); };
+#ifdef SK_TRACE
+  constexpr int RI = (ND + 3) / 4;                     // columns, then rows, per wave
+#define MF_LIFT_COLS RI
+#define MF_LIFT_COL(t) min(4 * (t) + wave, ND - 1)
+#else
+#define MF_LIFT_COLS ND
+#define MF_LIFT_COL(t) (t)
+#endif
+  int32_t gv[NV], n1[MF_LIFT_COLS];
+#pragma unroll
+  for (int v_ = 0; v_ < NV; ++v_) gv[v_] = geo[c * NV + v_];
+#pragma unroll
+  for (int t_ = 0; t_ < MF_LIFT_COLS; ++t_) n1[t_] = dm1[c * ND + MF_LIFT_COL(t_)];
+  double x[NV][3];
+#pragma unroll
+  for (int v_ = 0; v_ < NV; ++v_) {
+    x[v_][0] = xg[3 * (int64_t)gv[v_]]; x[v_][1] = xg[3 * (int64_t)gv[v_] + 1]; x[v_][2] = xg[3 * (int64_t)gv[v_] + 2];
+  }
+  double v[MF_LIFT_COLS * BS];
+  bool on[MF_LIFT_COLS * BS];
+  if (slot) {
+#pragma unroll
+    for (int k = 0; k < MF_LIFT_COLS * BS; ++k) on[k] = (mask >> ((MF_LIFT_COL(k / BS) * BS + k % BS) & 63)) & 1;
+  } else {
+#pragma unroll
+    for (int k = 0; k < MF_LIFT_COLS * BS; ++k) on[k] = live && bc1[(int64_t)BS * n1[k / BS] + k % BS] != 0;
+  }
+#pragma unroll
+  for (int k = 0; k < MF_LIFT_COLS * BS; ++k) v[k] = g[(int64_t)BS * n1[k / BS] + k % BS];
+  if (x0) {
+#pragma unroll
+    for (int k = 0; k < MF_LIFT_COLS * BS; ++k) v[k] -= x0[(int64_t)BS * n1[k / BS] + k % BS];
+  }
+#pragma unroll
+  for (int k = 0; k < MF_LIFT_COLS * BS; ++k) v[k] = on[k] ? scale * v[k] : 0.0;
 #ifdef SK_TRACE
 #pragma unroll
-  for (int j0 = 0; j0 < ND; j0 += 4) {
-    const int j = j0 + wave;
-    if (j >= ND) continue;
-    const int64_t col = dm1[c * ND + j];
-    const bool o = on(j, col);
-    son[j * 64 + (tid & 63)] = o;
-    sv[j * 64 + (tid & 63)] = o ? value(col) : 0.0;
-  }
-#else
-  double v[ND * BS];
-  uint64_t non[(ND + 63) / 64] = {};                   // nodes with a constrained component
-#pragma unroll
-  for (int j = 0; j < ND; ++j) {
-    const int64_t n1 = dm1[c * ND + j];
-#pragma unroll
-    for (int bb = 0; bb < BS; ++bb) {
-      const bool o = on(j * BS + bb, BS * n1 + bb);
-      non[j / 64] |= (uint64_t)o << (j % 64);
-      v[j * BS + bb] = o ? value(BS * n1 + bb) : 0.0;
-    }
+  for (int t_ = 0; t_ < RI; ++t_) {
+    if (4 * t_ + wave >= ND) continue;
+    son[(4 * t_ + wave) * 64 + (tid & 63)] = on[t_];
+    sv[(4 * t_ + wave) * 64 + (tid & 63)] = v[t_];
   }
 #endif
-  double x[NV][3];
-  for (int v_ = 0; v_ < NV; ++v_) {
-    const int64_t gv = geo[c * NV + v_];
-    x[v_][0] = xg[3 * gv]; x[v_][1] = xg[3 * gv + 1]; x[v_][2] = xg[3 * gv + 2];
-  }
   const double J00 = x[1][0] - x[0][0], J01 = x[2][0] - x[0][0], J02 = x[3][0] - x[0][0];
   const double J10 = x[1][1] - x[0][1], J11 = x[2][1] - x[0][1], J12 = x[3][1] - x[0][1];
   const double J20 = x[1][2] - x[0][2], J21 = x[2][2] - x[0][2], J22 = x[3][2] - x[0][2];
@@ -749,7 +771,6 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
   const double M01 = adet * (K[0] * K[3] + K[1] * K[4] + K[2] * K[5]);
   const double M02 = adet * (K[0] * K[6] + K[1] * K[7] + K[2] * K[8]);
   const double M12 = adet * (K[3] * K[6] + K[4] * K[7] + K[5] * K[8]);
-  constexpr int RI = (ND + 3) / 4;                     // rows per wave
   double be[RI];
 #pragma unroll
   for (int r = 0; r < RI; ++r) be[r] = 0.0;
@@ -775,7 +796,17 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
     const int i = wave * RI + r;
     if (!live || i >= ND) continue;
     if (slot) atomicAdd(&sacc[slot[(int64_t)li * ND + i]], be[r]);
-    else atomicAdd(&b[dm0[c * ND + i]], be[r]);
+    else sacc[(tid & 63) * ND + i] = be[r];
+  }
+  if (!slot) {
+    // the rows of a cell on neighbouring lanes: global atomics that meet in a
+    // cache line go together (20^3 P1, every column constrained, with the list:
+    // 27 -> 23 us)
+    __syncthreads();
+    for (int p = tid; p < min(64, nl - (int)blockIdx.x * 64) * ND; p += NT) {
+      const int64_t cp = ents[list[blockIdx.x * 64 + p / ND]];
+      atomicAdd(&b[dm0[cp * ND + p % ND]], sacc[p]);
+    }
   }
 #else
   double gi[NQ][3];
@@ -786,7 +817,9 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
   for (int a = 0; a < BS; ++a) be[a] = 0.0;
 #pragma unroll
   for (int j = 0; j < ND; ++j) {
-    if (!((non[j / 64] >> (j % 64)) & 1)) continue;
+    bool any = false;
+    for (int bb = 0; bb < BS; ++bb) any |= on[j * BS + bb];
+    if (!any) continue;
     double G[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     for (int q = 0; q < NQ; ++q) {
       double gj[3];
@@ -818,6 +851,8 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
       atomicAdd(&b[(int64_t)BS * row[p / BS] + p % BS], sacc[p]);
   }
 }
+#undef MF_LIFT_COLS
+#undef MF_LIFT_COL
 #undef MF_LIFT_BLOCK
 #undef MF_LIFT_ROWS
 )";

@@ -483,3 +483,30 @@ def test_lifting_of_zero_values_keeps_nan(form, noalloc):
     assert nan.any() and not nan.all()
     assert np.array_equal(np.isnan(got), nan)
     assert _rel(got[~nan], ref[~nan]) <= TOL
+
+
+@pytest.mark.parametrize("form,n,share", [
+    ((1,), 1, 0.2), ((1,), 5, 0.02), ((1,), 5, 1.0), ((2,), 3, 0.5), ((3,), 1, 0.0), ((3,), 4, 0.1), ((), 3, 0.3)])
+def test_lifting_without_a_list_on_the_host(form, n, share):
+    """mf_apply_lifting_noalloc: workgroups past the list's end, the last one
+    partly filled, every cell listed."""
+    import ctypes as C
+    import cudolfinx as cufem
+    from cudolfinx import _lib
+    print(f"[gpu-test] noalloc lifting {'P%d' % form if form else 'vector P2'} n={n} share={share}", flush=True)
+    V, a, L = _poisson(n, *form) if form else _elasticity(n)
+    bc = _some_dofs(V, share, 3)
+    x0 = np.random.default_rng(9).uniform(-1, 1, V.size)
+    af, Lf = cufem.form(a), cufem.form(L)
+    asm = cufem.CUDAAssembler()
+    dbc = asm.pack_bcs([bc])
+    b, xv = asm.create_vector(Lf), asm.create_vector(Lf)
+    xv.data.upload(x0)
+    asm.pack_coefficients(af)
+    _lib.check(_lib.lib().mf_apply_lifting_noalloc(
+        (C.c_void_p * 1)(af.handle.value), 1, b.ptr, b.size,
+        (C.c_void_p * 1)(dbc._get_cpp_bcs(V).handle.value), (C.c_void_p * 1)(xv.ptr.value), -0.7, None))
+    asm.synchronize()
+    ref = np.zeros(V.size)
+    cpu.OracleAssembler(a).apply_lifting(ref, [bc], x0=x0, scale=-0.7)
+    assert _rel(b.to_host(), ref) <= TOL
