@@ -750,6 +750,7 @@ std::string generate_system_source(const mf_form& a, const mf_form& L, const mf_
   m["$ND0"] = std::to_string(a.dm[0]->nd);
   m["$BS0"] = std::to_string(a.dm[0]->bs);
   m["$DBLOCK"] = std::to_string(block);
+  m["$DUN"] = std::to_string(ndb <= 4 ? ndb : 1);   // unrolling of the Dirichlet masks
   m["$DATTR"] = wpe > 0 ? "__attribute__((amdgpu_waves_per_eu(" + std::to_string(wpe) + ")))" : "";
   m["$MAXI"] = std::to_string(std::max(1, std::min(max_items, 6)));
   m["$SEGCAP"] = std::to_string(std::max<int64_t>(2, segcap));

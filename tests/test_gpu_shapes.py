@@ -510,3 +510,44 @@ def test_lifting_without_a_list_on_the_host(form, n, share):
     ref = np.zeros(V.size)
     cpu.OracleAssembler(a).apply_lifting(ref, [bc], x0=x0, scale=-0.7)
     assert _rel(b.to_host(), ref) <= TOL
+
+
+@pytest.mark.parametrize("sets", ["rows", "columns", "both"])
+@pytest.mark.parametrize("which,n", [("tet", 1), ("tet", 4), ("triangle", 1), ("triangle", 9)])
+def test_fused_system_masks_rows_and_columns(which, n, sets):
+    """Row and column sets of their own (four and three dofs per cell): the masks of
+    a cell's neighbours, overwriting and adding."""
+    import cudolfinx as cufem
+    from cudolfinx import _lib
+    from mifem.mesh import create_unit_square
+    from mifem.nonlinear import reference_test_forms
+    print(f"[gpu-test] DG1 system on {which} n={n}, {sets}", flush=True)
+    if which == "tet":
+        P = problems.dg_plaplace(n)
+        a, L, u = P.a, P.L, P.extras["u"]
+    else:
+        R = reference_test_forms(create_unit_square(n, n), 1)
+        a, L, u = R["matrix"][2], R["vector"][2], R["u_dg"]
+    V = a.function_spaces[0]
+    u.x[:] = np.random.default_rng(n).uniform(-1, 1, V.size)
+    b0, b1 = _some_dofs(V, 0.1, 1), _some_dofs(V, 0.05, 2)
+    J, F = cufem.form(a), cufem.form(L)
+    asm = cufem.CUDAAssembler()
+    p0, p1 = asm.pack_bcs([b0] if sets != "columns" else []), asm.pack_bcs([b1] if sets != "rows" else [])
+    A, b, S = asm.create_matrix(J), asm.create_vector(F), cufem.CUDASystem(J, F)
+    asm.pack_coefficients(J)
+    o = cpu.OracleAssembler(a)
+    rp, cols, _, _ = o.sparsity()
+    full, rhs = o.assemble_matrix(rp, cols, []), cpu.OracleAssembler(L).assemble_vector()
+    rows = np.repeat(np.arange(V.size), np.diff(rp))
+    m0, m1 = np.zeros(V.size, bool), np.zeros(V.size, bool)
+    m0[b0.dofs], m1[b1.dofs] = sets != "columns", sets != "rows"
+    for times in (1, 2):
+        _lib.check(_lib.lib().mf_system_assemble(S.handle, A.handle, p0._get_cpp_bcs(V).handle,
+                                                 p1._get_cpp_bcs(V).handle, 2.5, b.ptr, b.size, None,
+                                                 int(times == 1), None))
+        asm.synchronize()
+        ref = np.where(m0[rows] | m1[cols], 0.0, times * full)
+        ref[(rows == cols) & m0[rows]] = 2.5
+        assert _rel(A.csr()[2], ref) <= TOL
+        assert _rel(b.to_host(), times * rhs) <= TOL
