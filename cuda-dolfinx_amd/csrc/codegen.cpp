@@ -947,11 +947,22 @@ std::string compile_source(mf_form& f) {
   // nd x nd x 6 table in LDS: 2048 values, and for P3 3040, which its 64 rows
   // fill (four workgroups per CU in FP32); 256 pairs at P2 and P3, one per thread (P2 25^3 33.6 us at 384, 32.6 at
   // 256; P3 24^3 83 us at 2048 / 384, 75 at 3040 / 256), 384 at P1, whose rows
-  // have 24 each.  Vector forms 4640 values and 128 pairs, two full groups
-  // of lanes, at which four workgroups share a CU (vector P2 48^3: 4608 values and
-  // 384 pairs 757 us, 160 pairs 742; with the pairs dealt by bank 160 pairs 606,
-  // 4640 values and 128 pairs 597; 13^3 24.3 and 22.7 us).  Fewer pairs than a node has cells would send the form to
-  // another kernel, so then it is 384.  Hexahedra 4096.
+  // have 24 each.  Other forms so that values and pairs run out together, by the
+  // values that a pair brings:
+  // - three components at P2 (32): 4640 values and 128 pairs, two full groups
+  //   of lanes, at which four workgroups share a CU (48^3: 4608 values and
+  //   384 pairs 757 us, 160 pairs 742; with the pairs dealt by bank 160 pairs 606,
+  //   4640 values and 128 pairs 597; 13^3 24.3 and 22.7 us);
+  // - P1 (0.6 to 6): 2304 and 256 (three components 48^3: 4640 / 128 179 us,
+  //   4608 / 384 166, this 164; two 24^3 22.9, 23.2, 22.3; one 40^3 44.2,
+  //   35.3, 31.5);
+  // - one or two components (4 to 14): 3040 and 256 (one at P2 25^3: 4640 / 128
+  //   47.9 us, 4608 / 384 43.7, this 40.6; two at P2 16^3 24.6, 25.9, 24.9 and 28^3
+  //   91.6, 88 to 91, 90.8; one at P3 20^3 2048 / 384 370, this 338);
+  // - 128 pairs where 256 would leave half of the CUs without a chunk (P1 with
+  //   three components 8^3 9.2 us for 11.0, P2 with one 6^3 8.4 for 9.5).
+  // Fewer pairs than a node has cells would send the form to another kernel, so
+  // then it is 384.  Hexahedra 4096.
   bool trace = false, hex = false;
   for (auto& I : f.ints) {
     trace |= staged_trace(*I);
@@ -963,16 +974,23 @@ std::string compile_source(mf_form& f) {
   f.shape_default |= !given;
   const int nd = f.rank == 2 ? f.dm[0]->nd : 0;
   if (f.shape_default && f.rank == 2) {
-    f.options["chunk_values"] = trace ? (nd > 10 ? 3040 : 2048) : (hex ? 4096 : 4640);
+    const int bs = f.dm[0]->bs;
+    f.options["chunk_values"] = trace ? (nd > 10 ? 3040 : 2048) : hex ? 4096 : nd <= 4 ? 2304 : bs < 3 ? 3040 : 4640;
     if (!hex) {
       int most = 0;                                     // cells of a node
+      int64_t all = 0;                                  // (cell, row) pairs
       for (auto& I : f.ints) {
         if (I->type != MF_CELL || I->staged_src.empty()) continue;
         std::vector<int> cells(f.dm[0]->num_nodes, 0);
+        all += I->n * nd;
         for (int32_t c : I->h_ents)
           for (int i = 0; i < nd; ++i) most = std::max(most, ++cells[f.dm[0]->host[(int64_t)c * nd + i]]);
       }
-      f.options["owner_pairs"] = trace ? (nd > 4 && most <= 256 ? 256 : 384) : (most <= 128 ? 128 : 384);
+      int pairs = 384;
+      if (trace) pairs = nd > 4 ? 256 : 384;
+      else if ((nd > 4 && bs == 3) || (f.ctx && all < 128LL * f.ctx->num_cus && most <= 128)) pairs = 128;
+      else pairs = 256;
+      f.options["owner_pairs"] = most <= pairs ? pairs : 384;
     }
   }
   const int64_t cap = f.opt("chunk_values", trace ? 2048 : (hex ? 4096 : 4608));

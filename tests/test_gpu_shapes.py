@@ -551,3 +551,36 @@ def test_fused_system_masks_rows_and_columns(which, n, sets):
         ref[(rows == cols) & m0[rows]] = 2.5
         assert _rel(A.csr()[2], ref) <= TOL
         assert _rel(b.to_host(), times * rhs) <= TOL
+
+
+@pytest.mark.parametrize("degree,bs,n,times", [(1, 3, 1, 1), (1, 3, 5, 1), (1, 3, 11, 1), (1, 3, 2, 8), (1, 3, 2, 12),
+                                               (1, 1, 4, 1), (1, 1, 12, 1), (2, 1, 3, 1), (2, 1, 8, 1), (2, 1, 2, 12),
+                                               (3, 1, 2, 1)])
+def test_default_shapes_of_sums_over_points(degree, bs, n, times):
+    """The owner kernel of forms without a reference tensor, by degree and components:
+    meshes on both sides of the size at which a chunk's pairs change, and cells listed
+    several times (rows of more than 128 and 256 cells); the owner kernel runs
+    (matrix_kernel = 2 refuses any other)."""
+    import dataclasses
+    import cudolfinx as cufem
+    print(f"[gpu-test] default shape P{degree} x {bs} n={n} cells listed {times} times", flush=True)
+    if bs == 3:
+        mesh = create_unit_cube(n, jitter=0.2, seed=n)
+        V, D = functionspace(mesh, ("P", degree), shape=(3,)), functionspace(mesh, ("DG", 0))
+        mu, lam = Function(D), Function(D)
+        mu.x[:], lam.x[:] = np.random.default_rng(n).uniform(1, 2, (2, mesh.num_cells))
+        a = forms.elasticity(V, mu, lam)
+    else:
+        V, a, _ = _poisson(n, degree)
+        I = a.integrals[0]
+        a = dataclasses.replace(a, integrals=[dataclasses.replace(
+            I, staged=dataclasses.replace(I.staged, trace_only=False))])
+    ents = np.repeat(np.arange(V.mesh.num_cells, dtype=np.int32), times)
+    a = dataclasses.replace(a, integrals=[dataclasses.replace(a.integrals[0], entities=ents)])
+    bc = _some_dofs(V, 0.1, 3)
+    asm = cufem.CUDAAssembler()
+    A = asm.assemble_matrix(cufem.form(a, options={"matrix_kernel": 2}), bcs=[bc], diagonal=2.0)
+    asm.synchronize()
+    o = cpu.OracleAssembler(a)
+    rp, cols, _, _ = o.sparsity()
+    assert _rel(A.csr()[2], o.assemble_matrix(rp, cols, [bc], diagonal=2.0)) <= TOL
