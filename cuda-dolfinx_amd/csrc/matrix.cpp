@@ -546,6 +546,8 @@ DevArray<int32_t>& get_table(mf_form* a, Integral& I, mf_matrix* A, hipStream_t 
 // the prefix sum), null when the workspace would exceed 4 GiB (its offsets are
 // int32, and one matrix holds it for good), or when it does not exist yet and
 // s is being captured: the per-entity kernel with its offset table serves then.
+// That table is built along, so that any uncaptured call leaves what a captured
+// one may need, overwriting or adding.
 static GatherPlan* gather_plan(mf_form* a, Integral& I, mf_matrix* A, hipStream_t s) {
   const auto key = std::make_pair(a->uid, I.index);
   auto it = A->gathers.find(key);
@@ -558,6 +560,7 @@ static GatherPlan* gather_plan(mf_form* a, Integral& I, mf_matrix* A, hipStream_
   const int ncell = entity_ncell(I.type), ni = ncell * d0->nd, nj = ncell * d1->nd;
   const int64_t planes = (int64_t)ni * d0->bs * nj * d1->bs, ws = (I.n + 63) / 64 * 64 * planes;
   if (ws > (int64_t(1) << 29) || I.n * ni * nj >= INT32_MAX) return A->gathers[key].get();
+  get_table(a, I, A, s);
   auto g = std::make_unique<GatherPlan>();
   DevArray<int32_t> count, missing;
   count.alloc(std::max<int64_t>(1, A->nnz_b));

@@ -584,3 +584,55 @@ def test_default_shapes_of_sums_over_points(degree, bs, n, times):
     o = cpu.OracleAssembler(a)
     rp, cols, _, _ = o.sparsity()
     assert _rel(A.csr()[2], o.assemble_matrix(rp, cols, [bc], diagonal=2.0)) <= TOL
+
+
+def _replays(g, launches, state, eager, check):
+    """Each replay of graph g with another state, between eager runs of the same
+    calls, against them."""
+    import torch
+    for k in range(launches):
+        state(k)
+        torch.cuda.synchronize()
+        g.launch()
+        torch.cuda.synchronize()
+        got = check()
+        state(k)
+        eager()
+        torch.cuda.synchronize()
+        ref = check()
+        assert _rel(got, ref) <= TOL, k
+        state(k + launches)
+        eager()
+        torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("warm,captured", [(True, False), (False, True), (True, True)])
+def test_capture_of_a_gathered_matrix_after_either_mode(warm, captured):
+    """One uncaptured call, overwriting or adding, is enough for a captured one of
+    either kind (forms without an owner kernel)."""
+    import torch
+    import cudolfinx as cufem
+    from mifem.nonlinear import reference_test_forms
+    print(f"[gpu-test] gathered matrix: eager zero={warm}, captured zero={captured}", flush=True)
+    R = reference_test_forms(create_unit_cube(3, jitter=0.2, seed=1), 2)
+    a = R["matrix"][0]
+    V = a.function_spaces[0]
+    s = torch.cuda.Stream()
+    asm = cufem.CUDAAssembler(stream=s)
+    f = cufem.form(a)
+    u = torch.zeros(V.size, dtype=torch.float64, device="cuda")
+    f.set_coefficient_device(0, u.data_ptr(), V.size)
+    A = asm.create_matrix(f)
+    asm.assemble_matrix(f, A, zero=warm)
+    asm.synchronize()
+    g = cufem.CUDAGraph(s)
+    with g:
+        asm.assemble_matrix(f, A, zero=captured)
+
+    def state(k):
+        u.copy_(torch.from_numpy(np.random.default_rng(k).uniform(-1, 1, V.size)))
+        h = A.device_arrays()[2]
+        from cudolfinx import _lib
+        _lib.check(_lib.lib().mf_zero(asm._ctx.handle, h, A.nnz, asm._stream))
+
+    _replays(g, 3, state, lambda: asm.assemble_matrix(f, A, zero=captured), lambda: A.csr()[2].copy())
