@@ -387,10 +387,15 @@ static bool blocks_pay(const mf_form& L, Integral& I) {
 // Blocks of at most 256 entities (down to 64 where that leaves fewer than
 // three blocks per CU) whose rows fit 64 KB of LDS; null when rows are shared so
 // little that the blocks hold fewer than half their entities.  With a wave per
-// cell 32 cells (down to 4) and 32 KB, in blocks of 256 threads.
-static VectorBlocks* vector_blocks(mf_form* L, const Integral& I) {
+// cell 32 cells (down to 4) and 32 KB, in blocks of 256 threads.  Null also where
+// they do not exist yet and s is being captured: the kernels that need no
+// schedule serve then.
+static VectorBlocks* vector_blocks(mf_form* L, const Integral& I, hipStream_t s) {
   auto it = L->vblocks.find(I.index);
   if (it != L->vblocks.end()) return it->second.get();
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  MF_HIP(hipStreamIsCapturing(s, &cs));
+  if (cs != hipStreamCaptureStatusNone) return nullptr;
   const mf_dofmap* d0 = L->dm[0];
   const int nd = d0->nd, bs = d0->bs;
   auto B = std::make_unique<VectorBlocks>();
@@ -1011,7 +1016,7 @@ void assemble_vector(mf_form* L, double* b, int64_t n, int zero, hipStream_t s) 
   if (mode == 0 || mode == 4)
     for (auto& I : L->ints)
       if (I->type == MF_CELL && I->n && (I->k_vblk || I->k_hsrc)) {
-        if (mode == 4 || blocks_pay(*L, *I)) blocks = vector_blocks(L, *I);
+        if (mode == 4 || blocks_pay(*L, *I)) blocks = vector_blocks(L, *I, s);
         if (blocks) owner = I.get();
         break;
       }

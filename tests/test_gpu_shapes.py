@@ -636,3 +636,30 @@ def test_capture_of_a_gathered_matrix_after_either_mode(warm, captured):
         _lib.check(_lib.lib().mf_zero(asm._ctx.handle, h, A.nnz, asm._stream))
 
     _replays(g, 3, state, lambda: asm.assemble_matrix(f, A, zero=captured), lambda: A.csr()[2].copy())
+
+
+@pytest.mark.parametrize("zero", [True, False])
+def test_capture_of_a_right_hand_side_without_an_eager_call(zero):
+    """Forms of more than 32 nodes per cell need no schedule, so their first call
+    may be captured."""
+    import torch
+    import cudolfinx as cufem
+    print(f"[gpu-test] Q3 source, first call captured, zero={zero}", flush=True)
+    P = problems.helmholtz_q3(3, seed=2)
+    s = torch.cuda.Stream()
+    asm = cufem.CUDAAssembler(stream=s)
+    f = cufem.form(P.L)
+    b = asm.create_vector(f)
+    asm.assemble_vector(cufem.form(P.L, options={"vector_kernel": 1}), b)   # b holds something
+    asm.synchronize()
+    g = cufem.CUDAGraph(s)
+    with g:
+        asm.assemble_vector(f, b, zero=zero)
+    ref = cpu.OracleAssembler(P.L).assemble_vector()
+    for k in range(1, 4):
+        g.launch()
+        asm.synchronize()
+        assert _rel(b.to_host(), ref if zero else (2 * k) * ref) <= TOL
+        asm.assemble_vector(f, b, zero=zero)                 # eager calls between the replays
+        asm.synchronize()
+        assert _rel(b.to_host(), ref if zero else (2 * k + 1) * ref) <= TOL
