@@ -831,11 +831,20 @@ void assemble_matrix(mf_form* a, mf_matrix* A, const mf_bc* bc0, const mf_bc* bc
       }
   std::shared_ptr<OwnerPlan> plan;
   if (owner) {
-    // the matrix-core kernels of a hexahedral form have chunks of their own
+    // the matrix-core kernels of a hexahedral form have chunks of their own; every
+    // kernel takes both schedules, and a captured call the one that exists
     const bool hex = owner->k_hprep != nullptr, mfma = hex && a->opt("precision", 64) != 64;
-    auto key = std::make_pair(a->uid, owner->index + (mfma ? static_cast<int>(a->ints.size()) : 0));
+    const int second = static_cast<int>(a->ints.size());
+    auto key = std::make_pair(a->uid, owner->index + (mfma ? second : 0));
     auto it = A->plans.find(key);
-    if (it == A->plans.end() || it->second.first != a->gen) {
+    auto usable = [&] { return it != A->plans.end() && it->second.first == a->gen; };
+    if (hex && !usable()) {
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      MF_HIP(hipStreamIsCapturing(s, &cs));
+      if (cs != hipStreamCaptureStatusNone)
+        it = A->plans.find(std::make_pair(a->uid, owner->index + (mfma ? 0 : second)));
+    }
+    if (!usable()) {
       plan = build_owner_plan(*a, *owner, *A, a->opt("chunk_values", 4096),
                               static_cast<int>(a->opt("chunk_rows", 64)),
                               hex ? static_cast<int>(a->opt("owner_pairs", 384))

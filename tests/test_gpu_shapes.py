@@ -663,3 +663,40 @@ def test_capture_of_a_right_hand_side_without_an_eager_call(zero):
         asm.assemble_vector(f, b, zero=zero)                 # eager calls between the replays
         asm.synchronize()
         assert _rel(b.to_host(), ref if zero else (2 * k + 1) * ref) <= TOL
+
+
+@pytest.mark.parametrize("warm,captured", [(64, 32), (32, 64), (16, 64), (64, 16)])
+def test_capture_of_another_precision(warm, captured):
+    """Q3 matrices: one uncaptured call in one precision is enough for a captured
+    one in another (precision is set between calls)."""
+    import torch
+    import cudolfinx as cufem
+    print(f"[gpu-test] Q3 eager FP{warm}, captured FP{captured}", flush=True)
+    P = problems.helmholtz_q3(3, seed=2)
+    s = torch.cuda.Stream()
+    asm = cufem.CUDAAssembler(stream=s)
+    f = cufem.form(P.a, options={"precision": warm})
+    bcs = asm.pack_bcs([_some_dofs(P.V, 0.1, 3)])
+    A = asm.create_matrix(f)
+    asm.assemble_matrix(f, A, bcs=bcs)
+    asm.synchronize()
+    f.set_option("precision", captured)
+    g = cufem.CUDAGraph(s)
+    with g:
+        asm.assemble_matrix(f, A, bcs=bcs)
+    asm.assemble_matrix(f, A, bcs=bcs)                       # the schedule of its own
+    asm.synchronize()
+    ref = A.csr()[2].copy()
+    o = cpu.OracleAssembler(P.a)
+    rp, cols, _, _ = o.sparsity()
+    tol = {64: TOL, 32: 1e-6, 16: 2e-2}[captured]
+    assert _rel(ref, o.assemble_matrix(rp, cols, [_some_dofs(P.V, 0.1, 3)])) <= tol
+    for _ in range(3):
+        g.launch()
+        asm.synchronize()
+        # the same element arithmetic, summed in another order
+        assert _rel(A.csr()[2], ref) <= TOL
+        f.set_option("precision", warm)
+        asm.assemble_matrix(f, A, bcs=bcs)
+        asm.synchronize()
+        f.set_option("precision", captured)
