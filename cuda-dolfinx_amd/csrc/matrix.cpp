@@ -549,8 +549,8 @@ DevArray<int32_t>& get_table(mf_form* a, Integral& I, mf_matrix* A, hipStream_t 
 
 // Gather plan of one integral (built once per matrix, on the device but for
 // the prefix sum), null when the workspace would exceed 4 GiB (its offsets are
-// int32, and one matrix holds it for good), or when it does not exist yet and
-// s is being captured: the per-entity kernel with its offset table serves then.
+// int32, and one matrix holds it for good), when memory is short, or when it does
+// not exist yet and s is being captured: the per-entity kernel with its offset table serves then.
 // That table is built along, so that any uncaptured call leaves what a captured
 // one may need, overwriting or adding.
 static GatherPlan* gather_plan(mf_form* a, Integral& I, mf_matrix* A, hipStream_t s) {
@@ -568,7 +568,13 @@ static GatherPlan* gather_plan(mf_form* a, Integral& I, mf_matrix* A, hipStream_
   get_table(a, I, A, s);
   auto g = std::make_unique<GatherPlan>();
   DevArray<int32_t> count, missing;
-  count.alloc(std::max<int64_t>(1, A->nnz_b));
+  g->ws = A->gather_ws;
+  if (!g->ws || g->ws->n < ws) g->ws = std::make_shared<DevArray<double>>();
+  if (!(g->ws->n >= ws || g->ws->try_alloc(std::max<int64_t>(1, ws))) ||
+      !g->at.try_alloc(std::max<int64_t>(1, I.n * ni * nj)) ||      // one place per contribution
+      !g->pos.try_alloc(std::max<int64_t>(1, A->nnz_b)) || !g->ptr.try_alloc(A->nnz_b + 1) ||
+      !count.try_alloc(std::max<int64_t>(1, A->nnz_b)))
+    return (A->gathers[key] = nullptr).get();
   missing.alloc(1);
   k_fill_i32(count.ptr, A->nnz_b, 0, s);
   k_fill_i32(missing.ptr, 1, 0, s);
@@ -590,15 +596,13 @@ static GatherPlan* gather_plan(mf_form* a, Integral& I, mf_matrix* A, hipStream_
     ptr[q] = sum;
     sum += c;
   }
-  g->ptr.upload(ptr);
+  MF_HIP(hipMemcpy(g->ptr.ptr, ptr.data(), sizeof(int32_t) * ptr.size(), hipMemcpyHostToDevice));
   MF_HIP(hipMemcpyAsync(count.ptr, g->ptr.ptr, sizeof(int32_t) * A->nnz_b, hipMemcpyDeviceToDevice, s));
-  g->at.alloc(std::max<int32_t>(1, sum));
-  g->pos.alloc(std::max<int64_t>(1, A->nnz_b));
   pass(g->at.ptr);
   k_gather_sort(g->at.ptr, g->ptr.ptr, g->pos.ptr, A->nnz_b, A->nrows_b, A->rpb.ptr, A->row_ptr.ptr,
                 d0->bs, d1->bs, s);
-  g->ws.alloc(std::max<int64_t>(1, ws));
   MF_HIP(hipStreamSynchronize(s));                     // count and missing are freed here
+  A->gather_ws = g->ws;
   return (A->gathers[key] = std::move(g)).get();
 }
 
@@ -956,9 +960,9 @@ void assemble_matrix(mf_form* a, mf_matrix* A, const mf_bc* bc0, const mf_bc* bc
       const int nc = entity_ncell(I.type) * a->dm[1]->nd * a->dm[1]->bs;
       launch(I.k_ten, static_cast<uint32_t>((I.n + 63) / 64), 64, 0, s,
              static_cast<int32_t>(I.n), I.d_ents.ptr, a->mesh->cells.ptr, a->mesh->x.ptr,
-             a->packed.ptr, a->consts.ptr, a->dm[0]->dev.ptr, a->dm[1]->dev.ptr, m0, m1, g->ws.ptr,
+             a->packed.ptr, a->consts.ptr, a->dm[0]->dev.ptr, a->dm[1]->dev.ptr, m0, m1, g->ws->ptr,
              a->mesh->fperm.ptr);
-      k_gather(A->values, g->ws.ptr, g->ptr.ptr, g->at.ptr, g->pos.ptr, A->nnz_b, a->dm[0]->bs,
+      k_gather(A->values, g->ws->ptr, g->ptr.ptr, g->at.ptr, g->pos.ptr, A->nnz_b, a->dm[0]->bs,
                a->dm[1]->bs, nc, s);
     } else {
       gathered = nullptr;

@@ -60,6 +60,18 @@ struct DevArray {
     MF_HIP(hipMalloc(reinterpret_cast<void**>(&ptr), sizeof(T) * count));
     n = count;
   }
+  // false, and nothing left for a later call to report, where memory is short
+  bool try_alloc(int64_t count) {
+    reset();
+    if (count <= 0) return true;
+    if (hipMalloc(reinterpret_cast<void**>(&ptr), sizeof(T) * count) != hipSuccess) {
+      (void)hipGetLastError();
+      ptr = nullptr;
+      return false;
+    }
+    n = count;
+    return true;
+  }
   void upload(const T* host, int64_t count) {
     alloc(count);
     if (count > 0) MF_HIP(hipMemcpy(ptr, host, sizeof(T) * count, hipMemcpyHostToDevice));
@@ -296,12 +308,14 @@ struct Coef {
 };
 // Gather of one integral's element tensors into a matrix's values: per blocked
 // CSR entry q the contributions at[ptr[q] .. ptr[q + 1]) (workspace offsets,
-// ascending) and its place in the values.  The workspace belongs to the matrix:
-// a call that overwrites the values cannot run beside another on that matrix.
+// ascending) and its place in the values.  The plans of a matrix share a
+// workspace (a larger one replaces it in plans to come; captured graphs keep
+// the one that they were recorded with): a call that overwrites the values
+// cannot run beside another on that matrix.
 struct GatherPlan {
   DevArray<int32_t> ptr, at;
   DevArray<int2> pos;
-  DevArray<double> ws;
+  std::shared_ptr<DevArray<double>> ws;
 };
 // Blocks of consecutive entities of a cell integral of a linear form: entities
 // ent[k] .. ent[k + 1], the block's distinct nodes row[ptr[k] ..] (ascending)
@@ -421,8 +435,10 @@ struct mf_matrix {
   // makes them stale; they are rebuilt on the next assembly)
   std::map<std::pair<uint64_t, int>, std::pair<uint64_t, std::shared_ptr<mf::OwnerPlan>>> plans;
   std::map<uint64_t, std::shared_ptr<mf::DGPlan>> dgplans;   // per form uid (null: unsupported)
-  // per (form uid, integral index) gathers of element tensors (null: too large)
+  // per (form uid, integral index) gathers of element tensors (null: not for this
+  // integral), and the workspace for the next
   std::map<std::pair<uint64_t, int>, std::unique_ptr<mf::GatherPlan>> gathers;
+  std::shared_ptr<mf::DevArray<double>> gather_ws;
   // adopted caller pattern without the bs-unrolled block structure: the form
   // assembles into `inner` (its own pattern), whose value k is then added at
   // position inner_map[k] of this matrix's values

@@ -700,3 +700,32 @@ def test_capture_of_another_precision(warm, captured):
         asm.assemble_matrix(f, A, bcs=bcs)
         asm.synchronize()
         f.set_option("precision", captured)
+
+
+def test_forms_on_one_matrix_share_a_gather_workspace():
+    """A program that builds its form again and again for a matrix it keeps: device
+    memory grows by a form's own tables, not by another workspace."""
+    import dataclasses
+    import torch
+    import cudolfinx as cufem
+    print("[gpu-test] forms rebuilt against one matrix: device memory", flush=True)
+    V, a, _ = _elasticity(8)
+    a = dataclasses.replace(a, integrals=[dataclasses.replace(a.integrals[0], staged=None)])
+    asm = cufem.CUDAAssembler()
+    first = cufem.form(a)
+    A = asm.assemble_matrix(first)
+    asm.synchronize()
+    ref = A.csr()[2].copy()
+    workspace = 8 * 900 * V.mesh.num_cells                   # the element tensors
+    before = torch.cuda.mem_get_info()[0]
+    for _ in range(6):
+        f = cufem.form(a)
+        asm.assemble_matrix(f, A)
+        asm.synchronize()
+        assert _rel(A.csr()[2], ref) <= TOL
+        del f
+    used = before - torch.cuda.mem_get_info()[0]
+    assert used < 3 * workspace, (used, workspace)
+    asm.assemble_matrix(first, A)                            # its plan still holds what it needs
+    asm.synchronize()
+    assert _rel(A.csr()[2], ref) <= TOL

@@ -53,3 +53,23 @@ def test_hexahedral_shapes_compile(driver, options):
 def test_hexahedral_block_of_whole_waves(driver, block):
     K, msg = driver(problems.helmholtz_q3(2).a, hex_block=block)
     assert K is None and "hex_block" in msg and "error:" not in msg
+
+
+def test_allocation_that_may_fail(tmp_path):
+    """DevArray::try_alloc of a petabyte (or without a device, of anything): false and
+    no exception; with a device, no error left that the next call would report."""
+    if not shutil.which("hipcc"):
+        pytest.skip("hipcc not available")
+    (tmp_path / "t.cpp").write_text('''#include "mf_internal.h"
+int main() {
+  mf::DevArray<double> d;
+  if (d.try_alloc(int64_t(1) << 47) || d.ptr || d.n) return 1;
+  if (!d.try_alloc(0) || d.ptr) return 2;
+  int n = 0;
+  if (hipGetDeviceCount(&n) != hipSuccess || n == 0) return 0;
+  return hipGetLastError() == hipSuccess ? 0 : 3;
+}
+''')
+    subprocess.run(["hipcc", "--offload-arch=gfx950", "-std=c++17", "-O1", f"-I{ROOT / 'cuda-dolfinx_amd' / 'csrc'}",
+                    f"-I{ROOT / 'include'}", str(tmp_path / "t.cpp"), "-o", str(tmp_path / "t")], check=True)
+    assert subprocess.run([str(tmp_path / "t")], timeout=60).returncode == 0
