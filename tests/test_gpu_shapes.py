@@ -729,3 +729,30 @@ def test_forms_on_one_matrix_share_a_gather_workspace():
     asm.assemble_matrix(first, A)                            # its plan still holds what it needs
     asm.synchronize()
     assert _rel(A.csr()[2], ref) <= TOL
+
+
+@pytest.mark.parametrize("n,share", [(3, 30), (3, 70), (5, 200), (7, 2058)])
+def test_matrix_with_a_node_that_many_cells_share(n, share):
+    """Entries of 30 to 2,058 contributions, on both sides of the line between the
+    gather and the per-entity kernel."""
+    import cudolfinx as cufem
+    print(f"[gpu-test] P1 mass n={n}, one node in {share} cells", flush=True)
+    V = functionspace(create_unit_cube(n, jitter=0.2, seed=1), ("P", 1))
+    d = V.dofmap.copy()
+    for c in np.random.default_rng(1).permutation(d.shape[0])[:share]:
+        if 0 not in d[c]:
+            d[c, 3] = 0
+    V._dofmap = d
+    a = forms.mass(V)
+    bc = _some_dofs(V, 0.1, 3)
+    asm = cufem.CUDAAssembler()
+    f = cufem.form(a)
+    A = asm.assemble_matrix(f, bcs=[bc], diagonal=2.0)
+    asm.synchronize()
+    o = cpu.OracleAssembler(a)
+    rp, cols, _, _ = o.sparsity()
+    ref = o.assemble_matrix(rp, cols, [bc], diagonal=2.0)
+    assert _rel(A.csr()[2], ref) <= TOL
+    asm.assemble_matrix(f, A, zero=False)
+    asm.synchronize()
+    assert _rel(A.csr()[2], ref + o.assemble_matrix(rp, cols, [])) <= TOL
