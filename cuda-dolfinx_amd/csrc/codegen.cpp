@@ -430,21 +430,49 @@ bool owner_supported(const mf_form& f, const Integral& I) {
   return nd <= 32 && nd * bs <= 32;
 }
 
-OwnerShape owner_shape(const mf_form& f, const Integral& I) {
-  // Cells per batch (NB) and pairs per chunk (MAXP) so that the kernel's
-  // static LDS fits the per-workgroup budget.
-  const int nd = staged_define(I.staged_src, "SK_ND");
-  const int bs = staged_define(I.staged_src, "SK_BS");
+// The MF_SHARED slices of one owner-computes body (kOwnerTemplate), in
+// declaration order: name, element type, bytes (rounded up to 16).  The
+// last slice holds the reference tensors (sRS or sRT) of those variants, the
+// reference gradients (sDPHI) otherwise.
+struct LdsSlice {
+  const char* name;
+  const char* type;
+  int64_t bytes;
+};
+
+static std::vector<LdsSlice> owner_lds_slices(const mf_form& f, const Integral& I, bool f32) {
+  auto r16 = [](int64_t b) { return (b + 15) / 16 * 16; };
+  const int64_t nd = staged_define(I.staged_src, "SK_ND");
   const int64_t cap = f.opt("chunk_values", 4096), maxr = f.opt("chunk_rows", 64);
+  const int64_t maxp = f.opt("owner_pairs", 384);
+  const bool f32acc = f32 && f.opt("owner_f32acc", 0);
+  const char* at = f32 ? "float" : "double";
+  const int64_t as = f32 ? 4 : 8;
+  std::vector<LdsSlice> v = {{"acc", f32acc ? "float" : "double", r16((f32acc ? 4 : 8) * cap)},
+                             {"lrp", "int32_t", r16(4 * (maxr + 1))},
+                             {"snb", "int32_t", r16(4 * maxr)},
+                             {"spair", "int32_t", r16(4 * maxp)},
+                             {"skk", "uint8_t", r16(maxp * nd)}};
+  if (staged_trace(I)) v.push_back({"sRS", at, r16(as * nd * MF_REF_STRIDE(nd, as))});
+  else if (staged_fullrt(I)) v.push_back({"sRT", "double", r16(8 * nd * nd * 9)});
+  else v.push_back({"sDPHI", "double", r16(8 * staged_define(I.staged_src, "SK_NQ") * nd * 3)});
+  return v;
+}
+
+static int64_t owner_lds_bytes(const mf_form& f, const Integral& I, bool f32) {
+  int64_t b = 0;
+  for (const auto& sl : owner_lds_slices(f, I, f32)) b += sl.bytes;
+  return b;
+}
+
+OwnerShape owner_shape(const mf_form& f, const Integral& I) {
+  // Cells per batch (NB) and pairs per chunk (MAXP); the kernel's static LDS, in
+  // FP64, has to fit the per-workgroup budget.
   const int64_t budget = f.opt("owner_lds", 64 * 1024);
-  const int64_t fixed = 8 * cap + 4 * (maxr + 1) + 4 * (cap / (bs * bs) + 1) + 32;
   OwnerShape sh;
   sh.nb = static_cast<int>(std::min<int64_t>(f.opt("owner_nb", 64), 1023));
   sh.maxp = static_cast<int>(f.opt("owner_pairs", 384));
-  const int64_t nq = staged_define(I.staged_src, "SK_NQ");
-  const int64_t trace = staged_trace(I) ? 8LL * nd * nd * 6
-                                        : (staged_fullrt(I) ? 8LL * nd * nd * 9 : 8LL * nq * nd * 3);
-  const int64_t used = fixed + trace + (int64_t)sh.maxp * (4 + nd);
+  const int64_t used = owner_lds_bytes(f, I, false);
   MF_CHECK(used <= budget, MF_EUNSUPPORTED,
            "owner-computes kernel shape exceeds the LDS budget (" + std::to_string(used) + " > " +
                std::to_string(budget) + " bytes)");
@@ -459,7 +487,7 @@ bool owner_pipe_emitted(const mf_form& f, const Integral& I) {
   const int64_t maxp = owner_shape(f, I).maxp;
   const int64_t lists = 4 * maxp + (maxp * nd + 15) / 16 * 16 + 4 * (maxr + 1) + maxr;
   const int64_t nq = staged_define(I.staged_src, "SK_NQ");
-  const int64_t table = staged_trace(I) ? 8 * nd * nd * 6
+  const int64_t table = staged_trace(I) ? 8 * nd * MF_REF_STRIDE(nd, 8)
                                         : (staged_fullrt(I) ? 8 * nd * nd * 9 : 8 * nq * nd * 3);
   return f.opt("owner_f32acc", 0) == 0 && 16 * cap + 2 * lists + table + 256 <= 160 * 1024;
 }
@@ -758,48 +786,11 @@ std::string generate_system_source(const mf_form& a, const mf_form& L, const mf_
   return os.str();
 }
 
-// The MF_SHARED slices of one owner-computes body (kOwnerTemplate), in
-// declaration order: name, element type, bytes (rounded up to 16).  The
-// last slice holds the reference tensors (sRS or sRT) of those variants, the
-// reference gradients (sDPHI) otherwise.
-struct LdsSlice {
-  const char* name;
-  const char* type;
-  int64_t bytes;
-};
 static bool owner_f32(const mf_form& f, const Integral& I) {
   return staged_trace(I) && f.opt("precision", 64) == 32;
 }
 
-// MF_RST of the owner kernel: numbers of size sz between rows of the reference tensors
-static int64_t ref_stride(int64_t nd, int64_t sz) {
-  return nd * 6 + (8 - nd * 6 * (sz / 4) % 8 + 4) % 8 / (sz / 4);
-}
-
-static std::vector<LdsSlice> owner_lds_slices(const mf_form& f, const Integral& I) {
-  auto r16 = [](int64_t b) { return (b + 15) / 16 * 16; };
-  const int64_t nd = staged_define(I.staged_src, "SK_ND");
-  const int64_t cap = f.opt("chunk_values", 4096), maxr = f.opt("chunk_rows", 64);
-  const int64_t maxp = owner_shape(f, I).maxp;
-  const bool f32 = owner_f32(f, I), f32acc = f32 && f.opt("owner_f32acc", 0);
-  const char* at = f32 ? "float" : "double";
-  const int64_t as = f32 ? 4 : 8;
-  std::vector<LdsSlice> v = {{"acc", f32acc ? "float" : "double", r16((f32acc ? 4 : 8) * cap)},
-                             {"lrp", "int32_t", r16(4 * (maxr + 1))},
-                             {"snb", "int32_t", r16(4 * maxr)},
-                             {"spair", "int32_t", r16(4 * maxp)},
-                             {"skk", "uint8_t", r16((maxp * nd + 15) / 16 * 16)}};
-  if (staged_trace(I)) v.push_back({"sRS", at, r16(as * nd * ref_stride(nd, as))});
-  else if (staged_fullrt(I)) v.push_back({"sRT", "double", r16(8 * nd * nd * 9)});
-  else v.push_back({"sDPHI", "double", r16(8 * staged_define(I.staged_src, "SK_NQ") * nd * 3)});
-  return v;
-}
-
-int64_t owner_lds_bytes(const mf_form& f, const Integral& I) {
-  int64_t b = 0;
-  for (const auto& sl : owner_lds_slices(f, I)) b += sl.bytes;
-  return b;
-}
+int64_t owner_lds_bytes(const mf_form& f, const Integral& I) { return owner_lds_bytes(f, I, owner_f32(f, I)); }
 
 // The cell-integral vectors of several linear forms (one element group
 // each) in ONE launch: each form's owner vector body becomes a device
@@ -895,7 +886,7 @@ std::string generate_batch_source(const std::vector<const mf_form*>& forms,
     // each LDS slice arrives as its own __restrict__ parameter: slices carved
     // from one buffer would otherwise be assumed to overlap, which orders
     // every LDS load after every earlier LDS store
-    const auto slices = owner_lds_slices(f, I);
+    const auto slices = owner_lds_slices(f, I, owner_f32(f, I));
     std::string sparams, sargs;
     int64_t off = 0;
     for (const auto& sl : slices) {

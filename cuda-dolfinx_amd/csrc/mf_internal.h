@@ -463,6 +463,12 @@ bool hex_source_emitted(const mf_form& f, const Integral& I);
 constexpr int kHexSourceCells = 32;   // most cells in a block of the hexahedral source kernel
 int hex_batch(const mf_form& f, const Integral& I, int prec);
 int hex_block(const mf_form& f, int prec);
+// Numbers of size sz between the rows of the reference tensors in LDS (6 per
+// entry of a row of nd): for the LDS budget here and for the kernels' source.
+#define MF_REF_STRIDE(nd, sz) ((nd) * 6 + (8 - (nd) * 6 * ((sz) / 4) % 8 + 4) % 8 / ((sz) / 4))
+#define MF_STRING_(...) #__VA_ARGS__
+#define MF_STRING(...) MF_STRING_(__VA_ARGS__)
+#define MF_REF_STRIDE_DEFINE "#define MF_RST(nd, sz) " MF_STRING(MF_REF_STRIDE(nd, sz)) "\n"
 struct OwnerShape { int nb = 0, maxp = 0; };
 OwnerShape owner_shape(const mf_form& f, const Integral& I);
 // the warp-specialised owner kernels (mf_ownerp_*, mf_ownerp32_*) are emitted

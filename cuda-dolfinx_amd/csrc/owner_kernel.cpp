@@ -50,7 +50,7 @@ typedef float mf_f2 __attribute__((ext_vector_type(2)));
 // wave's lanes read different rows; P3's 120 doubles alone would give 4 places).
 // With the column list gone too: P3 24^3 93 -> 73 us, a batch of 48 P1-P3
 // instances in FP32 159 -> 110 us, vector P2 48^3 818 -> 778 us.
-#define MF_RST(nd, sz) ((nd) * 6 + (8 - (nd) * 6 * ((sz) / 4) % 8 + 4) % 8 / ((sz) / 4))
+)" MF_REF_STRIDE_DEFINE R"(
 // XCD-aware chunk order: consecutive workgroups land on different XCDs, so
 // each XCD gets a contiguous run of chunks (neighbouring chunks share cells).
 static __device__ __forceinline__ int mf_xcd_chunk(int nchunks)

@@ -55,6 +55,41 @@ def test_hexahedral_block_of_whole_waves(driver, block):
     assert K is None and "hex_block" in msg and "error:" not in msg
 
 
+def _stiffness(degree):
+    from mifem import forms
+    from mifem.fem import Function, functionspace
+    from mifem.mesh import create_unit_cube
+    m = create_unit_cube(2)
+    return forms.stiffness(functionspace(m, ("P", degree)), Function(functionspace(m, ("DG", 0))))
+
+
+@pytest.mark.parametrize("degree,options,fits", [
+    (3, {"chunk_values": 4096, "owner_pairs": 256}, True),               # 58,960 bytes of 65,536
+    (3, {"chunk_values": 4904, "owner_pairs": 256}, True),               # 65,424
+    (3, {"chunk_values": 4936, "owner_pairs": 256}, False),              # 65,680
+    (3, {"chunk_values": 8214, "owner_pairs": 256, "owner_lds": 160 * 1024}, True),
+    (3, {"chunk_values": 8192, "owner_pairs": 256, "owner_lds": 160 * 1024}, True),
+    (2, {"chunk_values": 6144, "owner_pairs": 384}, True),
+    (1, {"chunk_values": 7168, "owner_pairs": 384}, True),
+    (0, {"chunk_values": 6400, "owner_pairs": 128}, True),               # vector P2: its 16 or 32 gradients
+    (0, {"chunk_values": 4608, "owner_pairs": 384}, True),
+])
+def test_owner_shapes_that_fit_the_budget(driver, degree, options, fits):
+    """The LDS that the host counts is the LDS of the compiled kernel: a shape is
+    taken exactly when the kernel fits owner_lds, and a store-wave variant that does
+    not fit a CU is left out."""
+    K, msg = driver(_stiffness(degree) if degree else problems.elasticity_p2(2).a, **options)
+    if not fits:
+        assert K is None and "LDS budget" in msg
+        return
+    assert K is not None, msg[:1000]
+    lds = K["mf_owner_cell_0"][2]
+    assert lds <= options.get("owner_lds", 64 * 1024)
+    assert K.get("mf_ownerp_cell_0", (0, 0, 0))[2] <= 160 * 1024
+    short, msg = driver(_stiffness(degree) if degree else problems.elasticity_p2(2).a, **{**options, "owner_lds": lds - 1})
+    assert short is None and "LDS budget" in msg
+
+
 def test_allocation_that_may_fail(tmp_path):
     """DevArray::try_alloc of a petabyte (or without a device, of anything): false and
     no exception; with a device, no error left that the next call would report."""
