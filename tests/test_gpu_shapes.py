@@ -756,3 +756,105 @@ def test_matrix_with_a_node_that_many_cells_share(n, share):
     asm.assemble_matrix(f, A, zero=False)
     asm.synchronize()
     assert _rel(A.csr()[2], ref + o.assemble_matrix(rp, cols, [])) <= TOL
+
+
+def _two_components(n):
+    """An unsymmetric form of two components per node that depends on the cell's
+    coordinates, and its element tensors by numpy."""
+    V = functionspace(create_unit_cube(n, jitter=0.2, seed=n), ("P", 1), shape=(2,))
+    name = "tabulate_tensor_integral_unsymmetric2"
+    body = ("{\n  for (int i = 0; i < 8; ++i)\n    for (int j = 0; j < 8; ++j)\n"
+            "      A[8 * i + j] += (1 + i + 3 * j) * coordinate_dofs[0] + (2 + i * j) * coordinate_dofs[4] + 0.5 * i;\n}\n")
+    a = forms.Form(2, [V, V], [forms.Integral("cell", -1, np.arange(V.mesh.num_cells, dtype=np.int32), name,
+                                              forms._SIG.format(name=name) + "\n" + body)])
+    i, j = np.meshgrid(np.arange(8), np.arange(8), indexing="ij")
+    x = V.mesh.x[V.mesh.cells]
+    T = ((1 + i + 3 * j) * x[:, 0, 0, None, None] + (2 + i * j) * x[:, 1, 1, None, None] + 0.5 * i)
+    return V, V, a, T
+
+
+def _at_pattern(V, W, rp, cols, T):
+    """The CSR values of the sum of element tensors T (one per cell)."""
+    D = np.zeros((V.size, W.size))
+    for r, c, t in zip(V.unrolled_dofmap(), W.unrolled_dofmap(), T):
+        D[np.ix_(r, c)] += t
+    v = D[np.repeat(np.arange(V.size), np.diff(rp)), cols]
+    assert np.count_nonzero(D) == np.count_nonzero(v)
+    return v
+
+
+@pytest.mark.parametrize("sets", ["none", "equal", "different"])
+@pytest.mark.parametrize("which,n", [("three", 1), ("three", 3), ("two", 1), ("two", 4), ("rectangular", 3),
+                                     ("facets", 1), ("facets", 3), ("interior", 2), ("triangle", 5)])
+def test_gathered_blocks_spaces_and_facets(which, n, sets):
+    """The gather (mf_ten_* is in the source and no owner kernel) of blocks of 3 x 3 and
+    2 x 2, of different row and column spaces and of two-cell entities (facets of a
+    continuous space, whose cells share rows), and a discontinuous space out of order
+    (no gather), against the oracle (numpy for the 2 x 2 form): overwriting, then
+    adding."""
+    import dataclasses
+    import cudolfinx as cufem
+    from cudolfinx import _lib
+    from mifem.mesh import create_unit_square
+    from mifem.nonlinear import reference_test_forms
+    print(f"[gpu-test] gathered {which} n={n}, {sets} Dirichlet sets", flush=True)
+    T = None
+    if which == "three":
+        V, a, _ = _elasticity(n)
+        W = V
+        a = dataclasses.replace(a, integrals=[dataclasses.replace(a.integrals[0], staged=None)])
+    elif which == "two":
+        V, W, a, T = _two_components(n)
+    elif which == "rectangular":
+        m = create_unit_cube(n, jitter=0.2, seed=n)
+        V, W = functionspace(m, ("P", 2)), functionspace(m, ("P", 1))
+        a = forms.mass(V, W)
+    elif which == "facets":
+        from mifem.nonlinear import _int_forms
+        V = W = functionspace(create_unit_cube(n, jitter=0.2, seed=1), ("P", 1))
+        kap, u = Function(V), Function(V)
+        kap.x[:], u.x[:] = np.random.default_rng(4).uniform(0.5, 1, (2, V.size))
+        a = forms.Form(2, [V, V], [_int_forms(V, V, 2)], [kap, u])
+    else:
+        R = reference_test_forms(create_unit_cube(n, jitter=0.2, seed=1) if which == "interior"
+                                 else create_unit_square(n, n), 1)
+        if which == "interior":                              # a discontinuous space not numbered cell by cell
+            a = R["matrix"][2]
+            V = W = a.function_spaces[0]
+            V._dofmap = np.random.default_rng(2).permutation(V.size).astype(np.int32)[V._dofmap]
+            R["u_dg"].x[:] = np.random.default_rng(4).uniform(-1, 1, V.size)
+        else:
+            a = R["matrix"][0]
+            V = W = a.function_spaces[0]
+    f = cufem.form(a)
+    src = f.source()
+    kind = "int" if which in ("interior", "facets") else "cell"
+    assert "mf_mat_" + kind + "_0" in src and "mf_owner_" not in src
+    assert which == "interior" or "mf_ten_" + kind + "_0" in src
+    asm = cufem.CUDAAssembler()
+    A = asm.create_matrix(f)
+    b0 = _some_dofs(V, 0.1, 1)
+    b1 = b0 if sets == "equal" and V is W else _some_dofs(W, 0.2, 2)
+    none = sets == "none"
+    p0 = asm.pack_bcs([] if none else [b0])
+    p1 = p0 if b1 is b0 else asm.pack_bcs([] if none else [b1])
+    f.to_device()
+    asm.pack_coefficients(f)
+    o = cpu.OracleAssembler(a) if T is None else None
+    rp, cols, _ = A.csr()
+    if o is not None:
+        orp, ocols, _, _ = o.sparsity()
+        assert np.array_equal(rp, orp) and np.array_equal(cols, ocols)
+    full = o.assemble_matrix(rp, cols, []) if o is not None else _at_pattern(V, W, rp, cols, T)
+    rows = np.repeat(np.arange(V.size), np.diff(rp))
+    m0, m1 = np.zeros(V.size, bool), np.zeros(W.size, bool)
+    if not none:
+        m0[b0.dofs], m1[b1.dofs] = True, True
+    for times in (1, 2):
+        _lib.check(_lib.lib().mf_assemble_matrix(f.handle, A.handle, p0._get_cpp_bcs(V).handle,
+                                                 p1._get_cpp_bcs(W).handle, 2.5, int(times == 1), None))
+        asm.synchronize()
+        ref = np.where(m0[rows] | m1[cols], 0.0, times * full)
+        if V is W:
+            ref[(rows == cols) & m0[rows]] = 2.5
+        assert _rel(A.csr()[2], ref) <= TOL, times
