@@ -470,7 +470,8 @@ def linear_sum(a: Form, b: Form) -> Form:
     """L = a + b for rank-1 forms: integrals concatenated in cell, ext, int order.
 
     The coefficient/constant arrays of the two forms are merged and the
-    integral bodies rewritten so w/c offsets stay valid.
+    integral bodies rewritten so w/c offsets stay valid, under names of their
+    own: a body stands once in a form's source, by its name.
     """
     if a.rank != b.rank or a.function_spaces[0] is not b.function_spaces[0]:
         raise ValueError("forms must have equal rank and spaces")
@@ -478,9 +479,11 @@ def linear_sum(a: Form, b: Form) -> Form:
     consts_a = int(sum(c.value.size for c in a.constants))
     new_b = []
     for I in b.integrals:
-        src = I.source
+        src, name = I.source, I.name
         if coffs_a or consts_a:
+            name = f"{I.name}_w{coffs_a}c{consts_a}"
             src = src.replace("{\n", "{\n  w += %d; c += %d;\n" % (coffs_a, consts_a), 1)
+            src = src.replace(I.name, name)
         spec = dict(I.spec)
         for key, val in list(spec.items()):
             if isinstance(val, tuple) and val[0] == "w":
@@ -488,7 +491,7 @@ def linear_sum(a: Form, b: Form) -> Form:
             elif isinstance(val, tuple) and val[0] == "c":
                 spec[key] = ("c", val[1] + consts_a)
         staged = I.staged.shifted(consts_a) if hasattr(I.staged, "shifted") else I.staged
-        new_b.append(Integral(I.type, I.id, I.entities, I.name, src, staged, spec))
+        new_b.append(Integral(I.type, I.id, I.entities, name, src, staged, spec))
     order = {CELL: 0, EXTERIOR_FACET: 1, INTERIOR_FACET: 2}
     ints = sorted(a.integrals + new_b, key=lambda I: order[I.type])
     return Form(a.rank, a.function_spaces, ints, a.coefficients + b.coefficients,

@@ -858,3 +858,39 @@ def test_gathered_blocks_spaces_and_facets(which, n, sets):
         if V is W:
             ref[(rows == cols) & m0[rows]] = 2.5
         assert _rel(A.csr()[2], ref) <= TOL, times
+
+
+@pytest.mark.parametrize("which", ["constants", "functions", "vector", "hex", "three", "facets"])
+def test_sum_of_forms_with_one_body(which):
+    """Two terms with the same element body keep each their constants and
+    coefficients."""
+    import cudolfinx as cufem
+    from mifem.fem import Constant
+    print(f"[gpu-test] sum of forms with one body: {which}", flush=True)
+    if which == "hex":
+        V = functionspace(create_unit_cube(3, "hexahedron", jitter=0.2, seed=1), ("P", 2))
+        terms = [forms.hex_source(V, Constant(v)) for v in (1.0, -3.0)]
+    else:
+        V = functionspace(create_unit_cube(3, jitter=0.2, seed=1), ("P", 2), **({"shape": (3,)} if which == "vector" else {}))
+        rng = np.random.default_rng(1)
+        if which == "functions":
+            fs = [Function(V), Function(V)]
+            for f in fs:
+                f.x[:] = rng.uniform(-1, 1, V.size)
+            terms = [forms.source(V, f) for f in fs]
+        elif which == "facets":
+            m = V.mesh
+            ends = [m.locate_boundary_facets(lambda x, e=e: np.isclose(x[0], e)) for e in (0.0, 1.0)]
+            terms = [forms.facet_source(V, Constant(v), e) for v, e in zip((2.0, -5.0), ends)]
+        elif which == "vector":
+            terms = [forms.source(V, Constant(v)) for v in ([1.0, 2.0, 3.0], [0.5, -7.0, 2.0])]
+        else:
+            terms = [forms.source(V, Constant(v)) for v in (1.0, -3.0, 5.0)[:3 if which == "three" else 2]]
+    L = terms[0]
+    for t in terms[1:]:
+        L = forms.linear_sum(L, t)
+    asm = cufem.CUDAAssembler()
+    b = asm.assemble_vector(cufem.form(L))
+    asm.synchronize()
+    ref = sum(cpu.OracleAssembler(t).assemble_vector() for t in terms)
+    assert _rel(b.to_host(), ref) <= TOL
