@@ -92,6 +92,17 @@ std::shared_ptr<OwnerPlan> build_items(const std::vector<int32_t>& rows, const I
   return plan;
 }
 
+// sum[0 .. 8 V) = init[h ..] + the n rows at[.][h ..] (16-byte aligned)
+typedef uint16_t U16x8 __attribute__((vector_size(16), may_alias));
+template <int V>
+static void add_up(uint16_t* sum, uint16_t* const* at, int n, const uint16_t* init, int h) {
+  U16x8 m[V];
+  for (int v = 0; v < V; ++v) m[v] = reinterpret_cast<const U16x8*>(init + h)[v];
+  for (int i = 0; i < n; ++i)
+    for (int v = 0; v < V; ++v) m[v] += reinterpret_cast<const U16x8*>(at[i] + h)[v];
+  for (int v = 0; v < V; ++v) reinterpret_cast<U16x8*>(sum)[v] = m[v];
+}
+
 // Contiguous blocked-row chunks whose unrolled value segment fits `cap`
 // doubles, with at most `maxr` rows and `maxp` (cell, owned row) pairs; then
 // the per-chunk pair lists and, for every pair and column j of the cell, the
@@ -211,48 +222,75 @@ std::shared_ptr<OwnerPlan> build_owner_plan(const mf_form& a, const Integral& I,
     int32_t cell, i, row, turn;
     uint8_t kk[32];
   };
-  auto order_pairs = [&](std::vector<Pair>& P, int64_t c, std::vector<int32_t>& place) {
+  struct Scratch {                                     // of one thread
+    std::vector<int32_t> first, order;                 // order[first[r] ..]: the pairs of row r
+    std::vector<int32_t> where;                        // of a column node in the row at hand
+    std::vector<uint16_t> load, meet;
+    std::vector<int> fill;
+    std::vector<uint16_t*> at;
+  };
+  auto order_pairs = [&](const std::vector<Pair>& P, int64_t c, std::vector<int32_t>& place, Scratch& S) {
     const int np = static_cast<int>(P.size()), nb = (np + kGroup - 1) / kGroup, bs = A.bs0;
+    const int nr = rows[c + 1] - rows[c];
     const int64_t cb0 = A.h_rpb[rows[c]];
-    std::vector<std::array<int32_t, 4>> order(np);      // turn, row, local row, pair
-    for (int k = 0; k < np; ++k) order[k] = {P[k].row, P[k].turn, P[k].i, k};
-    std::sort(order.begin(), order.end());
-    std::vector<int32_t> count(rows[c + 1] - rows[c], 0);
-    for (auto& q : order) q = {count[q[0]]++, q[0], 0, q[3]};
-    std::sort(order.begin(), order.end());
     place.resize(np);
-    if (nb == 1) {
-      for (int k = 0; k < np; ++k) place[order[k][3]] = k;
-      return;
-    }
-    std::vector<uint8_t> load(static_cast<size_t>(nb) * nd * bs * 32, 0);
-    std::vector<int> fill(nb, 0);
-    std::vector<int> bank(nd * bs);
-    for (auto& q : order) {
-      const Pair& x = P[q[3]];
-      const int64_t R = rows[c] + x.row, len = A.h_rpb[R + 1] - A.h_rpb[R];
-      const int64_t lo = (int64_t)bs2 * (A.h_rpb[R] - cb0);
-      for (int j = 0; j < nd; ++j)
-        for (int e = 0; e < bs; ++e)
-          bank[j * bs + e] = (j * bs + e) * 32 + static_cast<int>((lo + e * A.bs1 * len + A.bs1 * x.kk[j]) & 31);
-      int best = -1, least = INT32_MAX;
-      for (int h = 0; h < nb; ++h) {
-        if (fill[h] == std::min(kGroup, np - kGroup * h)) continue;
-        const uint8_t* l = &load[(size_t)h * nd * bs * 32];
-        int meet = 0;
-        for (int k : bank) meet += l[k];
-        if (meet < least) {
-          least = meet;
-          best = h;
-        }
+    // in a row by (turn, local row), which no two pairs of it share
+    int most = 0;
+    auto key = [&](int k) { return P[k].turn * 64 + P[k].i; };
+    for (int r = 0; r < nr; ++r) {
+      most = std::max(most, S.first[r + 1] - S.first[r]);
+      for (int a = S.first[r] + 1; a < S.first[r + 1]; ++a) {
+        const int k = S.order[a];
+        int q = a;
+        for (; q > S.first[r] && key(S.order[q - 1]) > key(k); --q) S.order[q] = S.order[q - 1];
+        S.order[q] = k;
       }
-      for (int k : bank) ++load[(size_t)best * nd * bs * 32 + k];
-      place[q[3]] = kGroup * best + fill[best]++;
     }
+    // The pairs that meet in a bank, by (column, component), bank and group: the
+    // groups of one place lie side by side, so a pair is weighed against all of
+    // them at once.
+    const int NB = (nb + 7) / 8 * 8;
+    S.load.assign((static_cast<size_t>(nd) * bs * 32 + 1) * NB, 0);
+    S.meet.resize(NB);
+    S.at.resize(nd * bs);
+    S.fill.assign(nb, 0);
+    int dealt = 0;
+    for (int turn = 0; turn < most; ++turn)
+      for (int r = 0; r < nr; ++r) {
+        if (S.first[r] + turn >= S.first[r + 1]) continue;
+        const int k = S.order[S.first[r] + turn];
+        if (nb == 1) {
+          place[k] = dealt++;
+          continue;
+        }
+        const Pair& x = P[k];
+        const int64_t R = rows[c] + r, len = A.h_rpb[R + 1] - A.h_rpb[R];
+        const int64_t lo = (int64_t)bs2 * (A.h_rpb[R] - cb0);
+        for (int j = 0; j < nd; ++j)
+          for (int e = 0; e < bs; ++e) {
+            const int64_t b = (lo + e * A.bs1 * len + A.bs1 * x.kk[j]) & 31;
+            S.at[j * bs + e] = &S.load[((size_t)(j * bs + e) * 32 + b) * NB];
+          }
+        for (int h = 0; h < NB; h += 32) {
+          const int v = std::min(4, (NB - h) / 8);
+          (v == 1 ? add_up<1> : v == 2 ? add_up<2> : v == 3 ? add_up<3> : add_up<4>)(&S.meet[h], S.at.data(), nd * bs, &S.load[(size_t)nd * bs * 32 * NB], h);
+        }
+        int best = -1, least = INT32_MAX;
+        for (int h = 0; h < nb; ++h)
+          if (S.meet[h] < least) {
+            least = S.meet[h];
+            best = h;
+          }
+        for (uint16_t* l : S.at) ++l[best];
+        place[k] = kGroup * best + S.fill[best]++;
+        // a full group looks worse than any other (at most nd * bs * kGroup = 512 meet)
+        if (S.fill[best] == std::min(kGroup, np - kGroup * best)) S.load[(size_t)nd * bs * 32 * NB + best] = 1024;
+      }
   };
   auto work = [&](unsigned t) {
     std::vector<Pair> P;
     std::vector<int32_t> place, turn;
+    Scratch S;
     for (int64_t c = t; c < nch; c += nt) {
       P.clear();
       turn.assign(with_kk ? static_cast<size_t>(rows[c + 1] - rows[c]) * nd : 0, 0);
@@ -264,23 +302,49 @@ std::shared_ptr<OwnerPlan> build_owner_plan(const mf_form& a, const Integral& I,
           const int32_t R = d0->host[(int64_t)cell * nd + i];
           const int32_t* rb = A.h_colsb.data() + A.h_rpb[R];
           const int32_t* re = A.h_colsb.data() + A.h_rpb[R + 1];
-          const int64_t longest = with_kk ? 255 : 65535;
-          if (with_kk) P.push_back({cell, i, R - rows[c], turn[(size_t)(R - rows[c]) * nd + i]++, {}});
+          if (with_kk) {
+            P.push_back({cell, i, R - rows[c], turn[(size_t)(R - rows[c]) * nd + i]++, {}});
+            continue;
+          }
           for (int j = 0; j < nd; ++j) {
             const int32_t Cn = d1->host[(int64_t)cell * nd + j];
             const int32_t* f = std::lower_bound(rb, re, Cn);
-            const bool ok = f != re && *f == Cn && f - rb <= longest;
+            const bool ok = f != re && *f == Cn && f - rb <= 65535;
             if (!ok) bad[t % 16] = 1;
-            if (with_kk) P.back().kk[j] = ok ? static_cast<uint8_t>(f - rb) : 0;
-            else ppos[p * nd + j] = ok ? static_cast<uint16_t>(f - rb) : 0;
+            ppos[p * nd + j] = ok ? static_cast<uint16_t>(f - rb) : 0;
           }
           // hexahedral kernel: item in the chunk << 16 | row in the chunk << 6 | local row
-          if (!with_kk) plist[p++] = ((it - ci[c]) << 16) | ((R - rows[c]) << 6) | i;
+          plist[p++] = ((it - ci[c]) << 16) | ((R - rows[c]) << 6) | i;
         }
       }
       if (!with_kk) continue;
+      // the pairs by row, and a row's column positions for all its pairs from one
+      // pass over its columns (a search per pair and column took 40% of the time)
+      const int nr = rows[c + 1] - rows[c];
+      S.first.assign(nr + 1, 0);
+      for (auto& x : P) ++S.first[x.row + 1];
+      for (int r = 0; r < nr; ++r) S.first[r + 1] += S.first[r];
+      S.order.resize(P.size());
+      S.fill.assign(nr, 0);
+      for (size_t k = 0; k < P.size(); ++k)
+        S.order[S.first[P[k].row] + S.fill[P[k].row]++] = static_cast<int32_t>(k);
+      if (S.where.empty()) S.where.assign(d1->num_nodes, 0);
+      for (int r = 0; r < nr; ++r) {
+        const int32_t* rb = A.h_colsb.data() + A.h_rpb[rows[c] + r];
+        const int32_t len = A.h_rpb[rows[c] + r + 1] - A.h_rpb[rows[c] + r];
+        for (int32_t q = 0; q < len; ++q) S.where[rb[q]] = q;
+        for (int32_t a = S.first[r]; a < S.first[r + 1]; ++a) {
+          Pair& x = P[S.order[a]];
+          for (int j = 0; j < nd; ++j) {
+            const int32_t Cn = d1->host[(int64_t)x.cell * nd + j], q = S.where[Cn];
+            const bool ok = q < len && rb[q] == Cn && q <= 255;
+            if (!ok) bad[t % 16] = 1;
+            x.kk[j] = ok ? static_cast<uint8_t>(q) : 0;
+          }
+        }
+      }
       if (nd > 4) {
-        order_pairs(P, c, place);
+        order_pairs(P, c, place, S);
       } else {
         place.resize(P.size());
         std::iota(place.begin(), place.end(), 0);
