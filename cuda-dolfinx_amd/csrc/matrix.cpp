@@ -4,7 +4,10 @@
 #include <algorithm>
 #include <array>
 #include <cstdio>
+#include <exception>
+#include <functional>
 #include <numeric>
+#include <system_error>
 #include <thread>
 
 #include "mf_internal.h"
@@ -448,6 +451,96 @@ static bool blocks_pay(const mf_form& L, Integral& I) {
   return I.n >= (I.vown_regs < 100 ? 400000 : I.vown_regs < 160 ? 8000 : 2500);
 }
 
+// The distinct rows among row[0 .. n), appended to `rows` in ascending order, and
+// the place of each among them.  By a bitmap over the rows' range where that is
+// no longer than the list (entities that lie together have rows that do), else
+// by sorting.
+struct RowRanks {
+  std::vector<uint64_t> bits;
+  std::vector<int32_t> before, seen;
+  void operator()(const int32_t* row, size_t n, std::vector<int32_t>& rows, uint16_t* place) {
+    if (n == 0) return;
+    const auto ends = std::minmax_element(row, row + n);
+    const int64_t lo = *ends.first, words = (*ends.second - lo) / 64 + 1;
+    if (words > static_cast<int64_t>(n)) {
+      seen.assign(row, row + n);
+      std::sort(seen.begin(), seen.end());
+      seen.erase(std::unique(seen.begin(), seen.end()), seen.end());
+      for (size_t p = 0; p < n; ++p)
+        place[p] = static_cast<uint16_t>(std::lower_bound(seen.begin(), seen.end(), row[p]) - seen.begin());
+      rows.insert(rows.end(), seen.begin(), seen.end());
+      return;
+    }
+    bits.assign(words, 0);
+    before.resize(words);
+    for (size_t p = 0; p < n; ++p) bits[(row[p] - lo) / 64] |= uint64_t(1) << ((row[p] - lo) % 64);
+    int32_t count = 0;
+    for (int64_t w = 0; w < words; ++w) {
+      before[w] = count;
+      count += __builtin_popcountll(bits[w]);
+      for (uint64_t b = bits[w]; b; b &= b - 1) rows.push_back(static_cast<int32_t>(lo + 64 * w + __builtin_ctzll(b)));
+    }
+    for (size_t p = 0; p < n; ++p) {
+      const int64_t d = row[p] - lo;
+      place[p] = static_cast<uint16_t>(before[d / 64] + __builtin_popcountll(bits[d / 64] & ((uint64_t(1) << (d % 64)) - 1)));
+    }
+  }
+};
+
+// f(begin, end, t) over parts t = 0, 1, ... of [0, n), on threads of their own
+// where a part gets at least `grain` (on this one where no thread is to be had);
+// returns the number of parts.  What a part throws is thrown here.
+template <class F>
+static int in_parts(int64_t n, int64_t grain, const F& f) {
+  const int64_t cpus = std::max(1u, std::thread::hardware_concurrency());
+  const int parts = static_cast<int>(std::max<int64_t>(1, std::min({int64_t(8), cpus, n / grain})));
+  std::exception_ptr failed[8];
+  auto part = [&](int t) {
+    try {
+      f(n * t / parts, n * (t + 1) / parts, t);
+    } catch (...) {
+      failed[t] = std::current_exception();
+    }
+  };
+  std::vector<std::thread> th;
+  th.reserve(parts);
+  for (int t = 1; t < parts; ++t) {
+    try {
+      th.emplace_back(part, t);
+    } catch (const std::system_error&) {
+      part(t);
+    }
+  }
+  part(0);
+  for (auto& x : th) x.join();
+  for (auto& e : failed)
+    if (e) std::rethrow_exception(e);
+  return parts;
+}
+
+// Rows of consecutive blocks: row(k, out) gives the rows of block k's entries, in
+// order, place[at(k) ..] gets their places among its distinct rows, and ptr and rows
+// get the blocks' distinct rows one after the other.
+template <class Row>
+static void rank_blocks(int64_t nblk, int64_t grain, const Row& row, const std::function<int64_t(int64_t)>& at,
+                        std::vector<uint16_t>& place, std::vector<int32_t>& ptr, std::vector<int32_t>& rows) {
+  std::vector<std::vector<int32_t>> part(8);
+  ptr.assign(nblk + 1, 0);
+  const int parts = in_parts(nblk, grain, [&](int64_t k0, int64_t k1, int t) {
+    RowRanks rank;
+    std::vector<int32_t> entries;
+    for (int64_t k = k0; k < k1; ++k) {
+      entries.clear();
+      row(k, entries);
+      const size_t before = part[t].size();
+      rank(entries.data(), entries.size(), part[t], place.data() + at(k));
+      ptr[k + 1] = static_cast<int32_t>(part[t].size() - before);
+    }
+  });
+  for (int64_t k = 0; k < nblk; ++k) ptr[k + 1] += ptr[k];
+  for (int t = 0; t < parts; ++t) rows.insert(rows.end(), part[t].begin(), part[t].end());
+}
+
 // Blocks of at most 256 entities (down to 64 where that leaves fewer than
 // three blocks per CU) whose rows fit 64 KB of LDS; null when rows are shared so
 // little that the blocks hold fewer than half their entities.  With a wave per
@@ -467,37 +560,39 @@ static VectorBlocks* vector_blocks(mf_form* L, const Integral& I, hipStream_t s)
   while (most > (I.k_hsrc ? 4 : 64) && I.n < 3LL * L->ctx->num_cus * most) most /= 2;
   B->threads = I.k_hsrc ? 256 : most;
   const size_t cap = (I.k_hsrc ? 4096 : 8192) / bs;      // nodes per block
-  std::vector<int32_t> ent{0}, ptr{0}, row, place(d0->num_nodes, -1), nodes;
+  std::vector<int32_t> ent{0}, ptr, row;
   std::vector<uint16_t> slot(static_cast<size_t>(I.n) * nd);
-  for (int64_t e = 0; e < I.n;) {
-    const int64_t e0 = e;
-    nodes.clear();
-    for (; e < I.n && e - e0 < most; ++e) {
-      const size_t before = nodes.size();
-      const int32_t* dm = &d0->host[(int64_t)I.h_ents[e] * nd];
-      for (int i = 0; i < nd; ++i)
-        if (place[dm[i]] < 0) {
-          place[dm[i]] = 0;
-          nodes.push_back(dm[i]);
-        }
-      if (nodes.size() > cap) {                          // this entity starts the next block
-        for (size_t k = before; k < nodes.size(); ++k) place[nodes[k]] = -1;
-        nodes.resize(before);
-        break;
+  if (static_cast<size_t>(most) * nd <= cap) {
+    for (int64_t e = most; e < I.n + most; e += most) ent.push_back(static_cast<int32_t>(std::min(e, I.n)));
+  } else {
+    std::vector<int32_t> seen(d0->num_nodes, -1);          // the last block with the node
+    for (int64_t e = 0; e < I.n;) {
+      const int64_t e0 = e;
+      const int32_t blk = static_cast<int32_t>(ent.size());
+      size_t nodes = 0;
+      for (; e < I.n && e - e0 < most; ++e) {
+        const int32_t* dm = &d0->host[(int64_t)I.h_ents[e] * nd];
+        for (int i = 0; i < nd; ++i)
+          if (seen[dm[i]] != blk) {
+            seen[dm[i]] = blk;
+            ++nodes;
+          }
+        if (nodes > cap) break;                            // this entity starts the next block
       }
+      if (e == e0) return (L->vblocks[I.index] = nullptr).get();   // one entity's rows exceed a block
+      ent.push_back(static_cast<int32_t>(e));
     }
-    if (e == e0) return (L->vblocks[I.index] = nullptr).get();   // one entity's rows exceed a block
-    std::sort(nodes.begin(), nodes.end());
-    for (size_t k = 0; k < nodes.size(); ++k) place[nodes[k]] = static_cast<int32_t>(k);
-    for (int64_t q = e0; q < e; ++q)
-      for (int i = 0; i < nd; ++i)
-        slot[q * nd + i] = static_cast<uint16_t>(place[d0->host[(int64_t)I.h_ents[q] * nd + i]]);
-    for (int32_t r : nodes) place[r] = -1;
-    row.insert(row.end(), nodes.begin(), nodes.end());
-    ent.push_back(static_cast<int32_t>(e));
-    ptr.push_back(static_cast<int32_t>(row.size()));
-    B->lds = std::max(B->lds, static_cast<uint32_t>(8 * bs * nodes.size()));
   }
+  rank_blocks(static_cast<int64_t>(ent.size()) - 1, std::max(1, 20000 / (most * nd)),
+              [&](int64_t k, std::vector<int32_t>& out) {
+                for (int32_t q = ent[k]; q < ent[k + 1]; ++q) {
+                  const int32_t* dm = &d0->host[(int64_t)I.h_ents[q] * nd];
+                  out.insert(out.end(), dm, dm + nd);
+                }
+              },
+              [&](int64_t k) { return (int64_t)ent[k] * nd; }, slot, ptr, row);
+  for (size_t k = 0; k + 1 < ptr.size(); ++k)
+    B->lds = std::max(B->lds, static_cast<uint32_t>(8 * bs * (ptr[k + 1] - ptr[k])));
   B->n = static_cast<int64_t>(ent.size()) - 1;
   if (!I.k_hsrc && B->n * most > 2 * std::max<int64_t>(I.n, most)) return (L->vblocks[I.index] = nullptr).get();
   B->ent.upload(ent);
@@ -524,27 +619,37 @@ LiftList build_lift_list(const mf_form& f, const Integral& I, const mf_bc& bc, h
   if (n == 0) return L;
   std::vector<int32_t> list(n);
   MF_HIP(hipMemcpy(list.data(), L.list.ptr, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
-  std::sort(list.begin(), list.end());           // the kernel appends in no particular order
+  {                                              // the kernel appends in no particular order
+    std::vector<uint64_t> in(I.n / 64 + 1, 0);
+    for (int32_t e : list) in[e / 64] |= uint64_t(1) << (e % 64);
+    size_t k = 0;
+    for (size_t w = 0; w < in.size(); ++w)
+      for (uint64_t b = in[w]; b; b &= b - 1) list[k++] = static_cast<int32_t>(64 * w + __builtin_ctzll(b));
+  }
   L.list.upload(list);
   const int nd = d0->nd, bs1 = d1->bs;
   if (!I.k_slift || d1->nd * bs1 > 64 || (int64_t)n * nd >= INT32_MAX) return L;
   std::vector<uint8_t> constrained(d1->num_nodes * bs1, 0);
   for (int32_t d : bc.h_dofs) constrained[d] = 1;
   std::vector<uint64_t> mask(n, 0);
-  for (int32_t k = 0; k < n; ++k) {
-    const int64_t c = I.h_ents[list[k]];
-    for (int j = 0; j < d1->nd * bs1; ++j) {
-      const int64_t node = d1->host[c * d1->nd + j / bs1];
-      mask[k] |= static_cast<uint64_t>(constrained[bs1 * node + j % bs1]) << j;
+  in_parts(n, 2000, [&](int64_t k0, int64_t k1, int) {
+    for (int64_t k = k0; k < k1; ++k) {
+      const int64_t c = I.h_ents[list[k]];
+      uint64_t m = 0;
+      for (int j = 0; j < d1->nd * bs1; ++j) {
+        const int64_t node = d1->host[c * d1->nd + j / bs1];
+        m |= static_cast<uint64_t>(constrained[bs1 * node + j % bs1]) << j;
+      }
+      mask[k] = m;
     }
-  }
-  // row of every (cell, local row), in the order the kernel visits them
-  std::vector<int32_t> row(static_cast<size_t>(n) * nd);
+  });
+  // row of every (cell, local row), in the order the kernel visits them: by cell,
+  // or sorted by row
   const bool by_cell = staged_trace(I);
-  if (by_cell) {
-    for (int32_t k = 0; k < n; ++k)
-      for (int i = 0; i < nd; ++i) row[(size_t)k * nd + i] = d0->host[(int64_t)I.h_ents[list[k]] * nd + i];
-  } else {
+  const int64_t entries = (int64_t)n * nd;
+  std::vector<int32_t> row;
+  if (!by_cell) {
+    row.resize(entries);
     std::vector<int32_t> start(d0->num_nodes + 1, 0), pairs(row.size());
     for (int32_t k = 0; k < n; ++k)
       for (int i = 0; i < nd; ++i) start[d0->host[(int64_t)I.h_ents[list[k]] * nd + i] + 1]++;
@@ -557,19 +662,22 @@ LiftList build_lift_list(const mf_form& f, const Integral& I, const mf_bc& bc, h
       }
     L.pairs.upload(pairs);
   }
-  const size_t per = by_cell ? 64u * nd : 128u;          // contributions per workgroup
-  std::vector<int32_t> ptr{0}, rows, seen;
-  std::vector<uint16_t> slot(row.size());
-  for (size_t p0 = 0; p0 < row.size(); p0 += per) {
-    const size_t p1 = std::min(row.size(), p0 + per);
-    seen.assign(row.begin() + p0, row.begin() + p1);
-    std::sort(seen.begin(), seen.end());
-    seen.erase(std::unique(seen.begin(), seen.end()), seen.end());
-    for (size_t p = p0; p < p1; ++p)
-      slot[p] = static_cast<uint16_t>(std::lower_bound(seen.begin(), seen.end(), row[p]) - seen.begin());
-    rows.insert(rows.end(), seen.begin(), seen.end());
-    ptr.push_back(static_cast<int32_t>(rows.size()));
-  }
+  const int64_t per = by_cell ? 64 * nd : 128;           // contributions per workgroup
+  std::vector<int32_t> ptr, rows;
+  std::vector<uint16_t> slot(entries);
+  rank_blocks((entries + per - 1) / per, std::max<int64_t>(1, 20000 / per),
+              [&](int64_t b, std::vector<int32_t>& out) {
+                const int64_t p1 = std::min(entries, (b + 1) * per);
+                if (!by_cell) {
+                  out.insert(out.end(), row.begin() + b * per, row.begin() + p1);
+                  return;
+                }
+                for (int64_t k = b * 64; k * nd < p1; ++k) {
+                  const int32_t* dm = &d0->host[(int64_t)I.h_ents[list[k]] * nd];
+                  out.insert(out.end(), dm, dm + nd);
+                }
+              },
+              [&](int64_t b) { return b * per; }, slot, ptr, rows);
   L.slot.upload(slot);
   L.blk_ptr.upload(ptr);
   L.blk_row.upload(rows);
