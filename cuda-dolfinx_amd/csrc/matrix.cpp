@@ -432,11 +432,15 @@ std::shared_ptr<OwnerPlan> vector_plan(mf_form* L, Integral& I) {
 // The blocks cost a cleared vector (2.3 us of launch) and their atomics; the
 // other repeats cells, which weighs what the body weighs, and the registers it
 // needs tell light from heavy bodies.  Cell integral in us, rows / blocks:
-//   under 100 registers: P1 196 thousand cells 8.2 / 9.2, 750 thousand 19.0 /
-//     14.1; P2 94 thousand 7.5 / 9.1; vector P2 664 thousand 59 / 51;
-//   P3 source (104): 10 thousand cells 12.2 / 9.0, 83 thousand 23.3 / 13.9;
-//   P2 residual with 64 points (242): 1 thousand 37 / 43, 10 thousand 61 / 41,
-//     48 thousand 97 / 48; P1 with 27 points: 3 thousand 17 / 9.
+//   under 100 registers, line at 300 thousand cells: P1 105 thousand 5.8 / 5.9,
+//     384 thousand 12.1 / 7.5; P2 118 thousand 8.4 / 8.8, 280 thousand 15.4 / 14.2;
+//     vector P1 216 thousand 9.9 / 9.6; vector P2 280 thousand 24.6 / 25.6, 384
+//     thousand 34.7 / 31.0;
+//   to 160 registers, 300 cells: P1 residual with 27 points 162 cells 7.9 / 8.9, 384
+//     cells 13.2 / 8.9; P3 source (104) 6 cells 9.0 / 6.0, 384 cells 10.8 / 7.7, 83
+//     thousand 23.3 / 13.9;
+//   above, 9 thousand: P2 residual with 64 points (242) 1.3 thousand 37 / 43, 8.0
+//     thousand 37.4 / 40.4, 10.4 thousand 58 / 41, 48 thousand 97 / 48.
 // Cells of more than 32 nodes have no row-owning kernel: Q3 source on 14
 // thousand hexahedra 50 us, 78 us with one atomic per row, 14 us with a wave per
 // cell (mf_hsrc_*).
@@ -448,7 +452,7 @@ static bool blocks_pay(const mf_form& L, Integral& I) {
     MF_HIP(hipFuncGetAttribute(&regs, HIP_FUNC_ATTRIBUTE_NUM_REGS, I.k_vown));
     I.vown_regs = std::max(1, regs);
   }
-  return I.n >= (I.vown_regs < 100 ? 400000 : I.vown_regs < 160 ? 8000 : 2500);
+  return I.n >= (I.vown_regs < 100 ? 300000 : I.vown_regs < 160 ? 300 : 9000);
 }
 
 // The distinct rows among row[0 .. n), appended to `rows` in ascending order, and
