@@ -24,9 +24,14 @@ struct OwnerPlan {
   DevArray<int32_t> item_geo;         // hexahedral kernel: the 8 vertices of each item's cell
   DevArray<int32_t> diag_pos;         // hexahedral kernel: row-relative position of the diagonal
   int64_t nitems = 0, npairs = 0;
-  // host copies used while building matrix schedules
+  // host copies used while building schedules
   std::vector<int32_t> h_items, h_cell;
   std::vector<uint64_t> h_mask;
+  void drop_host() {                  // with their memory
+    std::vector<int32_t>().swap(h_items);
+    std::vector<int32_t>().swap(h_cell);
+    std::vector<uint64_t>().swap(h_mask);
+  }
 };
 
 namespace {
@@ -34,7 +39,8 @@ namespace {
 constexpr int kTableLanes = 64;
 
 // Items of a row partition: every entity of a cell integral that has a
-// row dof in a chunk, with the mask of its local rows the chunk owns.
+// row dof in a chunk, with the mask of its local rows the chunk owns (on the
+// host; each kernel's schedule holds what that kernel reads).
 std::shared_ptr<OwnerPlan> build_items(const std::vector<int32_t>& rows, const Integral& I,
                                        const mf_dofmap* d0) {
   const int nd = d0->nd;
@@ -79,16 +85,8 @@ std::shared_ptr<OwnerPlan> build_items(const std::vector<int32_t>& rows, const I
   auto plan = std::make_shared<OwnerPlan>();
   plan->nchunks = nch;
   plan->nitems = cnt[nch];
-  plan->chunk_rows.upload(rows);
   std::vector<int32_t> ci(nch + 1);
   for (int64_t c = 0; c <= nch; ++c) ci[c] = static_cast<int32_t>(cnt[c]);
-  plan->chunk_items.upload(ci);
-  plan->item_cell.upload(icell);
-  if (nd <= 32) {
-    std::vector<uint32_t> m32(imask.size());
-    for (size_t q = 0; q < imask.size(); ++q) m32[q] = static_cast<uint32_t>(imask[q]);
-    plan->item_mask.upload(m32);
-  }
   plan->h_items = std::move(ci);
   plan->h_cell = std::move(icell);
   plan->h_mask = std::move(imask);
@@ -381,6 +379,7 @@ std::shared_ptr<OwnerPlan> build_owner_plan(const mf_form& a, const Integral& I,
     mc[10] = static_cast<int32_t>(kkoff[c]);
   }
   if (!with_kk) {
+    plan->item_cell.upload(plan->h_cell);
     const mf_mesh& M = *a.mesh;
     std::vector<int32_t> geo(M.num_cells * M.nv), ig((plan->nitems + 1) * M.nv, 0);
     MF_HIP(hipMemcpy(geo.data(), M.cells.ptr, sizeof(int32_t) * geo.size(), hipMemcpyDeviceToHost));
@@ -406,7 +405,7 @@ std::shared_ptr<OwnerPlan> build_owner_plan(const mf_form& a, const Integral& I,
     plan->diag_pos.upload(dp);
   }
   plan->npairs = np;
-  plan->h_items.clear(); plan->h_cell.clear(); plan->h_mask.clear();
+  plan->drop_host();
   return plan;
 }
 
@@ -423,6 +422,12 @@ std::shared_ptr<OwnerPlan> vector_plan(mf_form* L, Integral& I) {
     for (int64_t r = 0; r < d0->num_nodes; r += per) rows.push_back(static_cast<int32_t>(r));
     rows.push_back(static_cast<int32_t>(d0->num_nodes));
     plan = build_items(rows, I, d0);
+    plan->chunk_rows.upload(rows);
+    plan->chunk_items.upload(plan->h_items);
+    plan->item_cell.upload(plan->h_cell);
+    std::vector<uint32_t> m32(plan->h_mask.begin(), plan->h_mask.end());   // 32 nodes at most
+    plan->item_mask.upload(m32);
+    plan->drop_host();
   }
   L->vplans[I.index] = plan;
   return plan;
