@@ -968,20 +968,21 @@ std::string compile_source(mf_form& f) {
     const int bs = f.dm[0]->bs;
     f.options["chunk_values"] = trace ? (nd > 10 ? 3040 : 2048) : hex ? 4096 : nd <= 4 ? 2304 : bs < 3 ? 3040 : 4640;
     if (!hex) {
-      int most = 0;                                     // cells of a node
       int64_t all = 0;                                  // (cell, row) pairs
+      for (auto& I : f.ints)
+        if (I->type == MF_CELL && !I->staged_src.empty()) all += I->n * nd;
+      const bool small = f.ctx && all < 128LL * f.ctx->num_cus;
+      int pairs = trace ? (nd > 4 ? 256 : 384) : (nd > 4 && bs == 3) || small ? 128 : 256;
+      // a row's cells have to fit, the most of them counted where 384 is not taken anyway
+      int most = 0;
       for (auto& I : f.ints) {
-        if (I->type != MF_CELL || I->staged_src.empty()) continue;
+        if (pairs == 384 || I->type != MF_CELL || I->staged_src.empty()) continue;
         std::vector<int> cells(f.dm[0]->num_nodes, 0);
-        all += I->n * nd;
         for (int32_t c : I->h_ents)
           for (int i = 0; i < nd; ++i) most = std::max(most, ++cells[f.dm[0]->host[(int64_t)c * nd + i]]);
       }
-      int pairs = 384;
-      if (trace) pairs = nd > 4 ? 256 : 384;
-      else if ((nd > 4 && bs == 3) || (f.ctx && all < 128LL * f.ctx->num_cus && most <= 128)) pairs = 128;
-      else pairs = 256;
-      f.options["owner_pairs"] = most <= pairs ? pairs : 384;
+      if (most > pairs) pairs = most <= 256 && !trace && !(nd > 4 && bs == 3) ? 256 : 384;
+      f.options["owner_pairs"] = pairs;
     }
   }
   const int64_t cap = f.opt("chunk_values", trace ? 2048 : (hex ? 4096 : 4608));
