@@ -17,6 +17,7 @@
 //    segment exactly once from LDS.
 #include <cctype>
 #include <cstdio>
+#include <cstdlib>
 #include <sstream>
 
 #include "mf_internal.h"
@@ -597,19 +598,39 @@ bool tensor_emitted(const mf_form& f, const Integral& I) {
            f.dm[0]->num_nodes == f.dm[0]->num_cells * f.dm[0]->nd);
 }
 
+// Quadrature points of an element body: the largest bound of its loops over iq
+// (as FFCx and mifem write them; 0 where there are none).
+static int body_points(const std::string& src) {
+  int most = 0;
+  for (size_t p = src.find("iq < "); p != std::string::npos; p = src.find("iq < ", p + 5))
+    most = std::max(most, std::atoi(src.c_str() + p + 5));
+  return most;
+}
+
 // Row groups of the per-entity lifting kernel.  The entities at a boundary are
-// few (1,600 cells for one face of 20^3 cubes), so the kernel lasts as long as
-// one thread's body; a group costs the geometry and coefficient part once more
-// but takes only its own rows.  Groups of about 20 tensor entries: P2 scalar,
-// 64 points, 168 us with one group, 115 with two, 79 with four, 56 with five, 81
-// with ten.  Tensors above 256 entries stay whole: the compiler keeps their
-// loops and the tensor in scratch memory, where no row can be dropped.
+// few (1,600 cells for one face of 20^3 cubes), so with a heavy body the kernel
+// lasts as long as one thread's body; a group costs the geometry and coefficient
+// part once more but takes only its own rows.  Groups of about 20 tensor entries:
+// P2 scalar, 64 points, 168 us with one group, 115 with two, 79 with four, 56 with
+// five, 81 with ten.  A body is heavy from 4,000 products of points and entries
+// on: P2 with 64 points (6,400) 128 us with one group, 51 with groups (16 thousand
+// cells, all constrained: 122 and 101), P2 mass (2,700) 18.9 and 18.6 (all
+// constrained 23.5 and 34), P2 stiffness (400) 10.8 and 12.1 (25^3: 18.8 and 28.5),
+// vector P1 (144) 22.8 and 19.0 (20^3: 28 and 36).  Facets between two cells stay
+// whole (P1 10^3: 12.6 us, 40 in groups: each repeats both cells' tables).
+// Tensors above 256 entries stay whole: the compiler keeps their loops and the
+// tensor in scratch memory, where no row can be dropped.
 int row_groups(const mf_form& f, const Integral& I) {
+  if (I.lift_groups > 0) return I.lift_groups;
   const int ncell = entity_ncell(I.type), ni = ncell * f.dm[0]->nd;
   const int entries = ni * f.dm[0]->bs * ncell * f.dm[1]->nd * f.dm[1]->bs;
-  if (entries > 256) return 1;
-  const int per = std::max(1, 20 * ni / entries);        // nodes per group
-  return (ni + per - 1) / per;
+  int groups = 1;
+  if (ncell == 1 && entries <= 256 && entries * body_points(I.tab_src) >= 4000) {
+    const int per = std::max(1, 20 * ni / entries);      // nodes per group
+    groups = (ni + per - 1) / per;
+  }
+  I.lift_groups = groups;
+  return groups;
 }
 
 bool dg_owner_emitted(const mf_form& f) {

@@ -269,6 +269,7 @@ struct Integral {
   int type = 0, id = -1;
   std::string tab_name, tab_src, staged_src;
   mutable std::atomic<int8_t> trace{-1};   // staged_trace (-1: not looked up)
+  mutable std::atomic<int> lift_groups{0};  // row_groups (0: not looked up)
   std::vector<int32_t> h_ents;
   DevArray<int32_t> d_ents;
   int64_t n = 0;

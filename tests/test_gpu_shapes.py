@@ -894,3 +894,44 @@ def test_sum_of_forms_with_one_body(which):
     asm.synchronize()
     ref = sum(cpu.OracleAssembler(t).assemble_vector() for t in terms)
     assert _rel(b.to_host(), ref) <= TOL
+
+
+@pytest.mark.parametrize("share", [0.02, 0.3, 1.0])
+@pytest.mark.parametrize("which,n", [("heavy", 1), ("heavy", 4), ("light", 3), ("whole", 2), ("facets", 3), ("exterior", 3)])
+def test_lifting_by_entity(which, n, share):
+    """The per-entity lifting kernel: a body heavy enough for row groups (P2 with 64
+    points), light ones, a tensor of more than 256 entries, facets between cells."""
+    import dataclasses
+    import cudolfinx as cufem
+    from mifem.nonlinear import _int_forms, reference_test_forms
+    print(f"[gpu-test] lifting by entity: {which} n={n} share={share}", flush=True)
+    mesh = create_unit_cube(n, jitter=0.2, seed=1)
+    rng = np.random.default_rng(4)
+    if which in ("heavy", "exterior"):
+        R = reference_test_forms(mesh, 2)
+        a = R["matrix"][0 if which == "heavy" else 1]
+        R["u"].x[:] = rng.uniform(-1, 1, R["u"].x.size)
+    elif which == "facets":
+        V = functionspace(mesh, ("P", 1))
+        kap, u = Function(V), Function(V)
+        kap.x[:], u.x[:] = rng.uniform(0.5, 1, (2, V.size))
+        a = forms.Form(2, [V, V], [_int_forms(V, V, 2)], [kap, u])
+    else:
+        a = _poisson(n, 2)[1] if which == "light" else _elasticity(n)[1]
+        a = dataclasses.replace(a, integrals=[dataclasses.replace(a.integrals[0], staged=None)])
+    V = a.function_spaces[0]
+    bc = _some_dofs(V, share, 6)
+    x0 = rng.uniform(-1, 1, V.size)
+    f = cufem.form(a)
+    kind = {"facets": "int", "exterior": "ext"}.get(which, "cell")
+    groups = f.source().split("mf_lift_" + kind + "_0(")[1].split("\n}\n")[0].count("case ")
+    assert (groups > 1) == (which == "heavy"), groups
+    asm = cufem.CUDAAssembler()
+    b = cufem.CUDAVector(asm._ctx, V.size)
+    xv = cufem.CUDAVector(asm._ctx, V.size)
+    xv.data.upload(x0)
+    asm.apply_lifting(b, [f], [asm.pack_bcs([bc])], x0=[xv], scale=0.6)
+    asm.synchronize()
+    ref = np.zeros(V.size)
+    cpu.OracleAssembler(a).apply_lifting(ref, [bc], x0=x0, scale=0.6)
+    assert _rel(b.to_host(), ref) <= TOL
