@@ -382,6 +382,8 @@ void compile_form(mf_form* f, int verbose) {
         if (mf::tensor_emitted(*f, *I))
           I->k_ten = f->mod->get(mf::kernel_name("ten", I->type, I->index));
         I->k_lift = f->mod->get(mf::kernel_name("lift", I->type, I->index));
+        if (mf::row_groups(*f, *I) > 1)
+          I->k_liftw = f->mod->get(mf::kernel_name("liftw", I->type, I->index));
         if (I->type == MF_CELL && mf::is_hex_staged(*I)) {
           if (mf::hex_lift_emitted(*f, *I))
             I->k_hlift = f->mod->get(mf::kernel_name("hlift", I->type, I->index));
@@ -1223,6 +1225,29 @@ int mf_assemble_vector(mf_form* L, double* b, int64_t n, int zero, mf_stream s) 
   });
 }
 
+namespace {
+// The per-entity lifting kernel over n entities of a list, or over *count <= n of
+// them: rows in groups up to row_groups_most entities, whole tensors beyond.  A
+// count on the device is not known here: then both are launched, and the kernel
+// whose range the count is not in returns at once.
+void entity_lift(const mf_form& f, const mf::Integral& I, int64_t n, const int32_t* count,
+                 const int32_t* list, const mf_bc& bc, const double* x0, double scale, double* b,
+                 hipStream_t s) {
+  const int64_t block = f.opt("block", 128);
+  const int ng = mf::row_groups(f, I);
+  const int64_t most = ng > 1 ? mf::row_groups_most(ng) : n;
+  auto go = [&](hipFunction_t k, int64_t entities, int groups) {
+    mf::launch(k, static_cast<uint32_t>((entities + block - 1) / block * groups),
+               static_cast<uint32_t>(block), 0, s, static_cast<int32_t>(n), count, list,
+               I.d_ents.ptr, f.mesh->cells.ptr, f.mesh->x.ptr, f.packed.ptr, f.consts.ptr,
+               f.dm[0]->dev.ptr, f.dm[1]->dev.ptr, bc.markers.ptr, bc.g.ptr, x0, scale, b,
+               f.mesh->fperm.ptr);
+  };
+  if (count || n <= most) go(I.k_lift, std::min(n, most), ng);
+  if (n > most) go(I.k_liftw, n, 1);
+}
+}  // namespace
+
 int mf_apply_lifting(mf_form* const* a, int nforms, double* b, int64_t n,
                      const mf_bc* const* bcs1, const double* const* x0, double scale,
                      mf_stream s) {
@@ -1247,7 +1272,6 @@ int mf_apply_lifting(mf_form* const* a, int nforms, double* b, int64_t n,
       MF_HIP(hipStreamIsCapturing(S(s), &cs));
       const bool capturing = cs != hipStreamCaptureStatusNone;
       const bool nothing = !xk && bc->g_zero && !capturing;   // b -= scale A[:, bc] (g - x0) = 0
-      const uint32_t block = static_cast<uint32_t>(f->opt("block", 128));
       for (auto& I : f->ints) {
         if (I->n == 0) continue;
         auto it = I->lift_lists.find(bc->key);
@@ -1276,13 +1300,7 @@ int mf_apply_lifting(mf_form* const* a, int nforms, double* b, int64_t n,
                      f->mesh->cells.ptr, f->mesh->x.ptr, f->dm[0]->dev.ptr, bc->markers.ptr,
                      bc->g.ptr, xk, scale, b);
         } else {
-          mf::launch(I->k_lift, static_cast<uint32_t>((nl + block - 1) / block * mf::row_groups(*f, *I)),
-                     block, 0, S(s),
-                     static_cast<int32_t>(nl), static_cast<const int32_t*>(nullptr),
-                     ll.list.ptr, I->d_ents.ptr,
-                     f->mesh->cells.ptr, f->mesh->x.ptr, f->packed.ptr, f->consts.ptr,
-                     f->dm[0]->dev.ptr, f->dm[1]->dev.ptr, bc->markers.ptr, bc->g.ptr, xk, scale,
-                     b, f->mesh->fperm.ptr);
+          entity_lift(*f, *I, nl, nullptr, ll.list.ptr, *bc, xk, scale, b, S(s));
         }
       }
     }
@@ -1317,7 +1335,6 @@ int mf_apply_lifting_noalloc(mf_form* const* a, int nforms, double* b, int64_t n
       int32_t* count = ptr;
       int32_t* list = ptr + 64;
       const double* xk = x0 ? x0[k] : nullptr;
-      const uint32_t block = static_cast<uint32_t>(f->opt("block", 128));
       for (auto& I : f->ints) {
         if (I->n == 0) continue;
         // the list of entities touching a constrained column, built on the
@@ -1344,12 +1361,7 @@ int mf_apply_lifting_noalloc(mf_form* const* a, int nforms, double* b, int64_t n
                      I->d_ents.ptr, f->mesh->cells.ptr, f->mesh->x.ptr, f->dm[0]->dev.ptr,
                      bc->markers.ptr, bc->g.ptr, xk, scale, b);
         } else {
-          mf::launch(I->k_lift, static_cast<uint32_t>((I->n + block - 1) / block * mf::row_groups(*f, *I)),
-                     block, 0, S(s),
-                     static_cast<int32_t>(I->n), static_cast<const int32_t*>(count), list,
-                     I->d_ents.ptr, f->mesh->cells.ptr, f->mesh->x.ptr, f->packed.ptr,
-                     f->consts.ptr, f->dm[0]->dev.ptr, f->dm[1]->dev.ptr, bc->markers.ptr,
-                     bc->g.ptr, xk, scale, b, f->mesh->fperm.ptr);
+          entity_lift(*f, *I, I->n, count, list, *bc, xk, scale, b, S(s));
         }
       }
     }

@@ -293,7 +293,8 @@ $KNAME(const int32_t nlist, const int32_t* __restrict__ nlist_dev, const int32_t
   // once per group with only that group's rows live, so the rest of its tensor
   // is dropped at compile time
   const int t = blockIdx.x / $NG * blockDim.x + threadIdx.x;
-  if (t >= (nlist_dev ? *nlist_dev : nlist)) return;
+  const int count = nlist_dev ? *nlist_dev : nlist;
+  if (t >= count$RANGE) return;
   const int e = list[t];
 $GATHER
 $ROWS}
@@ -632,6 +633,12 @@ int row_groups(const mf_form& f, const Integral& I) {
   I.lift_groups = groups;
   return groups;
 }
+
+// Most entities to lift in ng row groups: two waves per SIMD unit (1,024 units, 64
+// lanes); past that the groups' repeated parts take the time.  P2 with 64 points,
+// all constrained, five groups / whole: 16,464 cells 102 / 121 us, 24,576 cells
+// 110 / 123, 48,000 cells 211 / 133.
+int64_t row_groups_most(int ng) { return 131072 / ng; }
 
 bool dg_owner_emitted(const mf_form& f) {
   if (f.rank == 0) return false;
@@ -1148,22 +1155,29 @@ std::string generate_form_source(const mf_form& f) {
     if (f.rank == 2) {
       m["$KNAME"] = kernel_name("mat", I->type, I->index);
       os << subst(subst(kMatrix, {{"$GATHER", gather}}), m);
-      const int ni = ncell * d0->nd, ng = row_groups(f, *I);
-      const int per = (ni + ng - 1) / ng;
-      std::string groups;
-      for (int g = 0; g < ng; ++g)
-        groups += subst(kLiftGroup, {{"$GRP", std::to_string(g)}, {"$I0", std::to_string(g * per)},
-                                       {"$I1", std::to_string(std::min(ni, (g + 1) * per))}});
-      m["$NG"] = std::to_string(ng);
-      m["$UNROLL"] = ni * d0->bs * ncell * d1->nd * d1->bs <= 256 ? "#pragma unroll" : "#pragma unroll 1";
+      const int ni = ncell * d0->nd;
+      const bool whole = ni * d0->bs * ncell * d1->nd * d1->bs > 256;
+      m["$UNROLL"] = whole ? "#pragma unroll 1" : "#pragma unroll";
       if (tensor_emitted(f, *I)) {
         m["$KNAME"] = kernel_name("ten", I->type, I->index);
         os << subst(subst(kTensor, {{"$GATHER", gather}}), m);
       }
-      m["$KNAME"] = kernel_name("lift", I->type, I->index);
-      const bool whole = ni * d0->bs * ncell * d1->nd * d1->bs > 256;
-      const std::string rows = whole ? kLiftWhole : subst(kLiftRows, {{"$GROUPS", groups}});
-      os << subst(subst(kLift, {{"$GATHER", gather}, {"$ROWS", rows}}), m);
+      auto lift = [&](const char* name, int ng, const std::string& range) {
+        const int per = (ni + ng - 1) / ng;
+        std::string groups;
+        for (int g = 0; g < ng; ++g)
+          groups += subst(kLiftGroup, {{"$GRP", std::to_string(g)}, {"$I0", std::to_string(g * per)},
+                                         {"$I1", std::to_string(std::min(ni, (g + 1) * per))}});
+        m["$NG"] = std::to_string(ng);
+        m["$RANGE"] = range;
+        m["$KNAME"] = kernel_name(name, I->type, I->index);
+        const std::string rows = whole ? kLiftWhole : subst(kLiftRows, {{"$GROUPS", groups}});
+        os << subst(subst(kLift, {{"$GATHER", gather}, {"$ROWS", rows}}), m);
+      };
+      const int ng = row_groups(f, *I);
+      const std::string most = std::to_string(row_groups_most(ng));
+      lift("lift", ng, ng > 1 ? " || count > " + most : "");
+      if (ng > 1) lift("liftw", 1, " || count <= " + most);
       if (I->type == MF_CELL && is_hex_staged(*I)) {
         os << "\n" << I->staged_src << "\n";
         if (hex_lift_emitted(f, *I)) {

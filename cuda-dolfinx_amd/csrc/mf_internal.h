@@ -275,7 +275,7 @@ struct Integral {
   int64_t n = 0;
   int index = 0;                      // position in the form
   hipFunction_t k_ten = nullptr;      // element tensors into a workspace
-  hipFunction_t k_mat = nullptr, k_vec = nullptr, k_lift = nullptr, k_owner = nullptr;
+  hipFunction_t k_mat = nullptr, k_vec = nullptr, k_lift = nullptr, k_liftw = nullptr, k_owner = nullptr;
   hipFunction_t k_vblk = nullptr;     // rank 1: blocks of consecutive cells, a thread per cell
   hipFunction_t k_hsrc = nullptr;     // the same with a wave per cell (hexahedral source)
   int vown_regs = 0;                  // registers of k_vown (0: not queried)
@@ -480,6 +480,7 @@ std::string kernel_name(const char* what, int type, int index);
 bool tensor_emitted(const mf_form& f, const Integral& I);
 // row groups of the per-entity lifting kernel
 int row_groups(const mf_form& f, const Integral& I);
+int64_t row_groups_most(int ng);
 // owner vector kernel: the LDS accumulator's values (compile time) and the
 // scalar rows per workgroup of a form (run time, at most that)
 int64_t vector_cap(const mf_form& f);

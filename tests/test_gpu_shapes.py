@@ -935,3 +935,46 @@ def test_lifting_by_entity(which, n, share):
     ref = np.zeros(V.size)
     cpu.OracleAssembler(a).apply_lifting(ref, [bc], x0=x0, scale=0.6)
     assert _rel(b.to_host(), ref) <= TOL
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("share", [0.0005, 1.0])
+def test_lifting_of_many_heavy_cells(share, noalloc):
+    """A heavy body with few and with all of 29 thousand cells to lift: rows in
+    groups, and the whole tensor by one thread."""
+    import ctypes as C
+    import cudolfinx as cufem
+    from cudolfinx import _lib
+    from mifem.nonlinear import reference_test_forms
+    print(f"[gpu-test] lifting of heavy cells: share={share} noalloc={noalloc}", flush=True)
+    mesh = create_unit_cube(17, jitter=0.2, seed=1)
+    rng = np.random.default_rng(4)
+    R = reference_test_forms(mesh, 2)
+    a = R["matrix"][0]
+    R["u"].x[:] = rng.uniform(-1, 1, R["u"].x.size)
+    V = a.function_spaces[0]
+    bc = _some_dofs(V, share, 6)
+    x0 = rng.uniform(-1, 1, V.size)
+    f = cufem.form(a)
+    src = f.source()
+    most = int(src.split("mf_lift_cell_0(")[1].split("count > ")[1].split(")")[0])
+    marked = np.zeros(V.size, bool)
+    marked[bc.dofs] = True
+    listed = int(marked[V.dofmap].any(axis=1).sum())
+    assert (listed > most) == (share == 1.0) and len(V.dofmap) > most, (listed, most)
+    asm = cufem.CUDAAssembler()
+    b = cufem.CUDAVector(asm._ctx, V.size)
+    xv = cufem.CUDAVector(asm._ctx, V.size)
+    xv.data.upload(x0)
+    dbc = asm.pack_bcs([bc])
+    asm.pack_coefficients(f)
+    if noalloc:
+        _lib.check(_lib.lib().mf_apply_lifting_noalloc(
+            (C.c_void_p * 1)(f.handle.value), 1, b.ptr, b.size,
+            (C.c_void_p * 1)(dbc._get_cpp_bcs(V).handle.value), (C.c_void_p * 1)(xv.ptr.value), 0.6, None))
+    else:
+        asm.apply_lifting(b, [f], [dbc], x0=[xv], scale=0.6)
+    asm.synchronize()
+    ref = np.zeros(V.size)
+    cpu.OracleAssembler(a).apply_lifting(ref, [bc], x0=x0, scale=0.6)
+    assert _rel(b.to_host(), ref) <= TOL
