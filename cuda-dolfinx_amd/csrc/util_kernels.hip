@@ -403,25 +403,31 @@ __global__ void lift_list_kernel(int32_t* __restrict__ list, int32_t* __restrict
   }
 }
 
-// Workgroups land on the 8 XCDs in turn; with this order (grid a multiple of 8)
-// each XCD takes a contiguous eighth of the rows, so the part of x that they
-// share stays in its own L2.
+// Workgroups land on the 8 XCDs in turn; with this order (grid a multiple of 64)
+// each XCD takes eight contiguous runs of the rows, every eighth one, so most of
+// the part of x that they share stays in its own L2.  One run per XCD left XCDs
+// idle where the entries lie in one part of the rows (P2 20^3, first half of the
+// cells: 7.9 us, 5.9 with eight runs; eighth in the middle of 28^3: 27.2 and 6.6);
+// four and sixteen runs are within 5% of eight.
+constexpr int kXcdRuns = 8;
 __device__ __forceinline__ int64_t xcd_block() {
-  return (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+  const int64_t run = gridDim.x / (8 * kXcdRuns), w = blockIdx.x / 8;
+  return (w / run * 8 + blockIdx.x % 8) * run + w % run;
 }
 
 // y = A x for a CSR matrix (int32 row_ptr / cols, FP64 values): G lanes per
 // row (G a power of two <= 64, so a wave holds 64 / G rows); each lane sums a
 // strided part of its row and the lanes of a row combine with shuffles, in a
 // fixed order (repeated products are bit-identical).
-template <int G>
+template <int G, bool PAIRS>
 __global__ void __launch_bounds__(kBlock) spmv_kernel(int64_t nrows, const int32_t* __restrict__ rp,
                                                       const int32_t* __restrict__ cols,
                                                       const double* __restrict__ v,
                                                       const double* __restrict__ x,
                                                       double* __restrict__ y) {
-  // short rows: the x gathers weigh most (P1 50^3 7.3 -> 5.5 us, DG1 32^3 47.7 ->
-  // 43.5 us in XCD order); long rows stream their values (Q3 24^3: 2% slower)
+  // short rows: the x gathers weigh most (P1 50^3 7.3 us in launch order, 6.3 in
+  // XCD order; DG1 32^3 47.7 and 43.5); long rows stream their values (Q3 24^3: 2%
+  // slower)
   const int64_t wg = G <= 8 ? xcd_block() : (int64_t)blockIdx.x;
   const int64_t row = (wg * kBlock + threadIdx.x) / G;
   const int lane = threadIdx.x & (G - 1);
@@ -429,13 +435,13 @@ __global__ void __launch_bounds__(kBlock) spmv_kernel(int64_t nrows, const int32
   if (row < nrows) {
     const int32_t e = rp[row + 1];
     int32_t k = rp[row] + lane;
-    for (; k + G < e; k += 2 * G) {
+    if (PAIRS) for (; k + G < e; k += 2 * G) {
       const double v0 = v[k], v1 = v[k + G];
       const double x0 = x[cols[k]], x1 = x[cols[k + G]];
       acc += v0 * x0;
       acc += v1 * x1;
     }
-    if (k < e) acc += v[k] * x[cols[k]];
+    for (; k < e; k += G) acc += v[k] * x[cols[k]];
   }
   for (int o = G / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, G);
   if (row < nrows && lane == 0) y[row] = acc;
@@ -732,20 +738,28 @@ void k_lift_list(int32_t* list, int32_t* count, const int32_t* ents, int64_t nen
 void k_spmv(int64_t nrows, int64_t nnz, const int32_t* rp, const int32_t* cols, const double* v,
             const double* x, double* y, hipStream_t s) {
   if (nrows <= 0) return;
-  // lanes per row from the mean row length (about three entries per lane)
+  // lanes per row from the mean row length (about three entries per lane); two
+  // loads of a lane in flight, but one where a lane has no more than two of a row's
+  // entries and the pair only splits them (P1 48^3 6.2 us in pairs, 5.3 singly; DG1
+  // 32^3, 20 entries a row, 39.8 and 45.2)
   const double mean = (double)nnz / (double)nrows;
   int g = 2;
   while (g < 64 && g * 3 < mean) g *= 2;
   const int64_t threads = nrows * g;
-  MF_CHECK(threads / kBlock < (1LL << 31) - 16, MF_ESHAPE, "matrix too large for one SpMV launch");
-  const uint32_t grid = static_cast<uint32_t>((threads + kBlock - 1) / kBlock + 7) / 8 * 8;
+  MF_CHECK(threads / kBlock < (1LL << 31) - 8 * kXcdRuns, MF_ESHAPE,
+           "matrix too large for one SpMV launch");
+  const uint32_t grid = static_cast<uint32_t>((threads + kBlock - 1) / kBlock + 8 * kXcdRuns - 1) /
+                        (8 * kXcdRuns) * (8 * kXcdRuns);
   switch (g) {
-    case 2: spmv_kernel<2><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y); break;
-    case 4: spmv_kernel<4><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y); break;
-    case 8: spmv_kernel<8><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y); break;
-    case 16: spmv_kernel<16><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y); break;
-    case 32: spmv_kernel<32><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y); break;
-    default: spmv_kernel<64><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y); break;
+    case 2: spmv_kernel<2, true><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y); break;
+    case 4: spmv_kernel<4, true><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y); break;
+    case 8:
+      if (mean > 16) spmv_kernel<8, true><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y);
+      else spmv_kernel<8, false><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y);
+      break;
+    case 16: spmv_kernel<16, true><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y); break;
+    case 32: spmv_kernel<32, true><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y); break;
+    default: spmv_kernel<64, true><<<grid, kBlock, 0, s>>>(nrows, rp, cols, v, x, y); break;
   }
   MF_HIP(hipGetLastError());
 }

@@ -229,6 +229,31 @@ def test_product_rows_of_any_length(which, n):
     assert np.all(np.abs(y.cpu().numpy() - S @ x) <= 400 * 2.2e-16 * (abs(S) @ np.abs(x)) + 1e-300)
 
 
+@pytest.mark.parametrize("part", [(0, 1), (0, 0.5), (0.5, 0.625), (0.99, 1)])
+@pytest.mark.parametrize("degree,n", [(1, 11), (1, 12), (1, 21), (2, 9), (2, 12)])
+def test_product_with_rows_empty(degree, n, part):
+    """y = A x with the entries in one part of the rows: every row is written once,
+    in each order of the workgroups and for every width."""
+    import dataclasses
+    import scipy.sparse as sp
+    import torch
+    import cudolfinx as cufem
+    print(f"[gpu-test] product over a part: P{degree} n={n} {part}", flush=True)
+    V, a, L = _poisson(n, degree)
+    cells = np.arange(*(int(p * 6 * n**3) for p in part), dtype=np.int32)
+    a = dataclasses.replace(a, integrals=[dataclasses.replace(a.integrals[0], entities=cells)])
+    asm = cufem.CUDAAssembler()
+    A = asm.assemble_matrix(cufem.form(a))
+    asm.synchronize()
+    rp, cols, vals = A.csr()
+    x = np.random.default_rng(1).uniform(-1, 1, A.ncols)
+    y = torch.full((A.nrows,), 7.0, dtype=torch.float64, device="cuda")
+    A.mult(torch.from_numpy(x).cuda(), y)
+    S = sp.csr_matrix((vals, cols, rp), shape=(A.nrows, A.ncols))
+    # at most 400 products per row, each rounded once: 400 eps of the absolute sums
+    assert np.all(np.abs(y.cpu().numpy() - S @ x) <= 400 * 2.2e-16 * (abs(S) @ np.abs(x)) + 1e-300)
+
+
 @pytest.mark.parametrize("prec,tol", [(64, TOL), (32, 1e-6)])
 @pytest.mark.parametrize("n,share,subset", [(1, 0.1, False), (2, 0.0, False), (3, 0.3, True), (5, 0.05, True),
                                             (7, 0.1, False)])
