@@ -129,7 +129,7 @@ $CASES
     __syncthreads();                                  // the workgroup's values are in seg
     const int n = (int)(sege - segb);
     double* out = values + segb;
-    const int h = (int)(segb & 1);                    // peel to a 16-byte boundary
+    const int h = min((int)(segb & 1), n);            // peel to a 16-byte boundary
     if (h && threadIdx.x == 0) __builtin_nontemporal_store(seg[0], &out[0]);
     mf_dod2* o2 = reinterpret_cast<mf_dod2*>(out + h);
     for (int p = threadIdx.x; p < (n - h) >> 1; p += $DBLOCK) {
@@ -553,7 +553,7 @@ $CASES
     const int n = (int)(sege - segb);
     double* out = values + segb;
     if (zero) {
-      const int h = (int)(segb & 1);                    // peel to a 16-byte boundary
+      const int h = min((int)(segb & 1), n);            // peel to a 16-byte boundary
       if (h && threadIdx.x == 0) {
         __builtin_nontemporal_store(seg[0], &out[0]);
         seg[0] = 0.0;

@@ -760,7 +760,7 @@ $KNAME(const int32_t nchunks, const int32_t* __restrict__ chunk_meta,
   // write the segment and clear what was read
   double* out = values + (int64_t)(uint32_t)base;
   if (flags & 1) {
-    const int h = base & 1;                            // peel to a 16-byte boundary
+    const int h = min(base & 1, seglen);               // peel to a 16-byte boundary
     if (h && tid == 0) {
       __builtin_nontemporal_store(acc[0], &out[0]);
       acc[0] = 0.0;

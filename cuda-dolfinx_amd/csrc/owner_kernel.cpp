@@ -966,7 +966,7 @@ $OHEAD($OPARAMS)
     if (flags & 1) {
       // peel one value when the segment starts on an odd double, so the
       // rest goes out as aligned 16-byte non-temporal stores
-      const int h = base & 1;
+      const int h = min(base & 1, seglen);
       if (h && lane == 0) {
         __builtin_nontemporal_store(A[0], &out[0]);
         A[0] = 0.0;

@@ -289,6 +289,48 @@ def test_hexahedral_owner_chunks(n, share, subset, prec, tol):
     assert np.linalg.norm(A.csr()[2] - ref) <= 2 * tol * max(scale, np.linalg.norm(ref))
 
 
+@pytest.mark.parametrize("which", ["hex", "hex32", "pipe", "owner", "dg0"])
+def test_values_beside_rows_without_entries(which):
+    """Chunks without values that start on an odd entry, between and behind others:
+    they write nothing."""
+    import dataclasses
+    import cudolfinx as cufem
+    print(f"[gpu-test] values beside empty rows: {which}", flush=True)
+    if which.startswith("hex"):
+        P = problems.helmholtz_q3(8, seed=8)
+        V, a = P.V, P.a
+        mid = V.mesh.x[V.mesh.cells].mean(axis=1)
+        low = np.flatnonzero((mid < 0.25).all(axis=1))           # 2 x 2 x 2 cells: one row of 343
+        cells = np.concatenate([low, np.flatnonzero((mid > 0.7).all(axis=1))[:1]])
+    elif which == "dg0":
+        V = functionspace(create_unit_cube(7), ("DG", 0))
+        a = forms.mass(V)
+        cells = np.array([3, 70, 71, 900, 901, 902, 903, 904, 1500], dtype=np.int32)
+    else:
+        V, a = _poisson(9, 1)[:2]
+        cells = np.r_[0:2, 6:9, 3000:3002, 3900:3902]
+    cells = np.sort(cells).astype(np.int32)
+    a = dataclasses.replace(a, integrals=[dataclasses.replace(a.integrals[0], entities=cells)])
+    o = cpu.OracleAssembler(a)
+    orp, ocols, _, _ = o.sparsity()
+    empty = np.diff(orp) == 0
+    runs = np.split(np.arange(empty.size), np.flatnonzero(np.diff(empty.astype(int))) + 1)
+    odd = [r for r in runs if empty[r[0]] and r.size >= 128 and orp[r[0]] % 2]
+    assert odd, which
+    options = {"hex": {"matrix_kernel": 2}, "hex32": {"matrix_kernel": 2, "precision": 32},
+               "pipe": {"matrix_kernel": 2, "owner_pipe": 1}, "owner": {"matrix_kernel": 2}, "dg0": {}}[which]
+    f = cufem.form(a, options=options)
+    asm = cufem.CUDAAssembler()
+    ref = o.assemble_matrix(orp, ocols, [])
+    A = asm.assemble_matrix(f)
+    for _ in range(3):
+        asm.assemble_matrix(f, A)
+        asm.synchronize()
+        rp, cols, v = A.csr()
+        assert np.array_equal(rp, orp) and np.array_equal(cols, ocols)
+        assert np.abs(v - ref).max() <= (1e-6 if which == "hex32" else TOL) * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("k,m,n,subset", [(1, 2, 1, False), (1, 3, 9, True), (2, 2, 3, False), (3, 4, 1, False),
                                           (3, 4, 5, True), (3, 4, 13, False), (4, 6, 3, False), (5, 5, 2, True),
                                           (6, 7, 1, False)])
